@@ -464,6 +464,8 @@ int upload_world(World* w) {
       loose.insert(loose.end(), per_world[i].begin(), per_world[i].end());
     }
     w->n_tree = int(tree.size());
+    w->tree_statics = false;
+    for (int f : tree) w->tree_statics = w->tree_statics || host_is_static(w, f);
     if ((st = up(w->f.tree_list, tree, w->stream)) || (st = up(w->f.loose_off, loose_off, w->stream)) ||
         (st = up(w->f.loose, loose, w->stream)))
       return st;
@@ -510,6 +512,7 @@ int upload_world(World* w) {
     }
   }
   B2G_HIP(hipStreamSynchronize(w->stream));
+  toi_note_bodies(w);
   w->dev_nb = w->nb;
   w->dev_np = w->np;
   w->dirty = false;
@@ -633,6 +636,7 @@ int b2g_world_destroy(b2g_world* h) {
   rel(w->toi_cand); rel(w->toi_need); rel(w->toi_rank); rel(w->toi_snap);
   rel(w->toi_cadj_off); rel(w->toi_cadj); rel(w->toi_cadj_cur); rel(w->toi_bfix_off); rel(w->toi_bfix);
   rel(w->toi_bfix_cur); rel(w->toi_cl); rel(w->toi_in_list);
+  rel(w->toi_head); rel(w->toi_next); rel(w->toi_queue); rel(w->toi_queued);
   w->toi_bfix_np = -1;
   rel(w->toi_succ); rel(w->toi_drop_flag); rel(w->toi_drop_pos); rel(w->toi_drop_total);
   {
@@ -851,6 +855,7 @@ int b2g_world_set_body_states(b2g_world* h, const b2g_body_state* in, int32_t n)
   w->h_xf = xf;
   w->h_awake = awake;
   w->h_sleep_time = sleep_time;
+  toi_note_bodies(w);
   return B2G_OK;
 }
 
@@ -885,6 +890,7 @@ int b2g_world_set_bullet(b2g_world* h, int32_t body, int32_t flag) {
   World* w = &h->w;
   w->h_bullet[body] = flag ? 1 : 0;
   w->body_defs[body].bullet = flag ? 1 : 0;
+  toi_note_bodies(w);
   if (w->b.bullet.p && body < w->dev_nb) {
     B2G_HIP(hipMemcpyAsync(w->b.bullet.p + body, &w->h_bullet[body], sizeof(int), hipMemcpyHostToDevice, w->stream));
     B2G_HIP(hipStreamSynchronize(w->stream));

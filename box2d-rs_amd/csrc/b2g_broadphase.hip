@@ -294,44 +294,6 @@ __global__ void __launch_bounds__(kBlock) k_bvh4_collapse(int n_internal, const 
 }
 
 // ---- pair search --------------------------------------------------------------------------
-// B2body::should_collide's joint rule (src/private/dynamics/b2_body.rs:398-412): bodies joined by a
-// joint with collide_connected off do not collide
-__device__ inline bool joined_no_collide(int ba, int bb, const int* __restrict__ nc_off,
-                                         const int* __restrict__ nc_list) {
-  for (int i = nc_off[ba], e = nc_off[ba + 1]; i < e; ++i)
-    if (nc_list[i] == bb) return true;
-  return false;
-}
-
-struct PairFilter {
-  const int* __restrict__ fbody;
-  const int* __restrict__ btype;
-  const int2* __restrict__ filter;
-  const int4* __restrict__ fshape;
-  const int* __restrict__ world;
-  const int* __restrict__ nc_off;   // null: no joint forbids a collision
-  const int* __restrict__ nc_list;
-  __device__ bool ok(int q, int p) const {
-    int bq = fbody[q], bp = fbody[p];
-    if (bq == bp) return false;
-    if (world[q] != world[p]) return false;  // batched worlds never interact
-    // B2body::should_collide: at least one body dynamic (src/private/dynamics/b2_body.rs:391-416)
-    if (btype[bq] != 2 && btype[bp] != 2) return false;
-    if (nc_off && joined_no_collide(bq, bp, nc_off, nc_list)) return false;
-    // default contact filter (src/private/dynamics/b2_world_callbacks.rs:6-18)
-    int2 fq = filter[q], fp = filter[p];
-    if (fq.y == fp.y && fq.y != 0) {
-      if (fq.y < 0) return false;
-    } else {
-      unsigned catq = fq.x & 0xffff, maskq = (unsigned(fq.x) >> 16) & 0xffff;
-      unsigned catp = fp.x & 0xffff, maskp = (unsigned(fp.x) >> 16) & 0xffff;
-      if ((maskq & catp) == 0 || (catq & maskp) == 0) return false;
-    }
-    // a contact class must exist for the shape pair
-    return registry_swap(fshape[q].x & 0xff, fshape[p].x & 0xff) >= 0;
-  }
-};
-
 static constexpr int kTravBlock = 64;                  // one wave: 16 queries of 4 lanes
 static constexpr int kTravLanes = 4;                   // lanes per query, one per slot of a 4-wide node
 static constexpr int kTravQueries = kTravBlock / kTravLanes;

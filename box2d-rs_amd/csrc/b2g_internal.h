@@ -340,6 +340,11 @@ struct World {
   DevArray<int> toi_cl, toi_in_list;
   int toi_bfix_np = -1;
   int toi_events = 0;                 // TOI events solved in the last step
+  // Separable TOI passes (k_toi_bodies): what decides whether the world's passes are (set at upload,
+  // by set_bullet and by set_body_states), and whether a static fixture sits in the BVH
+  bool has_kinematic = false, has_bullet = false, statics_still = true, tree_statics = false;
+  DevArray<int> toi_head, toi_next;      // per body its contacts with static bodies, linked
+  DevArray<int> toi_queue, toi_queued;   // bodies with an event to run; per body: listed
   int cur = 0;         // index of the current contact set in c[]
   int n_pairs = 0;     // pairs in the current set
   int n_pairs_old = 0; // pairs in the previous set
@@ -350,7 +355,7 @@ struct World {
   // pinned host memory (kPinnedInts ints): [0, 134) the solver's counters read back after the
   // colouring (4 counters, 128 colour counts, last round, large-island constraints),
   // [kPinnedPairFlags, +4) the pair search's flags and total, [kPinnedColourOffsets, +385) the
-  // colour offsets uploaded for the solve
+  // colour offsets uploaded for the solve, [kPinnedToi, +4) the counters of a separable TOI pass
   int* h_counters = nullptr;
   int n_touch = 0, n_colors = 0, n_islands = 0;
   int color_rounds = 16;       // colouring rounds launched before the first readback
@@ -398,7 +403,7 @@ struct World {
   JointArrays j;
 };
 
-constexpr int kPinnedInts = 1024, kPinnedPairFlags = 192, kPinnedColourOffsets = 256;
+constexpr int kPinnedInts = 1024, kPinnedPairFlags = 192, kPinnedColourOffsets = 256, kPinnedToi = 768;
 
 // Capacity floor of the arrays sized by the contact set (the pairs, and the solver's arrays,
 // which the pairs bound): reserving for a multiple of the proxy count from the first step keeps a
@@ -453,6 +458,7 @@ int phase_collide(World* w);     // narrowphase on the current contact set
 int phase_solve(World* w, float dt, float dt_ratio, int vel_iters, int pos_iters);
 int phase_synchronize(World* w); // swept + fat AABBs of non-static proxies
 int phase_toi(World* w, float dt, int vi);  // continuous collision after the solve
+void toi_note_bodies(World* w);             // has_kinematic, has_bullet and statics_still from the host mirrors
 int toi_carry_state(World* w);              // TOI state of the previous contact set onto the current one
 void release_solve_graphs(World* w);
 // primitives
@@ -524,6 +530,44 @@ __device__ inline Xf xf_of(float4 t) {
   x.q.c = t.w;
   return x;
 }
+
+// B2body::should_collide's joint rule (src/private/dynamics/b2_body.rs:398-412): bodies joined by a
+// joint with collide_connected off do not collide
+__device__ inline bool joined_no_collide(int ba, int bb, const int* __restrict__ nc_off,
+                                         const int* __restrict__ nc_list) {
+  for (int i = nc_off[ba], e = nc_off[ba + 1]; i < e; ++i)
+    if (nc_list[i] == bb) return true;
+  return false;
+}
+
+struct PairFilter {
+  const int* __restrict__ fbody;
+  const int* __restrict__ btype;
+  const int2* __restrict__ filter;
+  const int4* __restrict__ fshape;
+  const int* __restrict__ world;
+  const int* __restrict__ nc_off;   // null: no joint forbids a collision
+  const int* __restrict__ nc_list;
+  __device__ bool ok(int q, int p) const {
+    int bq = fbody[q], bp = fbody[p];
+    if (bq == bp) return false;
+    if (world[q] != world[p]) return false;  // batched worlds never interact
+    // B2body::should_collide: at least one body dynamic (src/private/dynamics/b2_body.rs:391-416)
+    if (btype[bq] != 2 && btype[bp] != 2) return false;
+    if (nc_off && joined_no_collide(bq, bp, nc_off, nc_list)) return false;
+    // default contact filter (src/private/dynamics/b2_world_callbacks.rs:6-18)
+    int2 fq = filter[q], fp = filter[p];
+    if (fq.y == fp.y && fq.y != 0) {
+      if (fq.y < 0) return false;
+    } else {
+      unsigned catq = fq.x & 0xffff, maskq = (unsigned(fq.x) >> 16) & 0xffff;
+      unsigned catp = fp.x & 0xffff, maskp = (unsigned(fp.x) >> 16) & 0xffff;
+      if ((maskq & catp) == 0 || (catq & maskp) == 0) return false;
+    }
+    // a contact class must exist for the shape pair
+    return registry_swap(fshape[q].x & 0xff, fshape[p].x & 0xff) >= 0;
+  }
+};
 
 // B2fixture::synchronize + B2dynamicTree::move_proxy for proxy i of body b
 // (src/private/dynamics/b2_fixture.rs:147-173, src/private/collision/b2_dynamic_tree.rs:109-168):

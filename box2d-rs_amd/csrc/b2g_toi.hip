@@ -18,6 +18,9 @@
 //   re-fattened: the host rebuilds the contact set (find_new_contacts), lists the contacts whose
 //   time is not cached (k_toi_need) and recomputes them (k_toi_rescan: ranked into set order, the
 //   reference's sweep alignment on one thread in that order, the times in parallel).
+// * Separable passes (k_toi_scan, k_toi_bodies): without bullets and kinematic bodies every event
+//   moves one dynamic body against static ones, so the bodies' events are independent of each other
+//   and each body's run on a wave of its own, all at once (see "separable passes" below).
 // * Bullets: a contact gets a time of impact when one of its bodies is static, kinematic or a
 //   bullet, and a bullet's island gathers dynamic bodies too (src/private/dynamics/b2_world.rs:
 //   616-621, 770-777).
@@ -934,6 +937,408 @@ __global__ void __launch_bounds__(kLoopBlock) k_toi_loop(ToiArgs a, LoopArgs L) 
   }
 }
 
+// ---- separable passes ----------------------------------------------------------------------
+// Without kinematic bodies, bullets and sub-stepping, and with every static body at rest, an event
+// changes one dynamic body only: its contact is with a static body, its island gathers that body's
+// contacts with static bodies, and a static body's sweep is one point whatever its alpha0. The
+// events of different bodies then commute, and the sequence of k_toi_loop (smallest time first over
+// all contacts) restricted to one body is what that body would go through alone. So each body with
+// a time of impact below 1 runs its own events on one wave, all bodies side by side; the operations
+// on a body, and their order, are those of k_toi_loop, so the results are the same bit for bit.
+//
+// An event that re-fattens a proxy ends the sequence's use of the old contact set (find_new_contacts
+// follows each event). Only contacts with static bodies matter to the body's later events, and when
+// every static proxy is on its world's list of big ones (not in the BVH) the wave sees for itself
+// whether the new box meets one that it has no contact with (it then waits for the host's rebuild of
+// the set) or has left one that it has a contact with (that contact takes no further part, as the
+// rebuild would drop it). With static proxies in the BVH a re-fattened body always waits. The set is
+// rebuilt once at the end of the pass instead of after each such event.
+//
+// Bound by the latency of one body's chain of events (time of impact, manifolds, the island's solve),
+// which the waves of the other bodies overlap. The field of 65,536 bodies landing (about 400 events
+// a step): 22.5 ms a step in k_toi_loop, one event after another at 57 us each; here 45 us for the
+// scan over 390,000 contacts, 50 us for all events, and one rebuild instead of five (a step 25.4 ms
+// -> 1.6 ms). Stacks of 1,531 boxes, 40 steps with sleeping on: 59.8 -> 21.4 ms.
+constexpr int kSepMax = 62;         // contacts with static bodies of one body (2 + 62: as the LDS store)
+constexpr int kSepBlocks = 1024;    // waves launched; the queue is strided over
+
+struct SepCtl {
+  int queued, waiting, left, events, solved, pad[3];
+};
+
+struct SepArgs {
+  int* head;           // per body: first of its contacts with static bodies (-1: none)
+  int* next;           // per contact: the next one
+  int* queue;
+  int* queued;         // per body: in the queue
+  const int* bfix_off;
+  const int* bfix;
+  float4* faabb;
+  float4* ffat;
+  const int* loose_off;  // per world: its big static proxies
+  const int* loose;
+  int tree_statics;      // a static proxy is in the BVH
+  PairFilter pf;
+  SepCtl* ctl;
+};
+
+// Per body: no contacts, not queued; at the start of the pass its sweep starts at alpha0 = 0.
+__global__ void __launch_bounds__(kToiBlock) k_toi_begin(ToiArgs a, SepArgs p, int first) {
+  const int b = blockIdx.x * blockDim.x + threadIdx.x;
+  if (b == 0) {
+    p.ctl->queued = p.ctl->waiting = p.ctl->left = 0;
+    if (first) p.ctl->events = p.ctl->solved = 0;
+  }
+  if (b >= a.nb) return;
+  p.head[b] = -1;
+  p.queued[b] = 0;
+  if (first) a.alpha0[b] = 0.0f;
+}
+
+// One thread per contact of the set: contacts of a dynamic with a static body are linked to the
+// body, those without a cached time of impact get one, and the body of one below 1 is queued. The
+// two sweeps need no alignment in set order: the dynamic body's alpha0 is the largest (a static
+// body's is that of an earlier event), and a static sweep is the same at every alpha0.
+__global__ void __launch_bounds__(kToiBlock) k_toi_scan(ToiArgs a, SepArgs p, int first) {
+  const int k = blockIdx.x * blockDim.x + threadIdx.x;
+  if (k >= a.n) return;
+  if (first) {
+    a.tcount[k] = 0;
+    a.tflags[k] = 0;
+    a.toi[k] = 1.0f;
+  }
+  const int2 f = a.ab[k];
+  const int bA = a.fbody[f.x], bB = a.fbody[f.y];
+  const bool dA = a.btype[bA] == 2, dB = a.btype[bB] == 2;
+  if (dA == dB || (a.fshape[f.x].w | a.fshape[f.y].w)) return;
+  const int b = dA ? bA : bB;
+  p.next[k] = atomicExch(&p.head[b], k);
+  int flags = first ? 0 : a.tflags[k];
+  float t = first ? 1.0f : a.toi[k];
+  const int count = first ? 0 : a.tcount[k];
+  if (!(flags & (kToiValid | kToiDisabled)) && count <= kMaxSubSteps && is_awake(a, b)) {
+    SweepD sa = load_sweep(a, bA), sb = load_sweep(a, bB);
+    const float alpha0 = first ? 0.0f : a.alpha0[b];
+    sa.alpha0 = sb.alpha0 = alpha0;
+    t = toi_alpha(a, k, sa, sb, alpha0);
+    flags = kToiValid;
+    a.toi[k] = t;
+    a.tflags[k] = flags;
+  }
+  if (flags == kToiValid && count <= kMaxSubSteps && t < 1.0f && atomicExch(&p.queued[b], 1) == 0)
+    p.queue[atomicAdd(&p.ctl->queued, 1)] = b;
+}
+
+struct SepStore {
+  int n, raw[64], k[64];
+  int2 fab[64];
+  int dropped[64];
+  ContactConst c[64];
+  TGeom<float> geom[64];
+  float fr[64];
+  TPos<float> sp[64];  // the static body's position
+  TVelC<float> vc[64];
+  float lam[64][4];
+  SweepD sweep;        // the body's after the event
+  TVel<float> vel;
+  int refat, missing;
+};
+
+__device__ inline Xf sweep_end_xf(const SweepD& s) {
+  Xf x;
+  x.q = rot(s.a);
+  x.p = s.c - mul(x.q, s.lc);
+  return x;
+}
+
+__device__ inline void store_xf(const ToiArgs& a, int b, const Xf& x) {
+  a.xf[b] = make_float4(x.p.x, x.p.y, x.q.s, x.q.c);
+}
+
+// update_contact with the transforms in hand; the new manifold stays with the caller as well.
+// Returns whether it is touching; *changed: that changed (the body is woken).
+__device__ bool update_contact_xf(const ToiArgs& a, int k, int2 fab, const Xf& xa, const Xf& xb, int* type, int* count,
+                                  TGeom<float>* g, bool* changed) {
+  Manifold m;
+  evaluate(&m, a.shapes[fab.x], xa, a.shapes[fab.y], xb);
+  const int ocount = a.hdr[k] >> 8;
+  const uint2 oid = a.ids[k];
+  const float4 o0 = a.pt0[k], o1 = a.pt1[k];
+  float imp[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    if (i >= m.count) break;
+    if (ocount > 0 && m.id[i] == oid.x) {
+      imp[2 * i] = o0.z;
+      imp[2 * i + 1] = o0.w;
+    } else if (ocount > 1 && m.id[i] == oid.y) {
+      imp[2 * i] = o1.z;
+      imp[2 * i + 1] = o1.w;
+    }
+  }
+  a.hdr[k] = m.type | (m.count << 8);
+  a.geo[k] = make_float4(m.local_normal.x, m.local_normal.y, m.local_point.x, m.local_point.y);
+  a.pt0[k] = make_float4(m.lp[0].x, m.lp[0].y, imp[0], imp[1]);
+  a.pt1[k] = make_float4(m.lp[1].x, m.lp[1].y, imp[2], imp[3]);
+  a.ids[k] = make_uint2(m.id[0], m.id[1]);
+  *type = m.type;
+  *count = m.count;
+  g->ln = m.local_normal;
+  g->lpt = m.local_point;
+  g->lp[0] = m.lp[0];
+  g->lp[1] = m.lp[1];
+  *changed = (m.count > 0) != (ocount > 0);
+  return m.count > 0;
+}
+
+// B2island::solve_toi for the body and its touching contacts with static bodies: the event's
+// contact (lane `first`) first, the others of `mask` in set order (one thread). Static bodies keep
+// their positions and have no velocity, so each contact has its own copy of its static body.
+__device__ void sep_island(const ToiArgs& a, SepStore& s, unsigned long long mask, int first,
+                           unsigned long long body_is_a, const SweepD& at, TVel<float> V, float min_alpha) {
+  TPos<float> P;
+  P.c = at.c;
+  P.a = at.a;
+  const TVel<float> still = {v2(0.0f, 0.0f), 0.0f};
+  const unsigned long long others = mask & ~(1ull << first);
+  auto each = [&](auto&& fn) {
+    fn(first);
+    for (unsigned long long m = others; m; m &= m - 1) fn(__ffsll(static_cast<long long>(m)) - 1);
+  };
+  for (int it = 0; it < 20; ++it) {
+    float min_sep = 0.0f;
+    each([&](int j) {
+      TPos<float> S = s.sp[j];
+      const float sep = (body_is_a >> j) & 1 ? solve_position_t(s.c[j], s.geom[j], P, S, double(kToiBaumgarte))
+                                             : solve_position_t(s.c[j], s.geom[j], S, P, double(kToiBaumgarte));
+      min_sep = bmin(min_sep, sep);
+    });
+    if (min_sep >= -1.5f * kSlop) break;
+  }
+  SweepD sw = at;
+  sw.c0 = P.c;
+  sw.a0 = P.a;
+  each([&](int j) {
+    const bool ba = (body_is_a >> j) & 1;
+    const TPos<float> S = s.sp[j];
+    s.vc[j] = init_velocity_t(s.c[j], s.geom[j], s.fr[j], ba ? P : S, ba ? S : P, ba ? V : still, ba ? still : V,
+                              a.block_solve != 0);
+    s.lam[j][0] = s.lam[j][1] = s.lam[j][2] = s.lam[j][3] = 0.0f;
+  });
+  for (int it = 0; it < a.velocity_iterations; ++it)
+    each([&](int j) {
+      TVel<float> S = still;
+      if ((body_is_a >> j) & 1) solve_velocity_t(s.vc[j], s.c[j], s.lam[j], V, S, a.block_solve != 0);
+      else solve_velocity_t(s.vc[j], s.c[j], s.lam[j], S, V, a.block_solve != 0);
+    });
+  integrate_position_t(P, V, (1.0f - min_alpha) * a.dt);
+  sw.c = P.c;
+  sw.a = P.a;
+  s.sweep = sw;
+  s.vel = V;
+}
+
+// One wave per queued body, running the body's events. Lane i holds the body's i-th contact with a
+// static body in set order: its cached time of impact, its static body, its manifold update and its
+// new time of impact are that lane's work; the island's solve runs on lane 0.
+__global__ void __launch_bounds__(64) k_toi_bodies(ToiArgs a, SepArgs p) {
+  __shared__ SepStore s;
+  const int lane = threadIdx.x;
+  const int nq = p.ctl->queued;
+  for (int q = blockIdx.x; q < nq; q += gridDim.x) {
+    const int b = p.queue[q];
+    __syncthreads();  // the store is free again
+    if (lane == 0) {
+      int n = 0;
+      for (int k = p.head[b]; k >= 0; k = p.next[k], ++n)
+        if (n < 64) s.raw[n] = k;
+      s.n = n;
+    }
+    __syncthreads();
+    const int n = s.n;
+    if (n > kSepMax) {  // left to k_toi_loop
+      if (lane == 0) atomicAdd(&p.ctl->left, 1);
+      continue;
+    }
+    if (lane < n) {
+      const int x = s.raw[lane];
+      int r = 0;
+      for (int j = 0; j < n; ++j) r += s.raw[j] < x ? 1 : 0;
+      s.k[r] = x;
+    }
+    __syncthreads();
+    bool has = lane < n;
+    const int k = has ? s.k[lane] : 0;
+    int2 fab = make_int2(0, 0);
+    int stat = 0, flags = 0, count = 0;
+    float t = 1.0f;
+    bool is_a = false;
+    SweepD so = {};
+    if (has) {
+      fab = a.ab[k];
+      is_a = a.fbody[fab.x] == b;
+      stat = is_a ? a.fbody[fab.y] : a.fbody[fab.x];
+      so = load_sweep(a, stat);
+      flags = a.tflags[k];
+      count = a.tcount[k];
+      t = a.toi[k];
+      s.fab[lane] = fab;
+      s.dropped[lane] = 0;
+    }
+    const unsigned long long body_is_a = __ballot(is_a);
+    const Xf xs = sweep_end_xf(so);
+    SweepD sw = load_sweep(a, b);
+    bool awake = is_awake(a, b);
+    const float4 v4 = a.vel[b];
+    TVel<float> V = {v2(v4.x, v4.y), v4.z};
+    int events = 0, solved = 0;
+    bool waiting = false;
+    for (;;) {
+      unsigned long long best = ~0ull;
+      if (has && flags == kToiValid && count <= kMaxSubSteps && t < 1.0f) best = toi_key(t, k);
+      const unsigned long long mine = best;
+      best = wave_min_u64(best);
+      const float min_alpha = __uint_as_float(static_cast<unsigned>(best >> 32));
+      if (best == ~0ull || 1.0f - 10.0f * kFltEpsilon < min_alpha) break;
+      const int le = __ffsll(static_cast<long long>(__ballot(mine == best))) - 1;  // the event's contact
+      ++events;
+      // B2body::advance of the body (src/b2_body.rs:979-986)
+      const SweepD backup = sw;
+      sweep_advance(sw, min_alpha);
+      sw.c = sw.c0;
+      sw.a = sw.a0;
+      const Xf xb = sweep_end_xf(sw);
+      bool touching = false, changed = false;
+      int type = 0, points = 0;
+      TGeom<float> geom;
+      if (lane == le) {
+        touching = update_contact_xf(a, k, fab, is_a ? xb : xs, is_a ? xs : xb, &type, &points, &geom, &changed);
+        flags &= ~(kToiDisabled | kToiValid);
+        ++count;
+        if (!touching) flags |= kToiDisabled;
+        store_xf(a, stat, xs);
+      }
+      if (__ballot(changed)) {
+        if (lane == 0) set_awake(a, b);
+        awake = true;
+      }
+      if (!__ballot(touching)) {
+        sw = backup;
+        if (lane == 0) store_sweep(a, b, sw);
+        continue;
+      }
+      ++solved;
+      if (lane == 0) set_awake(a, b);
+      awake = true;
+      // the body's other contacts with static bodies, at the event's time
+      if (has && lane != le) {
+        touching = update_contact_xf(a, k, fab, is_a ? xb : xs, is_a ? xs : xb, &type, &points, &geom, &changed);
+        flags &= ~kToiDisabled;
+        store_xf(a, stat, xs);
+      }
+      if (touching) {
+        const float4 matA = a.fmat[fab.x], matB = a.fmat[fab.y];
+        const int bA = is_a ? b : stat, bB = is_a ? stat : b;
+        ContactConst c;
+        c.type = type;
+        c.count = points;
+        s.fr[lane] = sqrtf(matA.x * matB.x);  // mixing laws, src/b2_contact.rs:29-46
+        c.restitution = matA.y > matB.y ? matA.y : matB.y;
+        c.threshold = matA.z < matB.z ? matA.z : matB.z;
+        c.rA = __int_as_float(a.fshape[fab.x].z);
+        c.rB = __int_as_float(a.fshape[fab.y].z);
+        const float4 mA = a.bmass[bA], mB = a.bmass[bB];
+        c.mA = mA.x;
+        c.iA = mA.y;
+        c.mB = mB.x;
+        c.iB = mB.y;
+        c.lcA[0] = mA.z;
+        c.lcA[1] = mA.w;
+        c.lcB[0] = mB.z;
+        c.lcB[1] = mB.w;
+        s.c[lane] = c;
+        s.geom[lane] = geom;
+        s.sp[lane].c = so.c;
+        s.sp[lane].a = so.a;
+      }
+      const unsigned long long island = __ballot(touching);
+      if (lane == 0) s.refat = s.missing = 0;
+      __syncthreads();
+      if (lane == 0) {
+        sep_island(a, s, island, le, body_is_a, sw, V, min_alpha);
+        store_sweep(a, b, s.sweep);
+        a.vel[b] = make_float4(s.vel.v.x, s.vel.v.y, s.vel.w, 0.0f);
+      }
+      __syncthreads();
+      sw = s.sweep;
+      V = s.vel;
+      flags &= ~kToiValid;
+      // the body's proxies (sync_proxy reads the sweep stored above)
+      const int f0 = p.bfix_off[b], f1 = p.bfix_off[b + 1];
+      for (int i = f0 + lane; i < f1; i += 64) {
+        const int f = p.bfix[i];
+        const bool refat = sync_proxy(f, b, a.shapes[f], a.pos0, a.bmass, a.xf, p.faabb, p.ffat);
+        a.moved[f] = refat ? 1 : 0;
+        if (refat) s.refat = 1;
+      }
+      __syncthreads();
+      if (s.refat) {
+        if (p.tree_statics) {
+          waiting = true;
+          break;
+        }
+        if (has) {  // a contact whose boxes no longer meet takes no further part
+          const float4 fa = p.ffat[fab.x], fb = p.ffat[fab.y];
+          const Aabb x = {v2(fa.x, fa.y), v2(fa.z, fa.w)}, y = {v2(fb.x, fb.y), v2(fb.z, fb.w)};
+          if (!overlap(x, y)) {
+            has = false;
+            s.dropped[lane] = 1;
+          }
+        }
+        __syncthreads();
+        for (int i = f0; i < f1; ++i) {
+          const int f = p.bfix[i];
+          const float4 ff = p.ffat[f];
+          const Aabb x = {v2(ff.x, ff.y), v2(ff.z, ff.w)};
+          const int w = p.pf.world[f];
+          for (int e = p.loose_off[w] + lane; e < p.loose_off[w + 1]; e += 64) {
+            const int g = p.loose[e];
+            const float4 gf = p.ffat[g];
+            const Aabb y = {v2(gf.x, gf.y), v2(gf.z, gf.w)};
+            if (!overlap(x, y) || !p.pf.ok(f, g) || (a.fshape[f].w | a.fshape[g].w)) continue;
+            bool known = false;
+            for (int j = 0; j < n; ++j)
+              known = known || (!s.dropped[j] && ((s.fab[j].x == f && s.fab[j].y == g) ||
+                                                  (s.fab[j].x == g && s.fab[j].y == f)));
+            if (!known) s.missing = 1;
+          }
+        }
+        __syncthreads();
+        if (s.missing) {
+          waiting = true;
+          break;
+        }
+      }
+      if (has && !(flags & kToiDisabled) && count <= kMaxSubSteps && awake) {
+        SweepD sa = is_a ? sw : so, sb = is_a ? so : sw;
+        sa.alpha0 = sb.alpha0 = sw.alpha0;
+        t = toi_alpha(a, k, sa, sb, sw.alpha0);
+        flags = kToiValid;
+      }
+    }
+    if (lane < n) {
+      a.tflags[k] = flags;
+      a.tcount[k] = count;
+      a.toi[k] = t;
+    }
+    if (lane == 0) {
+      if (events) atomicAdd(&p.ctl->events, events);
+      if (solved) atomicAdd(&p.ctl->solved, solved);
+      if (waiting) atomicAdd(&p.ctl->waiting, 1);
+    }
+  }
+}
+
 }  // namespace
 
 static ToiArgs toi_args(World* w, float dt, int vi) {
@@ -1223,6 +1628,75 @@ int toi_carry_state(World* w) {
   return B2G_OK;
 }
 
+void toi_note_bodies(World* w) {
+  w->has_kinematic = w->has_bullet = false;
+  w->statics_still = true;
+  for (int b = 0; b < w->nb; ++b) {
+    w->has_bullet = w->has_bullet || w->h_bullet[b] != 0;
+    if (w->host_type[b] == B2G_KINEMATIC) w->has_kinematic = true;
+    if (w->host_type[b] != B2G_STATIC) continue;
+    const float4 p = w->h_pos[b], p0 = w->h_pos0[b], v = w->h_vel[b], m = w->h_mass[b];
+    w->statics_still = w->statics_still && p.x == p0.x && p.y == p0.y && p.z == p0.z && v.x == 0.0f && v.y == 0.0f &&
+                       v.z == 0.0f && m.x == 0.0f && m.y == 0.0f;
+  }
+}
+
+// The events of a separable pass. *dirty: an event changed manifolds after the last rebuild; *left:
+// bodies with more contacts with static bodies than a wave holds still have events to run.
+static int toi_separable(World* w, float dt, int vi, bool* dirty, bool* left) {
+  int st;
+  const int nb = w->nb;
+  if ((st = w->toi_head.reserve(nb)) || (st = w->toi_queue.reserve(nb)) || (st = w->toi_queued.reserve(nb))) return st;
+  SepCtl* host = reinterpret_cast<SepCtl*>(w->h_counters + kPinnedToi);
+  static_assert(kPinnedToi + sizeof(SepCtl) / sizeof(int) <= kPinnedInts, "pinned TOI counters");
+  // a body waits at most once per event, and its events are bounded by its contacts' counts
+  const long long kMaxRounds = 4ll * (kMaxSubSteps + 2) * (static_cast<long long>(w->n_pairs) + nb + 16);
+  long long solved = 0, events = 0;
+  for (long long round = 0;; ++round) {
+    const int n = w->n_pairs, first = round == 0;
+    if ((st = w->toi_next.reserve(pair_capacity(w, n)))) return st;
+    const ToiArgs a = toi_args(w, dt, vi);
+    const bool nc = w->n_nocollide > 0;
+    SepArgs p;
+    p.head = w->toi_head.p;
+    p.next = w->toi_next.p;
+    p.queue = w->toi_queue.p;
+    p.queued = w->toi_queued.p;
+    p.bfix_off = w->toi_bfix_off.p;
+    p.bfix = w->toi_bfix.p;
+    p.faabb = w->f.aabb.p;
+    p.ffat = w->f.fat.p;
+    p.loose_off = w->f.loose_off.p;
+    p.loose = w->f.loose.p;
+    p.tree_statics = w->tree_statics;
+    p.pf = PairFilter{w->f.body.p,  w->b.type.p,  w->f.filter.p,
+                      w->f.shape.p, w->f.world.p, nc ? w->j.nc_off.p : nullptr,
+                      nc ? w->j.nc_list.p : nullptr};
+    p.ctl = reinterpret_cast<SepCtl*>(w->toi_ctl.p);
+    hipLaunchKernelGGL(k_toi_begin, dim3(blocks_for(nb, kToiBlock)), dim3(kToiBlock), 0, w->stream, a, p, first);
+    if (n > 0) {
+      hipLaunchKernelGGL(k_toi_scan, dim3(blocks_for(n, kToiBlock)), dim3(kToiBlock), 0, w->stream, a, p, first);
+      hipLaunchKernelGGL(k_toi_bodies, dim3(std::min(nb, kSepBlocks)), dim3(64), 0, w->stream, a, p);
+    }
+    B2G_HIP(hipGetLastError());
+    B2G_HIP(hipMemcpyAsync(host, p.ctl, sizeof(SepCtl), hipMemcpyDeviceToHost, w->stream));
+    B2G_HIP(hipStreamSynchronize(w->stream));
+    if (host->events > events) *dirty = true;
+    events = host->events;
+    solved = host->solved;
+    *left = host->left > 0;
+    if (host->waiting == 0) break;
+    if (round > kMaxRounds) {
+      set_error("continuous collision: the TOI pass did not end");
+      return B2G_ERR_DEVICE;
+    }
+    if ((st = toi_rebuild(w))) return st;
+    *dirty = false;
+  }
+  w->toi_events += static_cast<int>(solved);
+  return B2G_OK;
+}
+
 // The TOI pass after the solve (src/private/dynamics/b2_world.rs:534-901). The current contact
 // set is the one find_new_contacts left. The events run on the device (k_toi_loop); the host
 // rebuilds the contact set when an event re-fattened a proxy. A pass starts from alpha0 = 0 and no
@@ -1235,11 +1709,25 @@ int phase_toi(World* w, float dt, int vi) {
   if ((st = carry_manifolds_for_toi(w))) return st;
   if ((st = toi_reserve(w))) return st;
   if ((st = toi_body_fixtures(w))) return st;
+  bool dirty = false;
+  // the check of the global island store (b2g_world_tune) runs every event in k_toi_loop
+  const bool separable = !resume && !w->sub_stepping && !w->has_kinematic && !w->has_bullet && w->statics_still &&
+                         !w->toi_force_big;
+  if (separable && w->nb > 0) {
+    bool left = false;
+    if ((st = toi_separable(w, dt, vi, &dirty, &left))) return st;
+    if (!left) {
+      w->step_complete = true;
+      return dirty ? toi_rebuild(w) : B2G_OK;
+    }
+  }
   static const ToiCtl kReset = {~0ull, 0, 0, {0, 0}, {0, 0, 0, 0}, 0, 0, 0, 0};
   B2G_HIP(hipMemcpyAsync(w->toi_ctl.p, &kReset, sizeof(kReset), hipMemcpyHostToDevice, w->stream));
   if (w->n_pairs > 0) {
     const ToiArgs b = toi_args(w, dt, vi);
-    if (!resume) {
+    if (separable) {
+      // every contact has its time: only the bodies left by the waves have one below 1
+    } else if (!resume) {
       hipLaunchKernelGGL(k_toi_first, dim3(blocks_for(w->n_pairs, kToiBlock)), dim3(kToiBlock), 0, w->stream, b);
     } else {
       // the times the last sub-step's event invalidated, and those of pairs found since, in set
@@ -1252,7 +1740,6 @@ int phase_toi(World* w, float dt, int vi) {
     B2G_HIP(hipGetLastError());
   }
   if ((st = toi_loop_setup(w, dt, vi))) return st;
-  bool dirty = false;
   long long total = 0;
   // every event either disables its contact or raises its TOI count, so the pass ends; the bound
   // is a guard against a logic error, not a limit of the reference

@@ -1,0 +1,137 @@
+"""Separable TOI passes (k_toi_bodies: each body's events on a wave of its own, all bodies at once)
+against the pass that runs one event after another over the whole world (k_toi_loop, which the check of
+the global island store forces): the operations on a body and their order are the same, so body states,
+boxes, contacts with their manifolds and event counts agree bit for bit.
+
+Scenes, where the routes differ most: a rain onto one big static box (not in the BVH: re-fattened bodies go
+on without a rebuild), onto many small static tiles (in the BVH: they wait for one), into a corner of walls
+and a rotated ramp (several static contacts in one island), with sleeping on, batched worlds, and a plank
+over 61, 62, 63 and 70 static fixtures (62 is the most that a wave holds; beyond, k_toi_loop takes the body).
+"""
+import numpy as np
+import pytest
+
+import b2g
+
+pytestmark = pytest.mark.gpu
+
+DT = np.float32(1.0 / 60.0)
+
+
+def _defs(n, nf):
+    bd = np.zeros(n, b2g.BODY_DEF)
+    bd["gravity_scale"] = 1.0
+    bd["awake"] = bd["allow_sleep"] = 1
+    fd = np.zeros(nf, b2g.FIXTURE_DEF)
+    fd["friction"], fd["density"], fd["restitution_threshold"] = 0.4, 1.0, 1.0
+    fd["category"], fd["mask"] = 1, 0xFFFF
+    return bd, fd
+
+
+def _drops(rng, n, width, speed=70.0):
+    """n dynamic bodies (boxes and circles by turns, every fifth with two fixtures) above x in +-width."""
+    bd, _ = _defs(n, 0)
+    bd["type"] = 2
+    bd["position"] = np.stack([rng.uniform(-width, width, n), rng.uniform(2.0, 9.0, n)], 1)
+    bd["linear_velocity"] = np.stack([rng.uniform(-20, 20, n), rng.uniform(-speed, -0.3 * speed, n)], 1)
+    bd["angular_velocity"] = rng.uniform(-20, 20, n)
+    bd["angle"] = rng.uniform(-3, 3, n)
+    fb, sd = [], []
+    for i in range(n):
+        for j in range(2 if i % 5 == 0 else 1):
+            s = np.zeros((), b2g.SHAPE_DEF)
+            if i % 2:
+                s["type"], s["radius"] = b2g.SHAPE_CIRCLE, rng.uniform(0.1, 0.4)
+                s["params"][:2] = (0.5 * j, 0.0)
+            else:
+                s["type"], s["flags"] = b2g.SHAPE_BOX, 1
+                s["params"][:5] = (rng.uniform(0.1, 0.4), rng.uniform(0.1, 0.4), 0.5 * j, 0.0, 0.3 * j)
+            fb.append(i)
+            sd.append(s)
+    return bd, np.array(fb, np.int32), np.stack(sd)
+
+
+def _box(hx, hy, cx=0.0, cy=0.0, angle=0.0):
+    s = np.zeros((), b2g.SHAPE_DEF)
+    s["type"], s["flags"] = b2g.SHAPE_BOX, 1
+    s["params"][:5] = (hx, hy, cx, cy, angle)
+    return s
+
+
+def _scene(kind, seed):
+    rng = np.random.default_rng(seed)
+    if kind.startswith("plank"):
+        n = int(kind[5:])
+        bd, fd = _defs(2, n + 1)
+        bd[1]["type"], bd[1]["position"], bd[1]["linear_velocity"] = 2, (0.0, 2.0), (0.0, -60.0)
+        xs = (np.arange(n) - 0.5 * (n - 1)) * 0.3
+        sd = np.stack([_box(0.15, 0.25, x) for x in xs] + [_box(0.2 * n, 0.1)])
+        return bd, np.array([0] * n + [1], np.int32), sd, fd
+    dyn, dfb, dsd = _drops(rng, 60, 12.0)
+    if kind == "tiles":
+        static = [_box(0.5, 0.05, x, 0.02 * (i % 3)) for i, x in enumerate(np.arange(-16.0, 16.5, 1.0))]
+    elif kind == "corner":
+        static = [_box(30.0, 0.05), _box(0.05, 30.0, -8.0), _box(0.05, 30.0, 8.0), _box(20.0, 0.05, 0.0, 1.0, 0.2)]
+    else:
+        static = [_box(30.0, 0.05)]
+    bd, fd = _defs(1, len(static) + len(dsd))
+    bd["angle"] = 0.1 if kind == "corner" else 0.0
+    return np.concatenate([bd, dyn]), np.concatenate([np.zeros(len(static), np.int32), 1 + dfb]), \
+        np.concatenate([np.stack(static), dsd]), fd
+
+
+def _run(scenes, sleep, steps, sequential):
+    w = b2g.World((0.0, -10.0))
+    w.set_flags(warm_starting=True, allow_sleep=sleep, continuous=True, block_solve=True)
+    if len(scenes) == 1:
+        w.add(*scenes[0])
+    else:
+        base = np.cumsum([0] + [len(s[0]) for s in scenes])
+        w.add_batched(np.concatenate([s[0] for s in scenes]), np.repeat(np.arange(len(scenes)), np.diff(base)),
+                      np.concatenate([s[1] + o for s, o in zip(scenes, base)]), np.concatenate([s[2] for s in scenes]),
+                      np.concatenate([s[3] for s in scenes]))
+    w.tune(b2g.TUNE_TOI_GLOBAL_ISLAND, int(sequential))
+    out, events = [], 0
+    for _ in range(steps):
+        w.step(DT, 8, 3)
+        e = w.profile()["toi_events"]
+        events += e
+        fab, flags, man = w.contacts()
+        out.append((e, w.body_states().tobytes(), w.fat_aabbs().tobytes(), fab.tobytes(), flags.tobytes(), man.tobytes()))
+    w.close()
+    return out, events
+
+
+@pytest.mark.parametrize("kind,sleep", [("ground", False), ("ground", True), ("tiles", False), ("tiles", True),
+                                        ("corner", False), ("corner", True), ("plank61", False), ("plank62", False),
+                                        ("plank63", False), ("plank70", False), ("batch", False)])
+def test_separable_pass_matches_the_sequential_one(kind, sleep):
+    scenes = [_scene("ground", 40 + i) for i in range(5)] if kind == "batch" else [_scene(kind, 11)]
+    steps = 12 if kind.startswith("plank") else 70
+    seq, events = _run(scenes, sleep, steps, True)
+    sep, _ = _run(scenes, sleep, steps, False)
+    assert events >= (1 if kind.startswith("plank") else 60)
+    for step, (x, y) in enumerate(zip(seq, sep)):
+        assert x[0] == y[0], "step %d: %d events, %d in the separable pass" % (step, x[0], y[0])
+        for name, u, v in zip(("states", "boxes", "contacts", "touching", "manifolds"), x[1:], y[1:]):
+            assert u == v, "step %d: %s differ" % (step, name)
+
+
+def test_moved_static_body_takes_the_sequential_pass():
+    """A static body whose sweep start is not its end (set_body_states) is a moving obstacle to the pass:
+    the events then depend on its alpha0, so they run one after another; both settings agree."""
+    out = []
+    for sequential in (True, False):
+        w = b2g.World((0.0, -10.0))
+        w.set_flags(warm_starting=True, allow_sleep=False, continuous=True, block_solve=True)
+        w.add(*_scene("ground", 3))
+        w.tune(b2g.TUNE_TOI_GLOBAL_ISLAND, int(sequential))
+        w.step(DT, 8, 3)
+        st = w.body_states()
+        st["c0"][0] = (0.0, -0.05)
+        w.set_body_states(st)
+        for _ in range(10):
+            w.step(DT, 8, 3)
+        out.append(w.body_states().tobytes())
+        w.close()
+    assert out[0] == out[1]
