@@ -9,14 +9,24 @@
 //
 // Backward: segments are replayed from their checkpoint with the frozen step (the recorded
 // contact set, features, solve order and iteration counts; all continuous quantities
-// recomputed by the templated step functions), keeping each step's start state; steps are then
-// reversed one by one: the step is replayed once more keeping every constraint's inputs, and
-// the vector-Jacobian products of b2g_adjoint_t.h are applied in reverse order -- position
+// recomputed by the templated step functions), keeping each step's start state and every
+// constraint's inputs (or, where a segment's do not fit kKeepBytes, replaying each step once more
+// for them); steps are then reversed one by one: the reverse functions of b2g_adjoint_t.h are applied in reverse order -- position
 // iterations (colours reversed), position integration, impulse storage, velocity iterations,
 // warm start, constraint initialisation and collide geometry, velocity integration. Within a
 // colour no two constraints share a dynamic body, so a colour's reverse pass is parallel like
 // its forward pass; contributions that several constraints make to one body (through the
 // constraint set-up and the manifold geometry) are accumulated with atomics.
+//
+// Where the recorded solve was grouped (bins of islands, worlds of a batch: no two groups share a
+// dynamic body), one workgroup runs a group's iterations with a constraint per thread, the
+// constraint and its cotangents in registers and the group's bodies in LDS, as k_solve_bins_* do:
+// one launch for all velocity iterations instead of one per colour and iteration. Steps that were not
+// grouped, or hold a group of more than 512 constraints, launch per colour.
+//
+// 192 worlds of 64 bodies, 30 steps, forward and backward: 128.7 -> 25.7 ms (9,500 launches -> 1,940), where
+// dual numbers per colour took 31 us per launch of the reverse velocity solve (1.6 ms a step) against
+// 82 us a step for k_ab_group_vel and 51 us for k_ab_init.
 #include "b2g_adjoint_t.h"
 #include "b2g_internal.h"
 
@@ -68,8 +78,10 @@ __global__ void __launch_bounds__(kBlock) k_tape_post(int nc, long long off, int
                                                       const long long* __restrict__ prev_slot,
                                                       long long* __restrict__ cur_slot, int4* __restrict__ t_slot,
                                                       int4* __restrict__ t_meta, uint2* __restrict__ t_ids,
-                                                      float4* __restrict__ t_lam0, float4* __restrict__ t_store) {
+                                                      float4* __restrict__ t_lam0, float4* __restrict__ t_store,
+                                                      int* __restrict__ group_max) {
   int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i == 0) *group_max = 0;
   if (i >= nc) return;
   const int k = k_contact[i];
   const long long s = off + i;
@@ -96,13 +108,36 @@ __global__ void __launch_bounds__(kBlock) k_tape_post(int nc, long long off, int
   cur_slot[k] = s;
 }
 
+// the step's (colour, group) offsets, and the size of its largest group
+__global__ void __launch_bounds__(kBlock) k_tape_groups(int ng, int ncolors, const int* __restrict__ off,
+                                                        int* __restrict__ out, int* __restrict__ group_max) {
+  const int g = blockIdx.x * blockDim.x + threadIdx.x;
+  if (g >= ng) return;
+  int n = 0;
+  for (int c = 0; c < ncolors; ++c) {
+    const int b0 = off[c * ng + g];
+    out[c * ng + g] = b0;
+    n += off[c * ng + g + 1] - b0;
+  }
+  if (g == 0) out[ncolors * ng] = off[ncolors * ng];
+  if (n > 0) atomicMax(group_max, n);
+}
+
 void tape_release(World* w) {
+  tape_reset(w);
   Tape& t = w->tape;
+  t.buf.release();
+  t.group_off.release(); t.group_max.release();
   t.slot.release(); t.meta.release(); t.ids.release(); t.lam0.release(); t.lam_store.release();
   t.c_lam0.release(); t.c_carry.release(); t.c_slot[0].release(); t.c_slot[1].release();
   t.ck_pos.release(); t.ck_vel.release();
+}
+
+void tape_reset(World* w) {
+  Tape& t = w->tape;
   t.steps.clear();
   t.total = 0;
+  t.group_total = 0;
   t.ck_count = 0;
   t.active = false;
   t.has_prev = false;
@@ -158,14 +193,18 @@ int tape_after_solve(World* w, float dt, float dt_ratio, int vel_iters, int pos_
   }
   int st;
   const size_t need = size_t(t.total + std::max(nc, 1));
+  const int ncolors = w->n_colors, ng = nc > 0 ? w->solve_groups : 0;
+  const size_t nsteps = t.steps.size();
+  const size_t gneed = size_t(t.group_total) + size_t(ng) * ncolors + 1;
   // a growing array copies its contents outside the world's stream: let the stream finish first
   if (need > t.slot.cap || need > t.meta.cap || need > t.ids.cap || need > t.lam0.cap || need > t.lam_store.cap ||
-      size_t(std::max(np, 1)) > t.c_slot[w->cur].cap)
+      size_t(std::max(np, 1)) > t.c_slot[w->cur].cap || gneed > t.group_off.cap || nsteps + 1 > t.group_max.cap)
     B2G_HIP(hipStreamSynchronize(w->stream));
   if ((st = t.slot.reserve(need, true, t.total)) || (st = t.meta.reserve(need, true, t.total)) ||
       (st = t.ids.reserve(need, true, t.total)) || (st = t.lam0.reserve(need, true, t.total)) ||
       (st = t.lam_store.reserve(need, true, t.total)) || (st = t.c_slot[w->cur].reserve(std::max(np, 1))) ||
-      (st = t.c_slot[1 - w->cur].reserve(1)))
+      (st = t.c_slot[1 - w->cur].reserve(1)) || (st = t.group_off.reserve(gneed, true, t.group_total)) ||
+      (st = t.group_max.reserve(nsteps + 1, true, nsteps)))
     return st;
   if (np > 0)
     hipLaunchKernelGGL(k_fill_ll, dim3(blocks_for(np, kBlock)), dim3(kBlock), 0, w->stream, static_cast<long long>(np),
@@ -176,7 +215,11 @@ int tape_after_solve(World* w, float dt, float dt_ratio, int vel_iters, int pos_
     hipLaunchKernelGGL(k_tape_post, dim3(blocks_for(nc, kBlock)), dim3(kBlock), 0, w->stream, nc, t.total,
                        int(t.has_prev), pos_iters, s.k_contact.p, s.k_bodies.p, s.k_info.p, s.isl_done.p, c.ab.p,
                        c.hdr.p, c.ids.p, c.pt0.p, c.pt1.p, t.c_lam0.p, t.c_carry.p, t.c_slot[1 - w->cur].p,
-                       t.c_slot[w->cur].p, t.slot.p, t.meta.p, t.ids.p, t.lam0.p, t.lam_store.p);
+                       t.c_slot[w->cur].p, t.slot.p, t.meta.p, t.ids.p, t.lam0.p, t.lam_store.p,
+                       t.group_max.p + nsteps);
+    if (ng > 0)
+      hipLaunchKernelGGL(k_tape_groups, dim3(blocks_for(ng, kBlock)), dim3(kBlock), 0, w->stream, ng, ncolors,
+                         s.cw_off.p, t.group_off.p + t.group_total, t.group_max.p + nsteps);
   }
   B2G_HIP(hipGetLastError());
   TapeStep ts;
@@ -184,6 +227,9 @@ int tape_after_solve(World* w, float dt, float dt_ratio, int vel_iters, int pos_
   ts.off = t.total;
   if (nc > 0) ts.color_off = w->h_color_off;
   else ts.color_off.assign(1, 0);
+  ts.ng = ng;
+  ts.goff = t.group_total;
+  if (ng > 0) t.group_total += static_cast<long long>(ng) * ncolors + 1;
   ts.dt = dt;
   ts.dt_ratio = dt_ratio;
   ts.vel_iters = vel_iters;
@@ -219,12 +265,12 @@ struct AdjCtx {
   int warm, block, record;
   // state
   float4 *pos, *vel;
-  const float4 *pos_n, *vel_n;  // at the start of the step
-  float4 *vstar, *geom, *lam_cur, *lam_init, *lam0eff;
-  float4 *t_ws, *t_vel, *t_ip, *t_pos;
+  float4 *pos_n, *vel_n;  // at the start of the step
+  float4 *vstar, *geom, *velc, *lam_cur, *lam_init, *lam0eff;
+  float4 *t_vel, *t_ip, *t_pos;
   // cotangents
-  float4 *pbar, *vbar, *lambar, *lam0bar, *qnbar, *gbar, *vsbar, *store_bar;
-  float *fricbar, *fric_grad;
+  float4 *pbar, *vbar, *lambar, *lam0bar, *qnbar, *gbar, *vsbar, *velcbar, *store_bar;
+  float* fric_grad;
   int* err;
 };
 
@@ -243,24 +289,61 @@ __device__ inline ContactConst contact_const(const AdjCtx& a, int4 sl, int hdr) 
   return k;
 }
 
+// what the velocity solve needs of it (the rest stays unset)
+__device__ inline ContactConst velocity_const(const AdjCtx& a, int4 sl) {
+  ContactConst k;
+  const float4 A = a.bmass[sl.x], B = a.bmass[sl.y];
+  k.mA = A.x; k.iA = A.y; k.mB = B.x; k.iB = B.y;
+  return k;
+}
+
 __device__ inline float friction_of(const AdjCtx& a, int4 sl) { return sqrtf(a.fmat[sl.z].x * a.fmat[sl.w].x); }
 
 __device__ inline void put3(float* x, float4 v) { x[0] = v.x; x[1] = v.y; x[2] = v.z; }
 __device__ inline float4 f4(const float* x) { return make_float4(x[0], x[1], x[2], 0.0f); }
+__device__ inline TVel<float> vel_from(float4 v) { return TVel<float>{v2(v.x, v.y), v.z}; }
+__device__ inline TPos<float> pos_from(float4 p) { return TPos<float>{v2(p.x, p.y), p.z}; }
+__device__ inline float4 f4(const TVel<float>& v) { return make_float4(v.v.x, v.v.y, v.w, 0.0f); }
+__device__ inline float4 f4(const TPos<float>& p) { return make_float4(p.c.x, p.c.y, p.a, 0.0f); }
 
-// the 31 inputs of the velocity-phase functors (b2g_adjoint_t.h)
-__device__ inline void vel_inputs(const AdjCtx& a, int i, int4 sl, float4 vA, float4 vB, float4 lam, float* x) {
-  put3(x, vA);
-  put3(x + 3, vB);
-  x[6] = lam.x; x[7] = lam.y; x[8] = lam.z; x[9] = lam.w;
-  put3(x + 10, a.pos_n[sl.x]);
-  put3(x + 13, a.pos_n[sl.y]);
-  const float4 g0 = a.geom[2 * i], g1 = a.geom[2 * i + 1];
-  x[16] = g0.x; x[17] = g0.y; x[18] = g0.z; x[19] = g0.w;
-  x[20] = g1.x; x[21] = g1.y; x[22] = g1.z; x[23] = g1.w;
-  x[24] = friction_of(a, sl);
-  put3(x + 25, a.vstar[sl.x]);
-  put3(x + 28, a.vstar[sl.y]);
+__device__ inline TGeom<float> load_geom(const float4* g) {
+  const float4 g0 = g[0], g1 = g[1];
+  TGeom<float> r;
+  r.ln = v2(g0.x, g0.y);
+  r.lpt = v2(g0.z, g0.w);
+  r.lp[0] = v2(g1.x, g1.y);
+  r.lp[1] = v2(g1.z, g1.w);
+  return r;
+}
+__device__ inline void store_geom(float4* g, const TGeom<float>& r) {
+  g[0] = make_float4(r.ln.x, r.ln.y, r.lpt.x, r.lpt.y);
+  g[1] = make_float4(r.lp[0].x, r.lp[0].y, r.lp[1].x, r.lp[1].y);
+}
+
+// a velocity constraint (or its cotangents) as kVelcRows float4
+constexpr int kVelcRows = 7;
+__device__ inline TVelC<float> load_velc(const float4* q) {
+  const float4 r0 = q[0], r1 = q[1], r2 = q[2], r3 = q[3], r4 = q[4], r5 = q[5], r6 = q[6];
+  TVelC<float> c;
+  c.normal = v2(r0.x, r0.y);
+  c.friction = r0.z;
+  c.vcount = __float_as_int(r0.w);
+  c.ra[0] = v2(r1.x, r1.y); c.rb[0] = v2(r1.z, r1.w);
+  c.ra[1] = v2(r2.x, r2.y); c.rb[1] = v2(r2.z, r2.w);
+  c.nm[0] = r3.x; c.tm[0] = r3.y; c.nm[1] = r3.z; c.tm[1] = r3.w;
+  c.bias[0] = r4.x; c.bias[1] = r4.y;
+  c.K[0] = r5.x; c.K[1] = r5.y; c.K[2] = r5.z; c.K[3] = r5.w;
+  c.NM[0] = r6.x; c.NM[1] = r6.y; c.NM[2] = r6.z; c.NM[3] = r6.w;
+  return c;
+}
+__device__ inline void store_velc(float4* q, const TVelC<float>& c) {
+  q[0] = make_float4(c.normal.x, c.normal.y, c.friction, __int_as_float(c.vcount));
+  q[1] = make_float4(c.ra[0].x, c.ra[0].y, c.rb[0].x, c.rb[0].y);
+  q[2] = make_float4(c.ra[1].x, c.ra[1].y, c.rb[1].x, c.rb[1].y);
+  q[3] = make_float4(c.nm[0], c.tm[0], c.nm[1], c.tm[1]);
+  q[4] = make_float4(c.bias[0], c.bias[1], 0.0f, 0.0f);
+  q[5] = make_float4(c.K[0], c.K[1], c.K[2], c.K[3]);
+  q[6] = make_float4(c.NM[0], c.NM[1], c.NM[2], c.NM[3]);
 }
 
 __device__ inline TBodyMass<float> body_mass(const AdjCtx& a, int b) {
@@ -272,32 +355,20 @@ __device__ inline TBodyMass<float> body_mass(const AdjCtx& a, int b) {
 }
 
 // -- forward replay
-__global__ void __launch_bounds__(kBlock) k_af_geom(AdjCtx a) {
-  int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= a.n) return;
-  const long long s = a.off + i;
-  const int4 sl = a.slot[s];
-  const int4 mt = a.meta[s];
-  const ShapeV &sa = a.shapes[sl.z], &sb = a.shapes[sl.w];
-  const float4 A = a.bmass[sl.x], B = a.bmass[sl.y];
-  const float lcA[2] = {A.z, A.w}, lcB[2] = {B.z, B.w};
-  int hdr = 0;
-  uint32_t id[2] = {0, 0};
-  GeomFn<float> f{&sa, &sb, lcA, lcB, &hdr, id};
-  float x[6], y[8];
-  put3(x, a.pos_n[sl.x]);
-  put3(x + 3, a.pos_n[sl.y]);
-  f(x, y);
-  const uint2 rid = a.ids[s];
-  if (hdr != mt.x || id[0] != rid.x || id[1] != rid.y) atomicOr(a.err, 1);
-  a.geom[2 * i] = make_float4(y[0], y[1], y[2], y[3]);
-  a.geom[2 * i + 1] = make_float4(y[4], y[5], y[6], y[7]);
-}
-
-__global__ void __launch_bounds__(kBlock) k_af_intvel(AdjCtx a) {
+// Per body: the step's start state kept (or, for the recorded replay, taken back), and the velocity
+// integration.
+__global__ void __launch_bounds__(kBlock) k_af_begin(AdjCtx a, int take_back) {
   int b = blockIdx.x * blockDim.x + threadIdx.x;
   if (b >= a.nb) return;
-  float4 v = a.vel[b];
+  float4 v;
+  if (take_back) {
+    a.pos[b] = a.pos_n[b];
+    v = a.vel_n[b];
+  } else {
+    v = a.vel[b];
+    a.pos_n[b] = a.pos[b];
+    a.vel_n[b] = v;
+  }
   if (a.btype[b] == 2) {
     const float4 f = a.force[b];
     IntVelFn<float> fn{body_mass(a, b), f.x, f.y, f.z, a.gx, a.gy, a.dt};
@@ -305,8 +376,8 @@ __global__ void __launch_bounds__(kBlock) k_af_intvel(AdjCtx a) {
     put3(x, v);
     fn(x, y);
     v = f4(y);
-    a.vel[b] = v;
   }
+  a.vel[b] = v;
   a.vstar[b] = v;
 }
 
@@ -316,12 +387,30 @@ __device__ inline float4 carried(const AdjCtx& a, int src, float n0, float t0) {
   return (src & 1) ? make_float4(s.z, s.w, 0.0f, 0.0f) : make_float4(s.x, s.y, 0.0f, 0.0f);
 }
 
-__global__ void __launch_bounds__(kBlock) k_af_lam(AdjCtx a) {
+// Per slot: manifold geometry (checked against the recorded features), carried impulses and the
+// constraint record, which the iterations then read instead of computing it anew each time.
+__global__ void __launch_bounds__(kBlock) k_af_init(AdjCtx a) {
   int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= a.n) return;
   const long long s = a.off + i;
+  const int4 sl = a.slot[s];
   const int4 mt = a.meta[s];
-  const int count = mt.x >> 8;
+  const ContactConst k = contact_const(a, sl, mt.x);
+  const float4 pA = a.pos_n[sl.x], pB = a.pos_n[sl.y];
+  float x[6], y[8];
+  put3(x, pA);
+  put3(x + 3, pB);
+  int hdr = 0;
+  uint32_t id[2] = {0, 0};
+  GeomFn<float> f{&a.shapes[sl.z], &a.shapes[sl.w], k.lcA, k.lcB, &hdr, id};
+  f(x, y);
+  const uint2 rid = a.ids[s];
+  if (hdr != mt.x || id[0] != rid.x || id[1] != rid.y) atomicOr(a.err, 1);
+  const TGeom<float> g = geom_of(y);
+  store_geom(a.geom + 2 * i, g);
+  const TVelC<float> c = init_velocity_t(k, g, friction_of(a, sl), pos_from(pA), pos_from(pB), vel_from(a.vstar[sl.x]),
+                                         vel_from(a.vstar[sl.y]), a.block != 0);
+  store_velc(a.velc + kVelcRows * i, c);
   const float4 l0 = a.lam0[s];
   const float4 c0 = carried(a, mt.y, l0.x, l0.y), c1 = carried(a, mt.z, l0.z, l0.w);
   const float4 e = make_float4(c0.x, c0.y, c1.x, c1.y);
@@ -330,7 +419,7 @@ __global__ void __launch_bounds__(kBlock) k_af_lam(AdjCtx a) {
   if (a.warm) {
     li.x = a.dt_ratio * e.x;
     li.y = a.dt_ratio * e.y;
-    if (count > 1) {
+    if (k.count > 1) {
       li.z = a.dt_ratio * e.z;
       li.w = a.dt_ratio * e.w;
     }
@@ -339,72 +428,18 @@ __global__ void __launch_bounds__(kBlock) k_af_lam(AdjCtx a) {
   a.lam_cur[i] = li;
 }
 
-__global__ void __launch_bounds__(kBlock) k_af_warm(AdjCtx a, int b0, int b1) {
-  int i = b0 + blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= b1) return;
-  const long long s = a.off + i;
-  const int4 sl = a.slot[s];
-  const ContactConst k = contact_const(a, sl, a.meta[s].x);
-  const float4 vA = a.vel[sl.x], vB = a.vel[sl.y];
-  if (a.record) {
-    a.t_ws[2 * i] = vA;
-    a.t_ws[2 * i + 1] = vB;
-  }
-  float x[kVelIn], y[6];
-  vel_inputs(a, i, sl, vA, vB, a.lam_cur[i], x);
-  WarmFn<float> fn{k, a.block != 0};
-  fn(x, y);
-  if (a.btype[sl.x] == 2) a.vel[sl.x] = f4(y);
-  if (a.btype[sl.y] == 2) a.vel[sl.y] = f4(y + 3);
-}
-
-__global__ void __launch_bounds__(kBlock) k_af_vel(AdjCtx a, int b0, int b1, int it) {
-  int i = b0 + blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= b1) return;
-  const long long s = a.off + i;
-  const int4 sl = a.slot[s];
-  const ContactConst k = contact_const(a, sl, a.meta[s].x);
-  const float4 vA = a.vel[sl.x], vB = a.vel[sl.y], lam = a.lam_cur[i];
-  if (a.record) {
-    float4* t = a.t_vel + 3 * (size_t(it) * a.n + i);
-    t[0] = vA;
-    t[1] = vB;
-    t[2] = lam;
-  }
-  float x[kVelIn], y[10];
-  vel_inputs(a, i, sl, vA, vB, lam, x);
-  VelFn<float> fn{k, a.block != 0};
-  fn(x, y);
-  if (a.btype[sl.x] == 2) a.vel[sl.x] = f4(y);
-  if (a.btype[sl.y] == 2) a.vel[sl.y] = f4(y + 3);
-  a.lam_cur[i] = make_float4(y[6], y[7], y[8], y[9]);
-}
-
-// velocity point count of a constraint (the block solver may drop to one point)
-__device__ inline int vcount_of(const AdjCtx& a, int i, int4 sl, const ContactConst& k) {
-  float x[kVelIn];
-  vel_inputs(a, i, sl, make_float4(0.0f, 0.0f, 0.0f, 0.0f), make_float4(0.0f, 0.0f, 0.0f, 0.0f),
-             make_float4(0.0f, 0.0f, 0.0f, 0.0f), x);
-  return velc_of(x, k, a.block != 0).vcount;
-}
-
-__global__ void __launch_bounds__(kBlock) k_af_store(AdjCtx a) {
-  int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= a.n) return;
-  const long long s = a.off + i;
-  const int4 sl = a.slot[s];
-  const ContactConst k = contact_const(a, sl, a.meta[s].x);
-  const int vc = vcount_of(a, i, sl, k);
-  const float4 l = a.lam_cur[i], e = a.lam0eff[i];
+// store_impulses: the velocity point count may have dropped to one
+__device__ inline float4 stored_impulses(const AdjCtx& a, int i, int count, int vcount, float4 l) {
   float4 out = make_float4(l.x, l.y, 0.0f, 0.0f);
-  if (vc > 1) {
+  if (vcount > 1) {
     out.z = l.z;
     out.w = l.w;
-  } else if (k.count > 1) {
+  } else if (count > 1) {
+    const float4 e = a.lam0eff[i];
     out.z = e.z;
     out.w = e.w;
   }
-  a.lam_store[s] = out;
+  return out;
 }
 
 __global__ void __launch_bounds__(kBlock) k_af_intpos(AdjCtx a) {
@@ -425,6 +460,297 @@ __global__ void __launch_bounds__(kBlock) k_af_intpos(AdjCtx a) {
   a.vel[b] = f4(y + 3);
 }
 
+// ---- groups: a workgroup per group, a constraint per thread ---------------------------------------
+// The group's bodies sit in an LDS hash table (as in k_solve_bins_velocity), its constraints in
+// registers; a barrier separates the colours. Each phase is one constraint's chain of dependent
+// arithmetic, about a microsecond, whatever the number of constraints: bound by that latency times
+// colours times iterations, with the other groups' workgroups beside it.
+struct GroupView {
+  const int* off;  // [colour * ng + group]
+  int ng, ncolors, iters;
+};
+
+// the thread's slot (or -1) and its bodies' table slots
+template <int T>
+struct GroupThread {
+  int i, colour, sa, sb;
+  long long s;
+  int4 sl;
+  bool dA, dB;
+};
+
+template <int T>
+__device__ inline GroupThread<T> group_enter(const AdjCtx& a, const GroupView& v, int2* rng, int* keys, float4* table,
+                                             const float4* body) {
+  constexpr int H = kBinHashPerThread * T, LG = ilog2(H);
+  bin_ranges<T>(v.off, v.ng, v.ncolors, rng);
+  for (int e = threadIdx.x; e < H; e += T) keys[e] = -1;
+  __syncthreads();
+  GroupThread<T> g;
+  g.i = bin_constraint(rng, v.ncolors, threadIdx.x, &g.colour);
+  g.sa = g.sb = 0;
+  g.s = 0;
+  g.sl = make_int4(0, 0, 0, 0);
+  g.dA = g.dB = false;
+  if (g.i >= 0) {
+    g.s = a.off + g.i;
+    g.sl = a.slot[g.s];
+    g.sa = bin_slot(keys, LG, g.sl.x);
+    g.sb = bin_slot(keys, LG, g.sl.y);
+    g.dA = a.btype[g.sl.x] == 2;
+    g.dB = a.btype[g.sl.y] == 2;
+  }
+  __syncthreads();
+  for (int e = threadIdx.x; e < H; e += T)
+    if (keys[e] >= 0) table[e] = body[keys[e]];
+  __syncthreads();
+  return g;
+}
+
+// the dynamic bodies' records back (a group's dynamic bodies are in no other group)
+template <int T>
+__device__ inline void group_leave(const AdjCtx& a, const int* keys, const float4* table, float4* body) {
+  for (int e = threadIdx.x; e < kBinHashPerThread * T; e += T)
+    if (keys[e] >= 0 && a.btype[keys[e]] == 2) body[keys[e]] = table[e];
+}
+
+template <int T>
+__global__ void __launch_bounds__(T) k_af_group_vel(AdjCtx a, GroupView v) {
+  __shared__ int2 rng[kMaxColors];
+  __shared__ int keys[kBinHashPerThread * T];
+  __shared__ float4 bv[kBinHashPerThread * T];
+  const GroupThread<T> g = group_enter<T>(a, v, rng, keys, bv, a.vel);
+  TVelC<float> c = {};
+  ContactConst k = {};
+  float lam[4] = {};
+  if (g.i >= 0) {
+    c = load_velc(a.velc + kVelcRows * g.i);
+    k = velocity_const(a, g.sl);
+    const float4 l = a.lam_cur[g.i];
+    lam[0] = l.x; lam[1] = l.y; lam[2] = l.z; lam[3] = l.w;
+  }
+  for (int it = a.warm ? -1 : 0; it < v.iters; ++it)  // -1: the warm start
+    for (int col = 0; col < v.ncolors; ++col) {
+      if (rng[col].x == rng[col].y) continue;  // uniform across the workgroup
+      if (g.colour == col) {
+        const float4 vA = bv[g.sa], vB = bv[g.sb];
+        TVel<float> A = vel_from(vA), B = vel_from(vB);
+        if (it < 0) {
+          warm_start_t(c, k, lam, A, B);
+        } else {
+          if (a.record) {
+            float4* t = a.t_vel + 3 * (size_t(it) * a.n + g.i);
+            t[0] = vA;
+            t[1] = vB;
+            t[2] = make_float4(lam[0], lam[1], lam[2], lam[3]);
+          }
+          solve_velocity_t(c, k, lam, A, B, a.block != 0);
+        }
+        if (g.dA) bv[g.sa] = f4(A);
+        if (g.dB) bv[g.sb] = f4(B);
+      }
+      __syncthreads();
+    }
+  if (g.i >= 0)
+    a.lam_store[g.s] = stored_impulses(a, g.i, a.meta[g.s].x >> 8, c.vcount,
+                                       make_float4(lam[0], lam[1], lam[2], lam[3]));
+  group_leave<T>(a, keys, bv, a.vel);
+}
+
+template <int T>
+__global__ void __launch_bounds__(T) k_af_group_pos(AdjCtx a, GroupView v) {
+  __shared__ int2 rng[kMaxColors];
+  __shared__ int keys[kBinHashPerThread * T];
+  __shared__ float4 bp[kBinHashPerThread * T];
+  const GroupThread<T> g = group_enter<T>(a, v, rng, keys, bp, a.pos);
+  ContactConst k = {};
+  TGeom<float> geom = {};
+  int runs = 0;
+  if (g.i >= 0) {
+    const int4 mt = a.meta[g.s];
+    k = contact_const(a, g.sl, mt.x);
+    geom = load_geom(a.geom + 2 * g.i);
+    runs = mt.w;  // iterations until the island stopped
+  }
+  for (int it = 0; it < v.iters; ++it)
+    for (int col = 0; col < v.ncolors; ++col) {
+      if (rng[col].x == rng[col].y) continue;
+      if (g.colour == col && it < runs) {
+        const float4 pA = bp[g.sa], pB = bp[g.sb];
+        if (a.record) {
+          float4* t = a.t_pos + 2 * (size_t(it) * a.n + g.i);
+          t[0] = pA;
+          t[1] = pB;
+        }
+        TPos<float> A = pos_from(pA), B = pos_from(pB);
+        solve_position_t(k, geom, A, B);
+        if (g.dA) bp[g.sa] = f4(A);
+        if (g.dB) bp[g.sb] = f4(B);
+      }
+      __syncthreads();
+    }
+  group_leave<T>(a, keys, bp, a.pos);
+}
+
+template <int T>
+__global__ void __launch_bounds__(T) k_ab_group_pos(AdjCtx a, GroupView v) {
+  __shared__ int2 rng[kMaxColors];
+  __shared__ int keys[kBinHashPerThread * T];
+  __shared__ float4 bb[kBinHashPerThread * T];
+  const GroupThread<T> g = group_enter<T>(a, v, rng, keys, bb, a.pbar);
+  ContactConst k = {};
+  TGeom<float> geom = {}, gb = {};
+  int runs = 0;
+  if (g.i >= 0) {
+    const int4 mt = a.meta[g.s];
+    k = contact_const(a, g.sl, mt.x);
+    geom = load_geom(a.geom + 2 * g.i);
+    runs = mt.w;
+  }
+  const float4 z = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+  float4 tA = z, tB = z;  // the iteration's inputs, loaded ahead of its barriers
+  auto fetch = [&](int it) {
+    if (it < 0 || it >= runs) return;
+    const float4* t = a.t_pos + 2 * (size_t(it) * a.n + g.i);
+    tA = t[0];
+    tB = t[1];
+  };
+  fetch(v.iters - 1);
+  for (int it = v.iters - 1; it >= 0; --it)
+    for (int col = v.ncolors - 1; col >= 0; --col) {
+      if (rng[col].x == rng[col].y) continue;
+      if (g.colour == col) {
+        if (it < runs) {
+          TPos<float> Ab = pos_from(g.dA ? bb[g.sa] : z), Bb = pos_from(g.dB ? bb[g.sb] : z);
+          solve_position_bar(k, geom, pos_from(tA), pos_from(tB), Ab, Bb, gb);
+          if (g.dA) bb[g.sa] = f4(Ab);
+          if (g.dB) bb[g.sb] = f4(Bb);
+        }
+        fetch(it - 1);
+      }
+      __syncthreads();
+    }
+  if (g.i >= 0) store_geom(a.gbar + 2 * g.i, gb);
+  group_leave<T>(a, keys, bb, a.pbar);
+}
+
+// cotangents of a slot's impulses after the last iteration, from those of its stored impulses;
+// *e0: of the carried impulses that were stored back unsolved
+__device__ inline float4 store_reverse(const AdjCtx& a, long long s, int count, int vcount, float4* e0) {
+  const float4 g = a.store_bar[s];
+  float4 lb = make_float4(g.x, g.y, 0.0f, 0.0f);
+  *e0 = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+  if (vcount > 1) {
+    lb.z = g.z;
+    lb.w = g.w;
+  } else if (count > 1) {
+    e0->z = g.z;
+    e0->w = g.w;
+  }
+  return lb;
+}
+
+template <int T>
+__global__ void __launch_bounds__(T) k_ab_group_vel(AdjCtx a, GroupView v) {
+  __shared__ int2 rng[kMaxColors];
+  __shared__ int keys[kBinHashPerThread * T];
+  __shared__ float4 bb[kBinHashPerThread * T];
+  const GroupThread<T> g = group_enter<T>(a, v, rng, keys, bb, a.vbar);
+  TVelC<float> c = {};
+  ContactConst k = {};
+  float lb[4] = {};
+  if (g.i >= 0) {
+    c = load_velc(a.velc + kVelcRows * g.i);
+    k = velocity_const(a, g.sl);
+    float4 e0;
+    const float4 l = store_reverse(a, g.s, a.meta[g.s].x >> 8, c.vcount, &e0);
+    a.lam0bar[g.i] = e0;
+    lb[0] = l.x; lb[1] = l.y; lb[2] = l.z; lb[3] = l.w;
+  }
+  TVelC<float> cb = zero_velc<float>();
+  const float4 z = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+  float4 tA = z, tB = z, tl = z;  // the iteration's inputs, loaded ahead of its barriers
+  auto fetch = [&](int it) {
+    if (it < 0) return;
+    const float4* t = a.t_vel + 3 * (size_t(it) * a.n + g.i);
+    tA = t[0];
+    tB = t[1];
+    tl = t[2];
+  };
+  if (g.i >= 0) fetch(v.iters - 1);
+  for (int it = v.iters - 1; it >= 0; --it)
+    for (int col = v.ncolors - 1; col >= 0; --col) {
+      if (rng[col].x == rng[col].y) continue;
+      if (g.colour == col) {
+        TVel<float> Ab = vel_from(g.dA ? bb[g.sa] : z), Bb = vel_from(g.dB ? bb[g.sb] : z);
+        const float lam[4] = {tl.x, tl.y, tl.z, tl.w};
+        solve_velocity_bar(c, k, lam, vel_from(tA), vel_from(tB), a.block != 0, Ab, Bb, lb, cb);
+        if (g.dA) bb[g.sa] = f4(Ab);
+        if (g.dB) bb[g.sb] = f4(Bb);
+        fetch(it - 1);
+      }
+      __syncthreads();
+    }
+  if (g.i >= 0) {
+    if (a.warm) {
+      const float4 l = a.lam_init[g.i];
+      const float lam[4] = {l.x, l.y, l.z, l.w};
+      warm_start_bar(c, k, lam, vel_from(g.dA ? bb[g.sa] : z), vel_from(g.dB ? bb[g.sb] : z), lb, cb);
+    }
+    a.lambar[g.i] = make_float4(lb[0], lb[1], lb[2], lb[3]);
+    store_velc(a.velcbar + kVelcRows * g.i, cb);
+  }
+  group_leave<T>(a, keys, bb, a.vbar);
+}
+
+// ---- per colour: a constraint per thread, state in memory ------------------------------------------
+// the cotangents the reverse kernels add to
+__global__ void __launch_bounds__(kBlock) k_ab_clear(AdjCtx a) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= a.n) return;
+  const float4 z = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+  a.gbar[2 * i] = a.gbar[2 * i + 1] = z;
+  for (int r = 0; r < kVelcRows; ++r) a.velcbar[kVelcRows * i + r] = z;
+}
+
+__global__ void __launch_bounds__(kBlock) k_af_warm(AdjCtx a, int b0, int b1) {
+  int i = b0 + blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= b1) return;
+  const int4 sl = a.slot[a.off + i];
+  const float4 l = a.lam_cur[i];
+  const float lam[4] = {l.x, l.y, l.z, l.w};
+  TVel<float> A = vel_from(a.vel[sl.x]), B = vel_from(a.vel[sl.y]);
+  warm_start_t(load_velc(a.velc + kVelcRows * i), velocity_const(a, sl), lam, A, B);
+  if (a.btype[sl.x] == 2) a.vel[sl.x] = f4(A);
+  if (a.btype[sl.y] == 2) a.vel[sl.y] = f4(B);
+}
+
+__global__ void __launch_bounds__(kBlock) k_af_vel(AdjCtx a, int b0, int b1, int it) {
+  int i = b0 + blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= b1) return;
+  const int4 sl = a.slot[a.off + i];
+  const float4 vA = a.vel[sl.x], vB = a.vel[sl.y], l = a.lam_cur[i];
+  if (a.record) {
+    float4* t = a.t_vel + 3 * (size_t(it) * a.n + i);
+    t[0] = vA;
+    t[1] = vB;
+    t[2] = l;
+  }
+  float lam[4] = {l.x, l.y, l.z, l.w};
+  TVel<float> A = vel_from(vA), B = vel_from(vB);
+  solve_velocity_t(load_velc(a.velc + kVelcRows * i), velocity_const(a, sl), lam, A, B, a.block != 0);
+  if (a.btype[sl.x] == 2) a.vel[sl.x] = f4(A);
+  if (a.btype[sl.y] == 2) a.vel[sl.y] = f4(B);
+  a.lam_cur[i] = make_float4(lam[0], lam[1], lam[2], lam[3]);
+}
+
+__global__ void __launch_bounds__(kBlock) k_af_store(AdjCtx a) {
+  int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= a.n) return;
+  const long long s = a.off + i;
+  a.lam_store[s] = stored_impulses(a, i, a.meta[s].x >> 8, __float_as_int(a.velc[kVelcRows * i].w), a.lam_cur[i]);
+}
+
 __global__ void __launch_bounds__(kBlock) k_af_pos(AdjCtx a, int b0, int b1, int it) {
   int i = b0 + blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= b1) return;
@@ -432,94 +758,83 @@ __global__ void __launch_bounds__(kBlock) k_af_pos(AdjCtx a, int b0, int b1, int
   const int4 mt = a.meta[s];
   if (mt.w <= it) return;  // the island stopped iterating
   const int4 sl = a.slot[s];
-  const ContactConst k = contact_const(a, sl, mt.x);
   const float4 pA = a.pos[sl.x], pB = a.pos[sl.y];
   if (a.record) {
     float4* t = a.t_pos + 2 * (size_t(it) * a.n + i);
     t[0] = pA;
     t[1] = pB;
   }
-  float x[14], y[6];
-  put3(x, pA);
-  put3(x + 3, pB);
-  const float4 g0 = a.geom[2 * i], g1 = a.geom[2 * i + 1];
-  x[6] = g0.x; x[7] = g0.y; x[8] = g0.z; x[9] = g0.w;
-  x[10] = g1.x; x[11] = g1.y; x[12] = g1.z; x[13] = g1.w;
-  PosFn<float> fn{k};
-  fn(x, y);
-  if (a.btype[sl.x] == 2) a.pos[sl.x] = f4(y);
-  if (a.btype[sl.y] == 2) a.pos[sl.y] = f4(y + 3);
+  TPos<float> A = pos_from(pA), B = pos_from(pB);
+  solve_position_t(contact_const(a, sl, mt.x), load_geom(a.geom + 2 * i), A, B);
+  if (a.btype[sl.x] == 2) a.pos[sl.x] = f4(A);
+  if (a.btype[sl.y] == 2) a.pos[sl.y] = f4(B);
 }
-
-// -- reverse
-__device__ inline void add4(float4& d, const float* x) { d.x += x[0]; d.y += x[1]; d.z += x[2]; d.w += x[3]; }
-__device__ inline void add3(float4& d, const float* x) { d.x += x[0]; d.y += x[1]; d.z += x[2]; }
-
-__global__ void __launch_bounds__(kBlock) k_ab_clear(AdjCtx a) {
-  int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= a.n) return;
-  const float4 z = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-  a.qnbar[2 * i] = a.qnbar[2 * i + 1] = z;
-  a.gbar[2 * i] = a.gbar[2 * i + 1] = z;
-  a.vsbar[2 * i] = a.vsbar[2 * i + 1] = z;
-  a.fricbar[i] = 0.0f;
-}
-
-// The reverse position solve runs kPosGroups threads per constraint, one per group of kPosLanes
-// dual lanes over its 14 inputs (adjacent lanes of one wave, as for the velocity solve below:
-// all read the position cotangents before any writes, each writes only its own inputs' entries)
-constexpr int kPosIn = 14, kPosLanes = 2, kPosGroups = 8;
-static_assert(kPosGroups * kPosLanes >= kPosIn && 64 % kPosGroups == 0, "position groups");
 
 __global__ void __launch_bounds__(kBlock) k_ab_pos(AdjCtx a, int b0, int b1, int it) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  const int i = b0 + t / kPosGroups, lo = (t % kPosGroups) * kPosLanes;
-  if (i >= b1 || lo >= kPosIn) return;
+  const int i = b0 + blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= b1) return;
   const long long s = a.off + i;
   const int4 mt = a.meta[s];
   if (mt.w <= it) return;
   const int4 sl = a.slot[s];
-  const ContactConst k = contact_const(a, sl, mt.x);
   const bool dA = a.btype[sl.x] == 2, dB = a.btype[sl.y] == 2;
-  const float4* tp = a.t_pos + 2 * (size_t(it) * a.n + i);
-  float x[kPosIn], yb[6], xb[kPosIn];
-  put3(x, tp[0]);
-  put3(x + 3, tp[1]);
-  const float4 g0 = a.geom[2 * i], g1 = a.geom[2 * i + 1];
-  x[6] = g0.x; x[7] = g0.y; x[8] = g0.z; x[9] = g0.w;
-  x[10] = g1.x; x[11] = g1.y; x[12] = g1.z; x[13] = g1.w;
   const float4 z = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-  put3(yb, dA ? a.pbar[sl.x] : z);
-  put3(yb + 3, dB ? a.pbar[sl.y] : z);
-  for (int j = 0; j < kPosIn; ++j) xb[j] = 0.0f;
-  vjp_group<kPosIn, 6, kPosLanes>(x, yb, xb, PosFn<float>{k}, lo);
-  const int hi = lo + kPosLanes;
-  auto put = [&](float* d, int j, bool assign) {
-    if (j >= lo && j < hi) {
-      if (assign) *d = xb[j];
-      else *d += xb[j];
-    }
-  };
-  float* pa = &a.pbar[sl.x].x;
-  float* pb = &a.pbar[sl.y].x;
-  float* ga = &a.gbar[2 * i].x;
-  float* gb = &a.gbar[2 * i + 1].x;
-#pragma unroll
-  for (int c = 0; c < 3; ++c) {
-    if (dA) put(pa + c, c, true);
-    if (dB) put(pb + c, 3 + c, true);
-  }
-  if (lo == 0) {  // the unused fourth component, as a whole-record write would leave it
-    if (dA) pa[3] = 0.0f;
-    if (dB) pb[3] = 0.0f;
-  }
-#pragma unroll
-  for (int c = 0; c < 4; ++c) {
-    put(ga + c, 6 + c, false);
-    put(gb + c, 10 + c, false);
-  }
+  TPos<float> Ab = pos_from(dA ? a.pbar[sl.x] : z), Bb = pos_from(dB ? a.pbar[sl.y] : z);
+  TGeom<float> gb = load_geom(a.gbar + 2 * i);
+  const float4* t = a.t_pos + 2 * (size_t(it) * a.n + i);
+  solve_position_bar(contact_const(a, sl, mt.x), load_geom(a.geom + 2 * i), pos_from(t[0]), pos_from(t[1]), Ab, Bb, gb);
+  if (dA) a.pbar[sl.x] = f4(Ab);
+  if (dB) a.pbar[sl.y] = f4(Bb);
+  store_geom(a.gbar + 2 * i, gb);
 }
 
+__global__ void __launch_bounds__(kBlock) k_ab_store(AdjCtx a) {
+  int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= a.n) return;
+  const long long s = a.off + i;
+  float4 e0;
+  a.lambar[i] = store_reverse(a, s, a.meta[s].x >> 8, __float_as_int(a.velc[kVelcRows * i].w), &e0);
+  a.lam0bar[i] = e0;
+}
+
+__global__ void __launch_bounds__(kBlock) k_ab_vel(AdjCtx a, int b0, int b1, int it) {
+  const int i = b0 + blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= b1) return;
+  const int4 sl = a.slot[a.off + i];
+  const bool dA = a.btype[sl.x] == 2, dB = a.btype[sl.y] == 2;
+  const float4 z = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+  TVel<float> Ab = vel_from(dA ? a.vbar[sl.x] : z), Bb = vel_from(dB ? a.vbar[sl.y] : z);
+  const float4 l = a.lambar[i];
+  float lb[4] = {l.x, l.y, l.z, l.w};
+  const float4* t = a.t_vel + 3 * (size_t(it) * a.n + i);
+  const float4 tl = t[2];
+  const float lam[4] = {tl.x, tl.y, tl.z, tl.w};
+  TVelC<float> cb = load_velc(a.velcbar + kVelcRows * i);
+  solve_velocity_bar(load_velc(a.velc + kVelcRows * i), velocity_const(a, sl), lam, vel_from(t[0]), vel_from(t[1]),
+                     a.block != 0, Ab, Bb, lb, cb);
+  if (dA) a.vbar[sl.x] = f4(Ab);
+  if (dB) a.vbar[sl.y] = f4(Bb);
+  a.lambar[i] = make_float4(lb[0], lb[1], lb[2], lb[3]);
+  store_velc(a.velcbar + kVelcRows * i, cb);
+}
+
+// all colours at once: the warm start's reverse leaves the velocities' cotangents as they are
+__global__ void __launch_bounds__(kBlock) k_ab_warm(AdjCtx a) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= a.n) return;
+  const int4 sl = a.slot[a.off + i];
+  const float4 z = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+  const float4 l = a.lambar[i], li = a.lam_init[i];
+  float lb[4] = {l.x, l.y, l.z, l.w};
+  const float lam[4] = {li.x, li.y, li.z, li.w};
+  TVelC<float> cb = load_velc(a.velcbar + kVelcRows * i);
+  warm_start_bar(load_velc(a.velc + kVelcRows * i), velocity_const(a, sl), lam,
+                 vel_from(a.btype[sl.x] == 2 ? a.vbar[sl.x] : z), vel_from(a.btype[sl.y] == 2 ? a.vbar[sl.y] : z), lb, cb);
+  a.lambar[i] = make_float4(lb[0], lb[1], lb[2], lb[3]);
+  store_velc(a.velcbar + kVelcRows * i, cb);
+}
+
+// ---- reverse: integration and set-up ----------------------------------------------------------------
 __global__ void __launch_bounds__(kBlock) k_ab_intpos(AdjCtx a) {
   int b = blockIdx.x * blockDim.x + threadIdx.x;
   if (b >= a.nb) return;
@@ -534,169 +849,95 @@ __global__ void __launch_bounds__(kBlock) k_ab_intpos(AdjCtx a) {
   a.vbar[b] = f4(xb + 3);
 }
 
-__global__ void __launch_bounds__(kBlock) k_ab_store(AdjCtx a) {
-  int i = blockIdx.x * blockDim.x + threadIdx.x;
+// The constraint record's cotangents through initialize_velocity_constraints, once a step: ten
+// threads per slot, each two of the 20 inputs as dual lanes, each writing its own inputs' entries.
+constexpr int kInitLanes = 2, kInitGroups = kInitIn / kInitLanes;
+static_assert(kInitGroups * kInitLanes == kInitIn, "the groups cover the inputs");
+__global__ void __launch_bounds__(kBlock) k_ab_init(AdjCtx a) {
+  const int t = blockIdx.x * blockDim.x + threadIdx.x;
+  const int i = t / kInitGroups, lo = (t % kInitGroups) * kInitLanes;
   if (i >= a.n) return;
   const long long s = a.off + i;
   const int4 sl = a.slot[s];
   const ContactConst k = contact_const(a, sl, a.meta[s].x);
-  const int vc = vcount_of(a, i, sl, k);
-  const float4 g = a.store_bar[s];
-  float4 lb = make_float4(g.x, g.y, 0.0f, 0.0f), eb = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-  if (vc > 1) {
-    lb.z = g.z;
-    lb.w = g.w;
-  } else if (k.count > 1) {
-    eb.z = g.z;
-    eb.w = g.w;
-  }
-  a.lambar[i] = lb;
-  a.lam0bar[i] = eb;
-}
-
-// The reverse velocity solve and warm start run kVelGroups threads per constraint, one per group
-// of kVelLanes dual lanes of the vector-Jacobian product (a colour holds a few thousand
-// constraints: one thread each would leave most of the GPU idle, and one thread's four passes
-// over 8-lane duals run at one wave per SIMD). The groups of a constraint are adjacent lanes of
-// one wave: each reads the body and impulse cotangents before any of them writes, and each
-// writes only the entries of its own inputs.
-constexpr int kVelLanes = 2;
-constexpr int kVelGroups = (kVelIn + kVelLanes - 1) / kVelLanes;
-static_assert(64 % kVelGroups == 0, "a constraint's groups share one wave");
-
-// cotangents of the velocity inputs of group [lo, lo + kVelLanes): body velocities replaced,
-// impulses replaced (kAssignLam) or accumulated, the rest accumulated
-template <bool kAssignLam>
-__device__ inline void vel_group_out(const AdjCtx& a, int i, int4 sl, bool dA, bool dB, const float* xb, int lo) {
-  const int hi = lo + kVelLanes;
-  auto put = [&](float* d, int j, bool assign) {
-    if (j >= lo && j < hi) {
-      if (assign) *d = xb[j];
-      else *d += xb[j];
-    }
-  };
-  float* va = &a.vbar[sl.x].x;
-  float* vb = &a.vbar[sl.y].x;
+  float x[kInitIn], yb[kInitOut], xb[kInitIn];
+  put3(x, a.pos_n[sl.x]);
+  put3(x + 3, a.pos_n[sl.y]);
+  const float4 g0 = a.geom[2 * i], g1 = a.geom[2 * i + 1];
+  x[6] = g0.x; x[7] = g0.y; x[8] = g0.z; x[9] = g0.w;
+  x[10] = g1.x; x[11] = g1.y; x[12] = g1.z; x[13] = g1.w;
+  put3(x + 14, a.vstar[sl.x]);
+  put3(x + 17, a.vstar[sl.y]);
+  InitFn<float>::put_velc(yb, load_velc(a.velcbar + kVelcRows * i));
+  for (int j = 0; j < kInitIn; ++j) xb[j] = 0.0f;
+  vjp_group<kInitIn, kInitOut, kInitLanes>(x, yb, xb, InitFn<float>{k, a.block != 0}, lo);
+  float* q = &a.qnbar[2 * i].x;   // rows of four: q.x, q.y, q.a, unused
+  float* g = &a.gbar[2 * i].x;
+  float* v = &a.vsbar[2 * i].x;
 #pragma unroll
-  for (int c = 0; c < 3; ++c) {
-    if (dA) put(va + c, c, true);
-    if (dB) put(vb + c, 3 + c, true);
-  }
-  if (lo == 0) {  // the unused fourth component, as a whole-record write would leave it
-    if (dA) va[3] = 0.0f;
-    if (dB) vb[3] = 0.0f;
-  }
-  float* lam = &a.lambar[i].x;
-  float* q0 = &a.qnbar[2 * i].x;
-  float* q1 = &a.qnbar[2 * i + 1].x;
-  float* g0 = &a.gbar[2 * i].x;
-  float* g1 = &a.gbar[2 * i + 1].x;
-  float* s0 = &a.vsbar[2 * i].x;
-  float* s1 = &a.vsbar[2 * i + 1].x;
-#pragma unroll
-  for (int c = 0; c < 4; ++c) put(lam + c, 6 + c, kAssignLam);
-#pragma unroll
-  for (int c = 0; c < 3; ++c) {
-    put(q0 + c, 10 + c, false);
-    put(q1 + c, 13 + c, false);
-  }
-#pragma unroll
-  for (int c = 0; c < 4; ++c) {
-    put(g0 + c, 16 + c, false);
-    put(g1 + c, 20 + c, false);
-  }
-  put(&a.fricbar[i], 24, false);
-#pragma unroll
-  for (int c = 0; c < 3; ++c) {
-    put(s0 + c, 25 + c, false);
-    put(s1 + c, 28 + c, false);
+  for (int j = 0; j < kInitIn; ++j) {
+    if (j < lo || j >= lo + kInitLanes) continue;
+    if (j < 6) q[j < 3 ? j : j + 1] = xb[j];
+    else if (j < 14) g[j - 6] += xb[j];
+    else v[j < 17 ? j - 14 : j - 13] = xb[j];
   }
 }
 
-__global__ void __launch_bounds__(kBlock) k_ab_vel(AdjCtx a, int b0, int b1, int it) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  const int i = b0 + t / kVelGroups, lo = (t % kVelGroups) * kVelLanes;
-  if (i >= b1) return;
-  const long long s = a.off + i;
-  const int4 sl = a.slot[s];
-  const ContactConst k = contact_const(a, sl, a.meta[s].x);
-  const bool dA = a.btype[sl.x] == 2, dB = a.btype[sl.y] == 2;
-  const float4* tv = a.t_vel + 3 * (size_t(it) * a.n + i);
-  float x[kVelIn], yb[10], xb[kVelIn];
-  vel_inputs(a, i, sl, tv[0], tv[1], tv[2], x);
-  const float4 z = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-  put3(yb, dA ? a.vbar[sl.x] : z);
-  put3(yb + 3, dB ? a.vbar[sl.y] : z);
-  const float4 lb = a.lambar[i];
-  yb[6] = lb.x; yb[7] = lb.y; yb[8] = lb.z; yb[9] = lb.w;
-  for (int j = 0; j < kVelIn; ++j) xb[j] = 0.0f;
-  vjp_group<kVelIn, 10, kVelLanes>(x, yb, xb, VelFn<float>{k, a.block != 0}, lo);
-  vel_group_out<true>(a, i, sl, dA, dB, xb, lo);
-}
-
-__global__ void __launch_bounds__(kBlock) k_ab_warm(AdjCtx a, int b0, int b1) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  const int i = b0 + t / kVelGroups, lo = (t % kVelGroups) * kVelLanes;
-  if (i >= b1) return;
-  const long long s = a.off + i;
-  const int4 sl = a.slot[s];
-  const ContactConst k = contact_const(a, sl, a.meta[s].x);
-  const bool dA = a.btype[sl.x] == 2, dB = a.btype[sl.y] == 2;
-  float x[kVelIn], yb[6], xb[kVelIn];
-  vel_inputs(a, i, sl, a.t_ws[2 * i], a.t_ws[2 * i + 1], a.lam_init[i], x);
-  const float4 z = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-  put3(yb, dA ? a.vbar[sl.x] : z);
-  put3(yb + 3, dB ? a.vbar[sl.y] : z);
-  for (int j = 0; j < kVelIn; ++j) xb[j] = 0.0f;
-  vjp_group<kVelIn, 6, kVelLanes>(x, yb, xb, WarmFn<float>{k, a.block != 0}, lo);
-  vel_group_out<false>(a, i, sl, dA, dB, xb, lo);
-}
-
-__device__ inline void atomic_add3(float4* p, float4 v) {
-  atomicAdd(&p->x, v.x);
-  atomicAdd(&p->y, v.y);
-  atomicAdd(&p->z, v.z);
-}
-
-// carried impulses, friction mixing, manifold geometry, and the constraint set-up's use of
-// the start-of-step positions and velocities
+// Four threads per slot. The first three: manifold geometry = collide(qA, qB), two of the six
+// position inputs each, and the constraint set-up's use of the start-of-step positions. The fourth:
+// carried impulses, friction mixing, and the set-up's use of the velocities.
 __global__ void __launch_bounds__(kBlock) k_ab_setup(AdjCtx a) {
-  int i = blockIdx.x * blockDim.x + threadIdx.x;
+  const int t = blockIdx.x * blockDim.x + threadIdx.x;
+  const int i = t >> 2, part = t & 3;
   if (i >= a.n) return;
   const long long s = a.off + i;
   const int4 sl = a.slot[s];
-  const int4 mt = a.meta[s];
-  const int count = mt.x >> 8;
-  float4 eb = a.lam0bar[i];
-  if (a.warm) {
-    const float4 lb = a.lambar[i];
-    eb.x += a.dt_ratio * lb.x;
-    eb.y += a.dt_ratio * lb.y;
-    if (count > 1) {
-      eb.z += a.dt_ratio * lb.z;
-      eb.w += a.dt_ratio * lb.w;
+  const bool dA = a.btype[sl.x] == 2, dB = a.btype[sl.y] == 2;
+  if (part == 3) {
+    const int4 mt = a.meta[s];
+    float4 eb = a.lam0bar[i];
+    if (a.warm) {
+      const float4 lb = a.lambar[i];
+      eb.x += a.dt_ratio * lb.x;
+      eb.y += a.dt_ratio * lb.y;
+      if (mt.x >> 8 > 1) {
+        eb.z += a.dt_ratio * lb.z;
+        eb.w += a.dt_ratio * lb.w;
+      }
     }
+    if (mt.y >= 0) {
+      float* d = &a.store_bar[mt.y >> 1].x + 2 * (mt.y & 1);
+      atomicAdd(d, eb.x);
+      atomicAdd(d + 1, eb.y);
+    }
+    if (mt.z >= 0) {
+      float* d = &a.store_bar[mt.z >> 1].x + 2 * (mt.z & 1);
+      atomicAdd(d, eb.z);
+      atomicAdd(d + 1, eb.w);
+    }
+    // friction = sqrt(fA fB)
+    const float fa = a.fmat[sl.z].x, fb = a.fmat[sl.w].x;
+    const float mu = sqrtf(fa * fb);
+    if (mu > 0.0f) {
+      const float g = a.velcbar[kVelcRows * i].z;
+      atomicAdd(&a.fric_grad[sl.z], g * 0.5f * fb / mu);
+      atomicAdd(&a.fric_grad[sl.w], g * 0.5f * fa / mu);
+    }
+    const float4 va = a.vsbar[2 * i], vb = a.vsbar[2 * i + 1];
+    if (dA) {
+      float* d = &a.vbar[sl.x].x;
+      atomicAdd(d, va.x);
+      atomicAdd(d + 1, va.y);
+      atomicAdd(d + 2, va.z);
+    }
+    if (dB) {
+      float* d = &a.vbar[sl.y].x;
+      atomicAdd(d, vb.x);
+      atomicAdd(d + 1, vb.y);
+      atomicAdd(d + 2, vb.z);
+    }
+    return;
   }
-  if (mt.y >= 0) {
-    float* d = &a.store_bar[mt.y >> 1].x + 2 * (mt.y & 1);
-    atomicAdd(d, eb.x);
-    atomicAdd(d + 1, eb.y);
-  }
-  if (mt.z >= 0) {
-    float* d = &a.store_bar[mt.z >> 1].x + 2 * (mt.z & 1);
-    atomicAdd(d, eb.z);
-    atomicAdd(d + 1, eb.w);
-  }
-  // friction = sqrt(fA fB)
-  const float fa = a.fmat[sl.z].x, fb = a.fmat[sl.w].x;
-  const float mu = sqrtf(fa * fb);
-  if (mu > 0.0f) {
-    const float g = a.fricbar[i];
-    atomicAdd(&a.fric_grad[sl.z], g * 0.5f * fb / mu);
-    atomicAdd(&a.fric_grad[sl.w], g * 0.5f * fa / mu);
-  }
-  // geometry = collide(qA, qB)
-  const ShapeV &sa = a.shapes[sl.z], &sb = a.shapes[sl.w];
   const float4 A = a.bmass[sl.x], B = a.bmass[sl.y];
   const float lcA[2] = {A.z, A.w}, lcB[2] = {B.z, B.w};
   float x[6], yb[8], xb[6] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
@@ -705,17 +946,14 @@ __global__ void __launch_bounds__(kBlock) k_ab_setup(AdjCtx a) {
   const float4 g0 = a.gbar[2 * i], g1 = a.gbar[2 * i + 1];
   yb[0] = g0.x; yb[1] = g0.y; yb[2] = g0.z; yb[3] = g0.w;
   yb[4] = g1.x; yb[5] = g1.y; yb[6] = g1.z; yb[7] = g1.w;
-  vjp<6, 8, 6>(x, yb, xb, GeomFn<float>{&sa, &sb, lcA, lcB, nullptr, nullptr});
-  float4 qa = a.qnbar[2 * i], qb = a.qnbar[2 * i + 1];
-  qa.x += xb[0]; qa.y += xb[1]; qa.z += xb[2];
-  qb.x += xb[3]; qb.y += xb[4]; qb.z += xb[5];
-  if (a.btype[sl.x] == 2) {
-    atomic_add3(&a.pbar[sl.x], qa);
-    atomic_add3(&a.vbar[sl.x], a.vsbar[2 * i]);
-  }
-  if (a.btype[sl.y] == 2) {
-    atomic_add3(&a.pbar[sl.y], qb);
-    atomic_add3(&a.vbar[sl.y], a.vsbar[2 * i + 1]);
+  const int lo = 2 * part;
+  vjp_group<6, 8, 2>(x, yb, xb, GeomFn<float>{&a.shapes[sl.z], &a.shapes[sl.w], lcA, lcB, nullptr, nullptr}, lo);
+  const float* q = &a.qnbar[2 * i].x;
+#pragma unroll
+  for (int j = 0; j < 6; ++j) {
+    if (j < lo || j >= lo + 2 || !(j < 3 ? dA : dB)) continue;
+    const int b = j < 3 ? sl.x : sl.y, c = j < 3 ? j : j - 3;
+    atomicAdd(&a.pbar[b].x + c, xb[j] + q[j < 3 ? j : j + 1]);
   }
 }
 
@@ -732,22 +970,6 @@ __global__ void __launch_bounds__(kBlock) k_ab_intvel(AdjCtx a) {
 }
 
 // ---- drivers ---------------------------------------------------------------------------------
-struct AdjBuffers {
-  DevArray<float4> pos, vel, seg_pos, seg_vel, vstar, geom, lam_cur, lam_init, lam0eff;
-  DevArray<float4> t_ws, t_vel, t_ip, t_pos;
-  DevArray<float4> pbar, vbar, lambar, lam0bar, qnbar, gbar, vsbar, store_bar;
-  DevArray<float> fricbar, fric_grad;
-  DevArray<int> err;
-  void release() {
-    for (auto* d : {&pos, &vel, &seg_pos, &seg_vel, &vstar, &geom, &lam_cur, &lam_init, &lam0eff, &t_ws, &t_vel, &t_ip,
-                    &t_pos, &pbar, &vbar, &lambar, &lam0bar, &qnbar, &gbar, &vsbar, &store_bar})
-      d->release();
-    fricbar.release();
-    fric_grad.release();
-    err.release();
-  }
-};
-
 static AdjCtx make_ctx(World* w, AdjBuffers& B) {
   Tape& t = w->tape;
   AdjCtx a;
@@ -775,10 +997,10 @@ static AdjCtx make_ctx(World* w, AdjBuffers& B) {
   a.pos_n = a.vel_n = nullptr;
   a.vstar = B.vstar.p;
   a.geom = B.geom.p;
+  a.velc = B.velc.p;
   a.lam_cur = B.lam_cur.p;
   a.lam_init = B.lam_init.p;
   a.lam0eff = B.lam0eff.p;
-  a.t_ws = B.t_ws.p;
   a.t_vel = B.t_vel.p;
   a.t_ip = B.t_ip.p;
   a.t_pos = B.t_pos.p;
@@ -789,14 +1011,24 @@ static AdjCtx make_ctx(World* w, AdjBuffers& B) {
   a.qnbar = B.qnbar.p;
   a.gbar = B.gbar.p;
   a.vsbar = B.vsbar.p;
+  a.velcbar = B.velcbar.p;
   a.store_bar = B.store_bar.p;
-  a.fricbar = B.fricbar.p;
   a.fric_grad = B.fric_grad.p;
   a.err = B.err.p;
   return a;
 }
 
-static void set_step(AdjCtx& a, const TapeStep& ts, const float4* pos_n, const float4* vel_n, int record) {
+// slot: the step's place among the kept ones (0 when each step is recorded just before its reverse)
+static void set_step(AdjCtx& a, const AdjBuffers& B, const TapeStep& ts, float4* pos_n, float4* vel_n, int record,
+                     size_t slot) {
+  const size_t n = B.max_slots * slot, nb = size_t(a.nb) * slot;
+  a.vstar = B.vstar.p + nb;
+  a.geom = B.geom.p + 2 * n;
+  a.velc = B.velc.p + kVelcRows * n;
+  a.lam_init = B.lam_init.p + n;
+  a.t_vel = B.t_vel.p + 3 * size_t(B.vel_iters) * n;
+  a.t_ip = B.t_ip.p + 2 * nb;
+  a.t_pos = B.t_pos.p + 2 * size_t(B.pos_iters) * n;
   a.off = ts.off;
   a.n = ts.n;
   a.dt = ts.dt;
@@ -808,37 +1040,63 @@ static void set_step(AdjCtx& a, const TapeStep& ts, const float4* pos_n, const f
   a.vel_n = vel_n;
 }
 
-// replays one frozen step on a.pos/a.vel (a.pos_n/a.vel_n: copies of the start state); with
-// a.record set, keeps every constraint's inputs for reverse_step
-static int replay_step(World* w, const AdjCtx& a, const TapeStep& ts) {
+// The group kernels hold one constraint per thread: workgroups of the smallest size that covers the
+// step's largest group; 0 (per-colour launches) for a step that was not grouped or whose largest
+// group exceeds 512, the most constraints whose bodies' table is worth its LDS (40 KB).
+static int group_threads(const TapeStep& ts, int group_max) {
+  if (ts.ng == 0 || group_max > 512) return 0;
+  return group_max <= 64 ? 64 : group_max <= 128 ? 128 : group_max <= 256 ? 256 : 512;
+}
+
+#define B2G_LAUNCH_GROUPS(T, kernel, stream, a, v)                                                             \
+  do {                                                                                                         \
+    const dim3 grid_((v).ng);                                                                                  \
+    if ((T) == 64) hipLaunchKernelGGL(kernel<64>, grid_, dim3(64), 0, stream, a, v);                           \
+    else if ((T) == 128) hipLaunchKernelGGL(kernel<128>, grid_, dim3(128), 0, stream, a, v);                   \
+    else if ((T) == 256) hipLaunchKernelGGL(kernel<256>, grid_, dim3(256), 0, stream, a, v);                   \
+    else hipLaunchKernelGGL(kernel<512>, grid_, dim3(512), 0, stream, a, v);                                   \
+  } while (0)
+
+static GroupView group_view(World* w, const TapeStep& ts, int iters) {
+  return GroupView{w->tape.group_off.p + ts.goff, ts.ng, int(ts.color_off.size()) - 1, iters};
+}
+
+// Replays one frozen step on a.pos/a.vel; a.pos_n/a.vel_n receive the start state, or (take_back)
+// hold it. With a.record set, keeps every constraint's inputs for reverse_step.
+static int replay_step(World* w, const AdjCtx& a, const TapeStep& ts, int group_max, bool take_back) {
   hipStream_t st = w->stream;
   const int gb = blocks_for(std::max(a.nb, 1), kBlock);
   const int gs = blocks_for(std::max(a.n, 1), kBlock);
   const std::vector<int>& co = ts.color_off;
   const int ncol = int(co.size()) - 1;
-  if (a.n > 0) hipLaunchKernelGGL(k_af_geom, dim3(gs), dim3(kBlock), 0, st, a);
-  hipLaunchKernelGGL(k_af_intvel, dim3(gb), dim3(kBlock), 0, st, a);
+  const int T = a.n > 0 ? group_threads(ts, group_max) : 0;
+  hipLaunchKernelGGL(k_af_begin, dim3(gb), dim3(kBlock), 0, st, a, int(take_back));
   if (a.n > 0) {
-    hipLaunchKernelGGL(k_af_lam, dim3(gs), dim3(kBlock), 0, st, a);
-    if (ts.warm)
-      for (int c = 0; c < ncol; ++c)
-        if (co[c + 1] > co[c])
-          hipLaunchKernelGGL(k_af_warm, dim3(blocks_for(co[c + 1] - co[c], kBlock)), dim3(kBlock), 0, st, a, co[c],
-                             co[c + 1]);
-    for (int it = 0; it < ts.vel_iters; ++it)
-      for (int c = 0; c < ncol; ++c)
-        if (co[c + 1] > co[c])
-          hipLaunchKernelGGL(k_af_vel, dim3(blocks_for(co[c + 1] - co[c], kBlock)), dim3(kBlock), 0, st, a, co[c],
-                             co[c + 1], it);
-    hipLaunchKernelGGL(k_af_store, dim3(gs), dim3(kBlock), 0, st, a);
+    hipLaunchKernelGGL(k_af_init, dim3(gs), dim3(kBlock), 0, st, a);
+    if (T > 0) {
+      const GroupView v = group_view(w, ts, ts.vel_iters);
+      B2G_LAUNCH_GROUPS(T, k_af_group_vel, st, a, v);
+    } else {
+      auto range = [&](int c) { return dim3(blocks_for(co[c + 1] - co[c], kBlock)); };
+      if (ts.warm)
+        for (int c = 0; c < ncol; ++c)
+          hipLaunchKernelGGL(k_af_warm, range(c), dim3(kBlock), 0, st, a, co[c], co[c + 1]);
+      for (int it = 0; it < ts.vel_iters; ++it)
+        for (int c = 0; c < ncol; ++c)
+          hipLaunchKernelGGL(k_af_vel, range(c), dim3(kBlock), 0, st, a, co[c], co[c + 1], it);
+      hipLaunchKernelGGL(k_af_store, dim3(gs), dim3(kBlock), 0, st, a);
+    }
   }
   hipLaunchKernelGGL(k_af_intpos, dim3(gb), dim3(kBlock), 0, st, a);
-  if (a.n > 0)
+  if (T > 0 && ts.pos_iters > 0) {
+    const GroupView v = group_view(w, ts, ts.pos_iters);
+    B2G_LAUNCH_GROUPS(T, k_af_group_pos, st, a, v);
+  } else if (a.n > 0) {
     for (int it = 0; it < ts.pos_iters; ++it)
       for (int c = 0; c < ncol; ++c)
-        if (co[c + 1] > co[c])
-          hipLaunchKernelGGL(k_af_pos, dim3(blocks_for(co[c + 1] - co[c], kBlock)), dim3(kBlock), 0, st, a, co[c],
-                             co[c + 1], it);
+        hipLaunchKernelGGL(k_af_pos, dim3(blocks_for(co[c + 1] - co[c], kBlock)), dim3(kBlock), 0, st, a, co[c],
+                           co[c + 1], it);
+  }
   B2G_HIP(hipGetLastError());
   return B2G_OK;
 }
@@ -847,38 +1105,46 @@ static int replay_step(World* w, const AdjCtx& a, const TapeStep& ts) {
 // state after the step and store_bar those of the step's stored impulses; on return pbar/vbar
 // hold the cotangents of the start state and store_bar has received those of the previous
 // step's stored impulses
-static int reverse_step(World* w, const AdjCtx& a, const TapeStep& ts) {
+static int reverse_step(World* w, const AdjCtx& a, const TapeStep& ts, int group_max) {
   hipStream_t st = w->stream;
   const int gb = blocks_for(std::max(a.nb, 1), kBlock);
   const int gs = blocks_for(std::max(a.n, 1), kBlock);
   const std::vector<int>& co = ts.color_off;
   const int ncol = int(co.size()) - 1;
-  auto range_groups = [&](int c) { return dim3(blocks_for((co[c + 1] - co[c]) * kVelGroups, kBlock)); };
-  auto range_pos = [&](int c) { return dim3(blocks_for((co[c + 1] - co[c]) * kPosGroups, kBlock)); };
-  if (a.n > 0) {
+  const int T = a.n > 0 ? group_threads(ts, group_max) : 0;
+  auto range = [&](int c) { return dim3(blocks_for(co[c + 1] - co[c], kBlock)); };
+  if (T > 0) {
+    const GroupView v = group_view(w, ts, ts.pos_iters);
+    B2G_LAUNCH_GROUPS(T, k_ab_group_pos, st, a, v);
+  } else if (a.n > 0) {
     hipLaunchKernelGGL(k_ab_clear, dim3(gs), dim3(kBlock), 0, st, a);
     for (int it = ts.pos_iters - 1; it >= 0; --it)
       for (int c = ncol - 1; c >= 0; --c)
-        if (co[c + 1] > co[c])
-          hipLaunchKernelGGL(k_ab_pos, range_pos(c), dim3(kBlock), 0, st, a, co[c], co[c + 1], it);
+        hipLaunchKernelGGL(k_ab_pos, range(c), dim3(kBlock), 0, st, a, co[c], co[c + 1], it);
   }
   hipLaunchKernelGGL(k_ab_intpos, dim3(gb), dim3(kBlock), 0, st, a);
   if (a.n > 0) {
-    hipLaunchKernelGGL(k_ab_store, dim3(gs), dim3(kBlock), 0, st, a);
-    for (int it = ts.vel_iters - 1; it >= 0; --it)
-      for (int c = ncol - 1; c >= 0; --c)
-        if (co[c + 1] > co[c])
-          hipLaunchKernelGGL(k_ab_vel, range_groups(c), dim3(kBlock), 0, st, a, co[c], co[c + 1], it);
-    if (ts.warm)
-      for (int c = ncol - 1; c >= 0; --c)
-        if (co[c + 1] > co[c])
-          hipLaunchKernelGGL(k_ab_warm, range_groups(c), dim3(kBlock), 0, st, a, co[c], co[c + 1]);
-    hipLaunchKernelGGL(k_ab_setup, dim3(gs), dim3(kBlock), 0, st, a);
+    if (T > 0) {
+      const GroupView v = group_view(w, ts, ts.vel_iters);
+      B2G_LAUNCH_GROUPS(T, k_ab_group_vel, st, a, v);
+    } else {
+      hipLaunchKernelGGL(k_ab_store, dim3(gs), dim3(kBlock), 0, st, a);
+      for (int it = ts.vel_iters - 1; it >= 0; --it)
+        for (int c = ncol - 1; c >= 0; --c)
+          hipLaunchKernelGGL(k_ab_vel, range(c), dim3(kBlock), 0, st, a, co[c], co[c + 1], it);
+      if (ts.warm) hipLaunchKernelGGL(k_ab_warm, dim3(gs), dim3(kBlock), 0, st, a);
+    }
+    hipLaunchKernelGGL(k_ab_init, dim3(blocks_for(static_cast<long long>(a.n) * kInitGroups, kBlock)), dim3(kBlock), 0,
+                       st, a);
+    hipLaunchKernelGGL(k_ab_setup, dim3(blocks_for(4ll * a.n, kBlock)), dim3(kBlock), 0, st, a);
   }
   hipLaunchKernelGGL(k_ab_intvel, dim3(gb), dim3(kBlock), 0, st, a);
   B2G_HIP(hipGetLastError());
   return B2G_OK;
 }
+
+// of the card's 288 GB: about 80 kept steps of 1024 worlds of 64 bodies (70,000 contacts)
+static constexpr size_t kKeepBytes = size_t(4) << 30;
 
 static int reserve_buffers(World* w, AdjBuffers& B, bool backward) {
   Tape& t = w->tape;
@@ -891,23 +1157,41 @@ static int reserve_buffers(World* w, AdjBuffers& B, bool backward) {
     maxv = std::max(maxv, ts.vel_iters);
     maxp = std::max(maxp, ts.pos_iters);
   }
-  const size_t K = size_t(t.every);
+  const size_t K = size_t(t.every), seg = std::min(K, t.steps.size());
+  // The reverse pass keeps what its replay of a segment records for all of the segment's steps when
+  // that fits kKeepBytes; otherwise each step is replayed once more just before its reverse.
+  const size_t step_bytes =
+      sizeof(float4) * (maxn * (3 + kVelcRows + 3 * size_t(maxv) + 2 * size_t(maxp)) + 3 * nb);
+  B.keep = backward && seg * step_bytes <= kKeepBytes;
+  B.max_slots = maxn;
+  B.vel_iters = maxv;
+  B.pos_iters = maxp;
+  const size_t S = B.keep ? seg : 1;
   int st;
-  if ((st = B.pos.reserve(nb)) || (st = B.vel.reserve(nb)) || (st = B.vstar.reserve(nb)) ||
-      (st = B.geom.reserve(2 * maxn)) || (st = B.lam_cur.reserve(maxn)) || (st = B.lam_init.reserve(maxn)) ||
-      (st = B.lam0eff.reserve(maxn)) || (st = B.err.reserve(1)) || (st = B.seg_pos.reserve(K * nb)) ||
-      (st = B.seg_vel.reserve(K * nb)))
+  if ((st = B.pos.reserve(nb)) || (st = B.vel.reserve(nb)) || (st = B.vstar.reserve(S * nb)) ||
+      (st = B.geom.reserve(S * 2 * maxn)) || (st = B.velc.reserve(S * kVelcRows * maxn)) ||
+      (st = B.lam_cur.reserve(maxn)) || (st = B.lam_init.reserve(S * maxn)) || (st = B.lam0eff.reserve(maxn)) || (st = B.err.reserve(1)) ||
+      (st = B.seg_pos.reserve(K * nb)) || (st = B.seg_vel.reserve(K * nb)))
     return st;
   if (backward) {
-    if ((st = B.t_ws.reserve(2 * maxn)) || (st = B.t_vel.reserve(3 * size_t(maxv) * maxn)) ||
-        (st = B.t_ip.reserve(2 * nb)) || (st = B.t_pos.reserve(2 * size_t(maxp) * maxn)) ||
-        (st = B.pbar.reserve(nb)) || (st = B.vbar.reserve(nb)) || (st = B.lambar.reserve(maxn)) ||
-        (st = B.lam0bar.reserve(maxn)) || (st = B.qnbar.reserve(2 * maxn)) || (st = B.gbar.reserve(2 * maxn)) ||
-        (st = B.vsbar.reserve(2 * maxn)) || (st = B.store_bar.reserve(size_t(std::max<long long>(t.total, 1)))) ||
-        (st = B.fricbar.reserve(maxn)) || (st = B.fric_grad.reserve(nf)))
+    if ((st = B.t_vel.reserve(S * 3 * size_t(maxv) * maxn)) || (st = B.t_ip.reserve(S * 2 * nb)) ||
+        (st = B.t_pos.reserve(S * 2 * size_t(maxp) * maxn)) || (st = B.pbar.reserve(nb)) || (st = B.vbar.reserve(nb)) ||
+        (st = B.lambar.reserve(maxn)) || (st = B.lam0bar.reserve(maxn)) || (st = B.qnbar.reserve(2 * maxn)) ||
+        (st = B.gbar.reserve(2 * maxn)) || (st = B.vsbar.reserve(2 * maxn)) ||
+        (st = B.velcbar.reserve(kVelcRows * maxn)) ||
+        (st = B.store_bar.reserve(size_t(std::max<long long>(t.total, 1)))) || (st = B.fric_grad.reserve(nf)))
       return st;
   }
   B2G_HIP(hipMemsetAsync(B.err.p, 0, sizeof(int), w->stream));
+  return B2G_OK;
+}
+
+// the largest group of every recorded step (steps without slots: unused)
+static int fetch_group_max(World* w, std::vector<int>& out) {
+  Tape& t = w->tape;
+  out.assign(t.steps.size(), 0);
+  B2G_HIP(hipMemcpyAsync(out.data(), t.group_max.p, sizeof(int) * out.size(), hipMemcpyDeviceToHost, w->stream));
+  B2G_HIP(hipStreamSynchronize(w->stream));
   return B2G_OK;
 }
 
@@ -948,32 +1232,25 @@ int tape_replay(World* w, float* final_state) {
     return B2G_ERR_INVALID_ARGUMENT;
   }
   const int nb = w->nb;
-  AdjBuffers B;
+  AdjBuffers& B = t.buf;
+  std::vector<int> group_max;
   int st = reserve_buffers(w, B, false);
-  if (st) { B.release(); return st; }
+  if (st || (st = fetch_group_max(w, group_max))) return st;
   AdjCtx a = make_ctx(w, B);
   hipStream_t s = w->stream;
   if (hipMemcpyAsync(B.pos.p, t.ck_pos.p, sizeof(float4) * nb, hipMemcpyDeviceToDevice, s) != hipSuccess ||
       hipMemcpyAsync(B.vel.p, t.ck_vel.p, sizeof(float4) * nb, hipMemcpyDeviceToDevice, s) != hipSuccess) {
-    B.release();
     set_error("adjoint: copy failed");
     return B2G_ERR_DEVICE;
   }
-  for (const TapeStep& ts : t.steps) {
-    if (hipMemcpyAsync(B.seg_pos.p, B.pos.p, sizeof(float4) * nb, hipMemcpyDeviceToDevice, s) != hipSuccess ||
-        hipMemcpyAsync(B.seg_vel.p, B.vel.p, sizeof(float4) * nb, hipMemcpyDeviceToDevice, s) != hipSuccess) {
-      B.release();
-      set_error("adjoint: copy failed");
-      return B2G_ERR_DEVICE;
-    }
-    set_step(a, ts, B.seg_pos.p, B.seg_vel.p, 0);
-    if ((st = replay_step(w, a, ts))) { B.release(); return st; }
+  for (size_t n = 0; n < t.steps.size(); ++n) {
+    set_step(a, B, t.steps[n], B.seg_pos.p, B.seg_vel.p, 0, 0);
+    if ((st = replay_step(w, a, t.steps[n], group_max[n], false))) return st;
   }
   std::vector<float4> p(nb), v(nb);
   bool ok = hipMemcpyAsync(p.data(), B.pos.p, sizeof(float4) * nb, hipMemcpyDeviceToHost, s) == hipSuccess &&
             hipMemcpyAsync(v.data(), B.vel.p, sizeof(float4) * nb, hipMemcpyDeviceToHost, s) == hipSuccess;
   st = ok ? check_replay(w, B) : B2G_ERR_DEVICE;
-  B.release();
   if (!ok) { set_error("adjoint: readback failed"); return B2G_ERR_DEVICE; }
   if (st) return st;
   from_float4(final_state, p, v, nb);
@@ -989,15 +1266,15 @@ int tape_backward(World* w, const float* cot, float* grad0, float* grad_friction
   const int nb = w->nb, nf = w->np;
   const int N = int(t.steps.size());
   const int K = t.every;
-  AdjBuffers B;
+  AdjBuffers& B = t.buf;
+  std::vector<int> group_max;
   int st = reserve_buffers(w, B, true);
-  if (st) { B.release(); return st; }
+  if (st || (st = fetch_group_max(w, group_max))) return st;
   AdjCtx a = make_ctx(w, B);
   hipStream_t s = w->stream;
   std::vector<float4> hp, hv;
   to_float4(cot, hp, hv, nb);
   auto fail = [&](const char* msg) {
-    B.release();
     set_error(msg);
     return B2G_ERR_DEVICE;
   };
@@ -1014,23 +1291,15 @@ int tape_backward(World* w, const float* cot, float* grad0, float* grad_friction
         hipMemcpyAsync(B.vel.p, t.ck_vel.p + size_t(seg) * nb, bytes, hipMemcpyDeviceToDevice, s) != hipSuccess)
       return fail("adjoint: copy failed");
     for (int n = n0; n < n1; ++n) {
-      float4* sp = B.seg_pos.p + size_t(n - n0) * nb;
-      float4* sv = B.seg_vel.p + size_t(n - n0) * nb;
-      if (hipMemcpyAsync(sp, B.pos.p, bytes, hipMemcpyDeviceToDevice, s) != hipSuccess ||
-          hipMemcpyAsync(sv, B.vel.p, bytes, hipMemcpyDeviceToDevice, s) != hipSuccess)
-        return fail("adjoint: copy failed");
-      set_step(a, t.steps[n], sp, sv, 0);
-      if ((st = replay_step(w, a, t.steps[n]))) { B.release(); return st; }
+      set_step(a, B, t.steps[n], B.seg_pos.p + size_t(n - n0) * nb, B.seg_vel.p + size_t(n - n0) * nb, B.keep,
+               B.keep ? n - n0 : 0);
+      if ((st = replay_step(w, a, t.steps[n], group_max[n], false))) return st;
     }
     for (int n = n1 - 1; n >= n0; --n) {
-      float4* sp = B.seg_pos.p + size_t(n - n0) * nb;
-      float4* sv = B.seg_vel.p + size_t(n - n0) * nb;
-      if (hipMemcpyAsync(B.pos.p, sp, bytes, hipMemcpyDeviceToDevice, s) != hipSuccess ||
-          hipMemcpyAsync(B.vel.p, sv, bytes, hipMemcpyDeviceToDevice, s) != hipSuccess)
-        return fail("adjoint: copy failed");
-      set_step(a, t.steps[n], sp, sv, 1);
-      if ((st = replay_step(w, a, t.steps[n]))) { B.release(); return st; }
-      if ((st = reverse_step(w, a, t.steps[n]))) { B.release(); return st; }
+      set_step(a, B, t.steps[n], B.seg_pos.p + size_t(n - n0) * nb, B.seg_vel.p + size_t(n - n0) * nb, 1,
+               B.keep ? n - n0 : 0);
+      if (!B.keep && (st = replay_step(w, a, t.steps[n], group_max[n], true))) return st;
+      if ((st = reverse_step(w, a, t.steps[n], group_max[n]))) return st;
     }
   }
   std::vector<float> fg(std::max(nf, 1));
@@ -1039,7 +1308,6 @@ int tape_backward(World* w, const float* cot, float* grad0, float* grad_friction
             hipMemcpyAsync(fg.data(), B.fric_grad.p, sizeof(float) * std::max(nf, 1), hipMemcpyDeviceToHost, s) ==
                 hipSuccess;
   st = ok ? check_replay(w, B) : B2G_ERR_DEVICE;
-  B.release();
   if (!ok) { set_error("adjoint: readback failed"); return B2G_ERR_DEVICE; }
   if (st) return st;
   from_float4(grad0, hp, hv, nb);

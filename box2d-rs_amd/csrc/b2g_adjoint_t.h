@@ -164,4 +164,346 @@ struct PosFn {
   }
 };
 
+// ---- reverse of the solve's inner functions, by hand --------------------------------------------
+// The velocity and position iterations run on every constraint eight and three times a step, and a
+// constraint is a function of 31 (14) inputs: contracting dual lanes costs 16 (7) evaluations of it.
+// These walk the same operations backwards once instead. The constraint record c (which only the
+// start of the solve fixes) is an input of its own: its cotangents are summed over the iterations
+// and go through initialize_velocity_constraints once (InitFn). Branches are those of the primal
+// functions (b2g_step_t.h), comparison by comparison.
+
+// cotangents of a velocity applied by the impulse P at the arms ra, rb (A.v -= mA P, A.w -= iA ra x P,
+// B.v += mB P, B.w += iB rb x P): returns P's, adds the arms'
+template <class T, class S>
+B2G_HD TV2<T> impulse_bar(const TContactConst<S>& k, TV2<T> ra, TV2<T> rb, TV2<T> P, const TVel<T>& Ab,
+                          const TVel<T>& Bb, TV2<T>& rab, TV2<T>& rbb) {
+  const T ca = -T(k.iA) * Ab.w, cb = T(k.iB) * Bb.w;
+  rab = rab + ca * v2(P.y, -P.x);
+  rbb = rbb + cb * v2(P.y, -P.x);
+  return v2(-T(k.mA) * Ab.v.x + T(k.mB) * Bb.v.x - ca * ra.y - cb * rb.y,
+            -T(k.mA) * Ab.v.y + T(k.mB) * Bb.v.y + ca * ra.x + cb * rb.x);
+}
+
+// cotangents through the relative velocity dv = B.v + B.w x rb - A.v - A.w x ra
+template <class T>
+B2G_HD void relative_velocity_bar(TV2<T> dvb, TV2<T> ra, TV2<T> rb, T wa, T wb, TVel<T>& Ab, TVel<T>& Bb, TV2<T>& rab,
+                                  TV2<T>& rbb) {
+  Ab.v = Ab.v - dvb;
+  Bb.v = Bb.v + dvb;
+  Ab.w -= ra.x * dvb.y - ra.y * dvb.x;
+  Bb.w += rb.x * dvb.y - rb.y * dvb.x;
+  rab = rab + v2(-wa * dvb.y, wa * dvb.x);
+  rbb = rbb + v2(wb * dvb.y, -wb * dvb.x);
+}
+
+// the contact tangent is cross(normal, 1)
+template <class T>
+B2G_HD void tangent_bar(TV2<T> tb, TV2<T>& nb) {
+  nb.x -= tb.y;
+  nb.y += tb.x;
+}
+
+// Reverse of solve_velocity_t at (c, lam, A, B): Ab, Bb, lb hold the cotangents of the velocities and
+// impulses after it and return those before it; cb (a record of cotangents) is added to.
+template <class T, class S>
+B2G_HD void solve_velocity_bar(const TVelC<T>& c, const TContactConst<S>& k, const T lam_in[4], TVel<T> A, TVel<T> B,
+                               bool block_solve, TVel<T>& Ab, TVel<T>& Bb, T lb[4], TVelC<T>& cb) {
+  const T mA = T(k.mA), iA = T(k.iA), mB = T(k.mB), iB = T(k.iB);
+  const TV2<T> n = c.normal, t = cross(n, T(1.0));
+  T lam[4] = {lam_in[0], lam_in[1], lam_in[2], lam_in[3]};
+  auto apply = [&](TV2<T> ra, TV2<T> rb, TV2<T> P) {
+    A.v = A.v - mA * P;
+    A.w -= iA * cross(ra, P);
+    B.v = B.v + mB * P;
+    B.w += iB * cross(rb, P);
+  };
+  auto relative = [&](TV2<T> ra, TV2<T> rb) { return ((B.v + cross(B.w, rb)) - A.v) - cross(A.w, ra); };
+  // forward, keeping what the way back needs: per friction point its relative velocity, angular
+  // velocities, impulse change and branch (0 inside, 1 at +limit, -1 at -limit)
+  TV2<T> fdv[2];
+  T fwa[2], fwb[2], fdl[2];
+  int fbr[2];
+#pragma unroll
+  for (int p = 0; p < 2; ++p) {
+    if (p >= c.vcount) break;
+    fdv[p] = relative(c.ra[p], c.rb[p]);
+    fwa[p] = A.w;
+    fwb[p] = B.w;
+    const T vt = dot(fdv[p], t) - T(0.0);
+    const T u = lam[2 * p + 1] + c.tm[p] * (-vt);
+    const T hi = c.friction * lam[2 * p], lo = -hi;
+    const T m = u < hi ? u : hi;
+    fbr[p] = lo > m ? -1 : u < hi ? 0 : 1;
+    const T nw = lo > m ? lo : m;
+    fdl[p] = nw - lam[2 * p + 1];
+    lam[2 * p + 1] = nw;
+    apply(c.ra[p], c.rb[p], fdl[p] * t);
+  }
+  TV2<T> nb = v2(T(0.0), T(0.0)), tb = nb;
+  if (c.vcount == 1 || !block_solve) {
+    TV2<T> dv[2];
+    T wa[2], wb[2], dl[2];
+    bool pos[2];
+#pragma unroll
+    for (int p = 0; p < 2; ++p) {
+      if (p >= c.vcount) break;
+      dv[p] = relative(c.ra[p], c.rb[p]);
+      wa[p] = A.w;
+      wb[p] = B.w;
+      const T u = lam[2 * p] + -c.nm[p] * (dot(dv[p], n) - c.bias[p]);
+      pos[p] = u > T(0.0);
+      const T nw = pos[p] ? u : T(0.0);
+      dl[p] = nw - lam[2 * p];
+      lam[2 * p] = nw;
+      apply(c.ra[p], c.rb[p], dl[p] * n);
+    }
+#pragma unroll
+    for (int p = 1; p >= 0; --p) {
+      if (p >= c.vcount) continue;
+      const TV2<T> Pb = impulse_bar(k, c.ra[p], c.rb[p], dl[p] * n, Ab, Bb, cb.ra[p], cb.rb[p]);
+      const T dlb = dot(Pb, n);
+      nb = nb + dl[p] * Pb;
+      const T ub = pos[p] ? lb[2 * p] + dlb : T(0.0);
+      lb[2 * p] = ub - dlb;
+      const T e = dot(dv[p], n) - c.bias[p];
+      cb.nm[p] -= e * ub;
+      cb.bias[p] += c.nm[p] * ub;
+      const T vnb = -c.nm[p] * ub;
+      nb = nb + vnb * dv[p];
+      relative_velocity_bar(vnb * n, c.ra[p], c.rb[p], wa[p], wb[p], Ab, Bb, cb.ra[p], cb.rb[p]);
+    }
+  } else {
+    // The impulses' change d = x - aa solves K d = -r with r = vn - bias (case 1), or one row of it
+    // with the other impulse at zero (cases 2 and 3). The cotangents are those of that solve: written
+    // through K, its inverse and aa separately, as the primal computes x, they would be differences
+    // of terms up to a thousand times larger (the condition number the block solver allows).
+    const TV2<T> aa = v2(lam[0], lam[2]);
+    const TV2<T> dv1 = relative(c.ra[0], c.rb[0]), dv2 = relative(c.ra[1], c.rb[1]);
+    const TV2<T> Ka = v2(c.K[0] * aa.x + c.K[2] * aa.y, c.K[1] * aa.x + c.K[3] * aa.y);
+    const TV2<T> b = v2(dot(dv1, n) - c.bias[0], dot(dv2, n) - c.bias[1]) - Ka;
+    int which = 0;  // the case taken; 0: none
+    TV2<T> x = -v2(c.NM[0] * b.x + c.NM[2] * b.y, c.NM[1] * b.x + c.NM[3] * b.y);
+    if (x.x >= T(0.0) && x.y >= T(0.0)) {
+      which = 1;
+    } else {
+      const T x0 = -c.nm[0] * b.x, x1 = -c.nm[1] * b.y;
+      if (x0 >= T(0.0) && c.K[1] * x0 + b.y >= T(0.0)) {
+        which = 2;
+        x = v2(x0, T(0.0));
+      } else if (x1 >= T(0.0) && c.K[2] * x1 + b.x >= T(0.0)) {
+        which = 3;
+        x = v2(T(0.0), x1);
+      } else if (b.x >= T(0.0) && b.y >= T(0.0)) {
+        which = 4;
+        x = v2(T(0.0), T(0.0));
+      }
+    }
+    if (which) {
+      const TV2<T> d = x - aa;
+      const TV2<T> P1b = impulse_bar(k, c.ra[0], c.rb[0], d.x * n, Ab, Bb, cb.ra[0], cb.rb[0]);
+      const TV2<T> P2b = impulse_bar(k, c.ra[1], c.rb[1], d.y * n, Ab, Bb, cb.ra[1], cb.rb[1]);
+      nb = nb + (d.x * P1b + d.y * P2b);
+      const TV2<T> db = v2(dot(P1b, n), dot(P2b, n));
+      const TV2<T> xb = v2(lb[0] + db.x, lb[2] + db.y);
+      TV2<T> bb = v2(T(0.0), T(0.0));  // of r
+      if (which == 1) {
+        bb = -v2(c.NM[0] * xb.x + c.NM[1] * xb.y, c.NM[2] * xb.x + c.NM[3] * xb.y);
+        cb.K[0] += d.x * bb.x;
+        cb.K[2] += d.y * bb.x;
+        cb.K[1] += d.x * bb.y;
+        cb.K[3] += d.y * bb.y;
+      } else if (which == 2) {
+        bb.x = -c.nm[0] * xb.x;
+        cb.K[0] += d.x * bb.x;
+        cb.K[2] -= aa.y * bb.x;
+        lb[2] = -db.y - c.K[2] * bb.x;
+      } else if (which == 3) {
+        bb.y = -c.nm[1] * xb.y;
+        cb.K[3] += d.y * bb.y;
+        cb.K[1] -= aa.x * bb.y;
+        lb[0] = -db.x - c.K[1] * bb.y;
+      } else {
+        lb[0] = -db.x;
+        lb[2] = -db.y;
+      }
+      cb.bias[0] -= bb.x;
+      cb.bias[1] -= bb.y;
+      nb = nb + (bb.x * dv1 + bb.y * dv2);
+      const T wa = A.w, wb = B.w;
+      relative_velocity_bar(bb.x * n, c.ra[0], c.rb[0], wa, wb, Ab, Bb, cb.ra[0], cb.rb[0]);
+      relative_velocity_bar(bb.y * n, c.ra[1], c.rb[1], wa, wb, Ab, Bb, cb.ra[1], cb.rb[1]);
+    }
+  }
+#pragma unroll
+  for (int p = 1; p >= 0; --p) {
+    if (p >= c.vcount) continue;
+    const TV2<T> Pb = impulse_bar(k, c.ra[p], c.rb[p], fdl[p] * t, Ab, Bb, cb.ra[p], cb.rb[p]);
+    const T dlb = dot(Pb, t);
+    tb = tb + fdl[p] * Pb;
+    const T nwb = lb[2 * p + 1] + dlb;
+    const T ub = fbr[p] == 0 ? nwb : T(0.0);
+    const T limb = fbr[p] == 0 ? T(0.0) : T(fbr[p]) * nwb;
+    lb[2 * p + 1] = ub - dlb;
+    cb.friction += limb * lam_in[2 * p];
+    lb[2 * p] += limb * c.friction;
+    cb.tm[p] -= dot(fdv[p], t) * ub;
+    const T vtb = -c.tm[p] * ub;
+    tb = tb + vtb * fdv[p];
+    relative_velocity_bar(vtb * t, c.ra[p], c.rb[p], fwa[p], fwb[p], Ab, Bb, cb.ra[p], cb.rb[p]);
+  }
+  tangent_bar(tb, nb);
+  cb.normal = cb.normal + nb;
+}
+
+// Reverse of warm_start_t: the velocities' cotangents pass through unchanged, so the constraints
+// of all colours may be taken in any order.
+template <class T, class S>
+B2G_HD void warm_start_bar(const TVelC<T>& c, const TContactConst<S>& k, const T lam[4], const TVel<T>& Ab,
+                           const TVel<T>& Bb, T lb[4], TVelC<T>& cb) {
+  const TV2<T> n = c.normal, t = cross(n, T(1.0));
+  TV2<T> nb = v2(T(0.0), T(0.0)), tb = nb;
+#pragma unroll
+  for (int p = 0; p < 2; ++p) {
+    if (p >= c.vcount) break;
+    const TV2<T> P = lam[2 * p] * n + lam[2 * p + 1] * t;
+    const TV2<T> Pb = impulse_bar(k, c.ra[p], c.rb[p], P, Ab, Bb, cb.ra[p], cb.rb[p]);
+    lb[2 * p] += dot(Pb, n);
+    lb[2 * p + 1] += dot(Pb, t);
+    nb = nb + lam[2 * p] * Pb;
+    tb = tb + lam[2 * p + 1] * Pb;
+  }
+  tangent_bar(tb, nb);
+  cb.normal = cb.normal + nb;
+}
+
+// Reverse of solve_position_t at (g, A, B): Ab, Bb hold the cotangents of the positions after it and
+// return those before it; gb is added to.
+template <class T, class S>
+B2G_HD void solve_position_bar(const TContactConst<S>& k, const TGeom<T>& g, TPos<T> A, TPos<T> B, TPos<T>& Ab,
+                               TPos<T>& Bb, TGeom<T>& gb) {
+  const T mA = T(k.mA), iA = T(k.iA), mB = T(k.mB), iB = T(k.iB);
+  const TV2<T> lcA = v2(T(k.lcA[0]), T(k.lcA[1])), lcB = v2(T(k.lcB[0]), T(k.lcB[1]));
+  // cotangents of u = X.c + R(X.a) (l - lc): X's and l's
+  auto point_bar = [](TV2<T> ub, TV2<T> arm, TRot<T> q, TPos<T>& X, TV2<T>& lb) {
+    const TV2<T> r = mul(q, arm);
+    X.c = X.c + ub;
+    X.a += r.x * ub.y - r.y * ub.x;
+    lb = lb + mulT(q, ub);
+  };
+  TPos<T> A1 = A, B1 = B;  // before the second point
+  if (k.count > 1) {
+    TContactConst<S> one = k;
+    one.count = 1;
+    solve_position_t(one, g, A1, B1);
+  }
+  for (int p = k.count - 1; p >= 0; --p) {
+    const TPos<T> a = p == 1 ? A1 : A, b = p == 1 ? B1 : B;
+    const TRot<T> qA = rot(a.a), qB = rot(b.a);
+    const bool face_a = k.type == kFaceA, circles = k.type == kCircles;
+    // first: the face (or circle A) point l1 on body 1; second: the other point l2 on body 2
+    const bool on_a = circles || face_a;
+    const TRot<T> q1 = on_a ? qA : qB, q2 = on_a ? qB : qA;
+    const TV2<T> arm1 = g.lpt - (on_a ? lcA : lcB), arm2 = (circles ? g.lp[0] : g.lp[p]) - (on_a ? lcB : lcA);
+    const TV2<T> u1 = (on_a ? a.c : b.c) + mul(q1, arm1), u2 = (on_a ? b.c : a.c) + mul(q2, arm2);
+    const TV2<T> d = u2 - u1;
+    TV2<T> nf = mul(q1, g.ln);  // the face normal
+    T length = T(0.0);
+    if (circles) {
+      nf = d;
+      length = normalize(&nf);
+    }
+    const T separation = dot(d, nf) - T(k.rA) - T(k.rB);
+    const TV2<T> point = circles ? T(0.5) * (u1 + u2) : u2;
+    const TV2<T> n = on_a ? nf : -nf;
+    const TV2<T> rA = point - a.c, rB = point - b.c;
+    const T y = T(kBaumgarteD) * (separation + T(kLinearSlopD));
+    const T lo = -T(kMaxLinearCorrectionD), m = y < T(0.0) ? y : T(0.0);
+    const bool inside = !(lo > m) && y < T(0.0);
+    const T C = lo > m ? lo : m;
+    const T rnA = cross(rA, n), rnB = cross(rB, n);
+    const T K = mA + mB + iA * rnA * rnA + iB * rnB * rnB;
+    const T impulse = K > T(0.0) ? -C / K : T(0.0);
+    const TV2<T> P = impulse * n;
+    // back
+    const T ca = -iA * Ab.a, cb = iB * Bb.a;
+    TV2<T> rAb = ca * v2(P.y, -P.x), rBb = cb * v2(P.y, -P.x);
+    const TV2<T> Pb = v2(-mA * Ab.c.x + mB * Bb.c.x - ca * rA.y - cb * rB.y,
+                         -mA * Ab.c.y + mB * Bb.c.y + ca * rA.x + cb * rB.x);
+    TV2<T> nb = impulse * Pb;
+    T sb = T(0.0);
+    if (K > T(0.0)) {
+      const T ib = dot(Pb, n) / K;
+      const T Kb = -ib * impulse;
+      const T ra = T(2.0) * iA * rnA * Kb, rb = T(2.0) * iB * rnB * Kb;
+      rAb = rAb + ra * v2(n.y, -n.x);
+      rBb = rBb + rb * v2(n.y, -n.x);
+      nb = nb + (ra * v2(-rA.y, rA.x) + rb * v2(-rB.y, rB.x));
+      if (inside) sb = -ib * T(kBaumgarteD);
+    }
+    const TV2<T> pb = rAb + rBb;
+    Ab.c = Ab.c - rAb;
+    Bb.c = Bb.c - rBb;
+    TV2<T> nfb = (on_a ? nb : -nb) + sb * d;
+    TV2<T> db = sb * nf;
+    TV2<T> u1b = v2(T(0.0), T(0.0)), u2b = pb;
+    TPos<T>& X1 = on_a ? Ab : Bb;
+    TPos<T>& X2 = on_a ? Bb : Ab;
+    if (circles) {
+      u1b = u2b = T(0.5) * pb;
+      // nf = d / |d| (left alone below the length where normalize does nothing)
+      if (length > T(0.0)) db = db + (T(1.0) / length) * (nfb - dot(nf, nfb) * nf);
+      else db = db + nfb;
+    } else {
+      X1.a += nf.x * nfb.y - nf.y * nfb.x;
+      gb.ln = gb.ln + mulT(q1, nfb);
+    }
+    point_bar(u1b - db, arm1, q1, X1, gb.lpt);
+    point_bar(u2b + db, arm2, q2, X2, p == 1 && !circles ? gb.lp[1] : gb.lp[0]);
+  }
+}
+
+// initialize_velocity_constraints as a function of what the solve holds fixed:
+// x = qA (3), qB (3), g (8), v*A (3), v*B (3) -> y = normal, ra[2], rb[2], nm[2], tm[2], bias[2], K[4]
+// (20; the friction passes through, and K's inverse has no cotangent of its own: see solve_velocity_bar)
+constexpr int kInitIn = 20, kInitOut = 20;
+template <class S>
+struct InitFn {
+  TContactConst<S> k;
+  bool block;
+  template <class T>
+  B2G_HD void operator()(const T* x, T* y) const {
+    const TVelC<T> c = init_velocity_t(k, geom_of(x + 6), T(0.0), pos_of(x), pos_of(x + 3), vel_of(x + 14),
+                                       vel_of(x + 17), block);
+    put_velc(y, c);
+  }
+  template <class T>
+  B2G_HD static void put_velc(T* y, const TVelC<T>& c) {
+    y[0] = c.normal.x; y[1] = c.normal.y;
+    for (int p = 0; p < 2; ++p) {
+      y[2 + 2 * p] = c.ra[p].x; y[3 + 2 * p] = c.ra[p].y;
+      y[6 + 2 * p] = c.rb[p].x; y[7 + 2 * p] = c.rb[p].y;
+      y[10 + p] = c.nm[p];
+      y[12 + p] = c.tm[p];
+      y[14 + p] = c.bias[p];
+    }
+    for (int i = 0; i < 4; ++i) y[16 + i] = c.K[i];
+  }
+};
+
+// a record of zeros (cotangents to be added to)
+template <class T>
+B2G_HD TVelC<T> zero_velc() {
+  TVelC<T> c;
+  const TV2<T> z = v2(T(0.0), T(0.0));
+  c.normal = z;
+  c.friction = T(0.0);
+  for (int p = 0; p < 2; ++p) {
+    c.ra[p] = c.rb[p] = z;
+    c.nm[p] = c.tm[p] = c.bias[p] = T(0.0);
+  }
+  for (int i = 0; i < 4; ++i) c.K[i] = c.NM[i] = T(0.0);
+  c.vcount = 0;
+  return c;
+}
+
 }  // namespace b2g

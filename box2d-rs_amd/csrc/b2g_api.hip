@@ -1547,7 +1547,7 @@ int b2g_tape_begin(b2g_world* h, int32_t checkpoint_every) {
   int st;
   if ((st = ensure_uploaded(w))) return st;
   B2G_HIP(hipStreamSynchronize(w->stream));
-  tape_release(w);
+  tape_reset(w);
   w->tape.active = true;
   w->tape.every = checkpoint_every;
   w->tape.nb = w->nb;

@@ -221,12 +221,34 @@ struct KernelTimer {
   long long aux = 0;  // a second count known only after the launch (pairs found by the traversal)
 };
 
+// Working memory of the adjoint's replay and reverse passes, kept with the tape (b2g_tape_free gives
+// it back).
+struct AdjBuffers {
+  DevArray<float4> pos, vel, seg_pos, seg_vel, vstar, geom, velc, lam_cur, lam_init, lam0eff;
+  DevArray<float4> t_vel, t_ip, t_pos;
+  DevArray<float4> pbar, vbar, lambar, lam0bar, qnbar, gbar, vsbar, velcbar, store_bar;
+  DevArray<float> fric_grad;
+  DevArray<int> err;
+  size_t max_slots = 0;  // slots of the largest step: the stride of the kept steps
+  int vel_iters = 0, pos_iters = 0;
+  bool keep = false;     // a segment's recorded inputs are kept for all of its steps
+  void release() {
+    for (auto* d : {&pos, &vel, &seg_pos, &seg_vel, &vstar, &geom, &velc, &lam_cur, &lam_init, &lam0eff, &t_vel, &t_ip,
+                    &t_pos, &pbar, &vbar, &lambar, &lam0bar, &qnbar, &gbar, &vsbar, &velcbar, &store_bar})
+      d->release();
+    fric_grad.release();
+    err.release();
+  }
+};
+
 // Recorded forward run for the adjoint. A slot is one touching contact of one step, in that
 // step's solve order; slots of all steps are concatenated.
 struct TapeStep {
   int n = 0;                    // slots of this step
   long long off = 0;            // first slot
   std::vector<int> color_off;   // colour offsets (relative to off)
+  int ng = 0;                   // groups per colour (bins or worlds) when the step's solve was grouped
+  long long goff = 0;           // its (colour, group) offsets in Tape::group_off
   float dt = 0.0f, dt_ratio = 0.0f;
   int vel_iters = 0, pos_iters = 0;
   bool warm = true, block = true;
@@ -242,12 +264,16 @@ struct Tape {
   DevArray<uint2> ids;          // feature ids (checked when the manifold is recomputed)
   DevArray<float4> lam0;        // impulses as collide carried them (the source when carry is -1)
   DevArray<float4> lam_store;   // impulses as store_impulses left them in the manifold
+  DevArray<int> group_off;      // per grouped step: first slot of each (colour, group), and the total
+  DevArray<int> group_max;      // per step: slots of its largest group
+  long long group_total = 0;
   DevArray<float4> c_lam0;      // contact-indexed scratch of the current step
   DevArray<int2> c_carry;       // per point: previous-set contact * 2 + point, or -1
   DevArray<long long> c_slot[2];// slot of each contact of the two contact sets, or -1
   DevArray<float4> ck_pos, ck_vel;  // body state at the start of every checkpointed step
   int ck_count = 0;
   int nb = 0;
+  AdjBuffers buf;
 };
 
 // Joints (distance, revolute): definitions, persistent impulses and per-step solver rows,
@@ -375,6 +401,7 @@ struct World {
   int island_solve = -1;
   int bin_threads = 256;
   int n_bins = 0;  // bins of the last solve
+  int solve_groups = 0;  // groups per colour of the last solve's constraints (s.cw_off); 0: not grouped
   bool worlds_contiguous = false;         // every world's bodies are one index range (set at upload)
   std::vector<int> h_world_body_off;      // n_worlds + 1 (when contiguous)
   std::vector<int> h_world_order;         // worlds by bucket, larger worlds first within a bucket
@@ -415,11 +442,54 @@ inline size_t pair_capacity(const World* w, size_t n) {
   return std::max(std::max(n, size_t(1)), size_t(w->np) * kPairsPerProxy);
 }
 
+constexpr int kMaxColors = 128;  // solve colours (two 64-bit masks)
+
+// ---- solve groups in one workgroup each (islands packed into bins, worlds of a batch) -------------
+constexpr int kBinHashPerThread = 4;  // body slots per thread (a bin has < 2T bodies)
+
+// slot of body (or island) id `key` in a linear-probing table of H = 2^lg entries (-1 = empty);
+// the table never fills (at most H/2 keys), so the probe ends
+__device__ inline int bin_slot(int* keys, int lg, int key) {
+  const int mask = (1 << lg) - 1;
+  int h = static_cast<int>((static_cast<unsigned>(key) * 2654435761u) >> (32 - lg));
+  for (;;) {
+    const int prev = atomicCAS(&keys[h], -1, key);
+    if (prev == -1 || prev == key) return h;
+    h = (h + 1) & mask;
+  }
+}
+
+// this thread's constraint: the t-th of its bin in colour order (-1: none); rng holds the bin's
+// range per colour
+__device__ inline int bin_constraint(const int2* rng, int ncolors, int t, int* colour) {
+  int base = 0;
+  for (int c = 0; c < ncolors; ++c) {
+    const int2 r = rng[c];
+    const int n = r.y - r.x;
+    if (t >= base && t < base + n) {
+      *colour = c;
+      return r.x + t - base;
+    }
+    base += n;
+  }
+  *colour = -1;
+  return -1;
+}
+
+template <int T>
+__device__ inline void bin_ranges(const int* __restrict__ off, int ng, int ncolors, int2* rng) {
+  const int g = blockIdx.x;
+  for (int c = threadIdx.x; c < ncolors; c += T) rng[c] = make_int2(off[c * ng + g], off[c * ng + g + 1]);
+}
+
+constexpr int ilog2(int x) { return x <= 1 ? 0 : 1 + ilog2(x / 2); }
+
 // adjoint tape hooks of b2g_world_step (b2g_adjoint.hip)
 int tape_step_begin(World* w);
 int tape_after_collide(World* w);
 int tape_after_solve(World* w, float dt, float dt_ratio, int vel_iters, int pos_iters);
-void tape_release(World* w);
+void tape_reset(World* w);    // empties the tape, keeping its memory for the next recording
+void tape_release(World* w);  // and gives the memory back
 int tape_replay(World* w, float* final_state);
 int tape_backward(World* w, const float* cotangent, float* grad_state, float* grad_friction);
 

@@ -19,7 +19,6 @@
 namespace b2g {
 
 static constexpr int kBlock = 256;
-static constexpr int kMaxColors = 128;
 // solver counter after the colour histogram and the last colouring round: constraints in islands
 // too large for the island solve's bins
 static constexpr int kBigIslandSlot = 4 + kMaxColors + 1;
@@ -896,47 +895,23 @@ __device__ inline void velocity_core(const float4 m, const float4 nf, float4& la
     V2 b = v2(vn1 - bias.x, vn2 - bias.y);
     V2 Ka = v2(K.x * aa.x + K.z * aa.y, K.y * aa.x + K.w * aa.y);
     b = b - Ka;
-    for (;;) {
-      // case 1: vn = 0
-      V2 x = -v2(NM.x * b.x + NM.z * b.y, NM.y * b.x + NM.w * b.y);
-      if (x.x >= 0.0f && x.y >= 0.0f) {
-        apply_normal_pair(va, wa, vb, wb, mA, iA, mB, iB, normal, r1a, r2a, r1b, r2b, x - aa);
-        lam.x = x.x;
-        lam.z = x.y;
-        break;
-      }
-      // case 2: vn1 = 0 and x2 = 0
-      x.x = -ms.x * b.x;
-      x.y = 0.0f;
-      vn2 = K.y * x.x + b.y;
-      if (x.x >= 0.0f && vn2 >= 0.0f) {
-        apply_normal_pair(va, wa, vb, wb, mA, iA, mB, iB, normal, r1a, r2a, r1b, r2b, x - aa);
-        lam.x = x.x;
-        lam.z = x.y;
-        break;
-      }
-      // case 3: vn2 = 0 and x1 = 0
-      x.x = 0.0f;
-      x.y = -ms.z * b.y;
-      vn1 = K.z * x.y + b.x;
-      if (x.y >= 0.0f && vn1 >= 0.0f) {
-        apply_normal_pair(va, wa, vb, wb, mA, iA, mB, iB, normal, r1a, r2a, r1b, r2b, x - aa);
-        lam.x = x.x;
-        lam.z = x.y;
-        break;
-      }
-      // case 4: x1 = 0 and x2 = 0
-      x.x = 0.0f;
-      x.y = 0.0f;
-      vn1 = b.x;
-      vn2 = b.y;
-      if (vn1 >= 0.0f && vn2 >= 0.0f) {
-        apply_normal_pair(va, wa, vb, wb, mA, iA, mB, iB, normal, r1a, r2a, r1b, r2b, x - aa);
-        lam.x = x.x;
-        lam.z = x.y;
-        break;
-      }
-      break;  // no solution: give up
+    // Total enumeration: 1: vn = 0; 2: vn1 = 0 and x2 = 0; 3: vn2 = 0 and x1 = 0; 4: x1 = 0 and x2 = 0.
+    // The lanes of a wave pick their cases first and then apply the impulses together: with the
+    // application inside each case a wave ran it once per case its lanes had taken.
+    V2 x = -v2(NM.x * b.x + NM.z * b.y, NM.y * b.x + NM.w * b.y);
+    bool solved = x.x >= 0.0f && x.y >= 0.0f;
+    if (!solved) {
+      const float x1 = -ms.x * b.x, x2 = -ms.z * b.y;
+      const bool c2 = x1 >= 0.0f && K.y * x1 + b.y >= 0.0f;
+      const bool c3 = x2 >= 0.0f && K.z * x2 + b.x >= 0.0f;
+      x.x = c2 ? x1 : 0.0f;
+      x.y = !c2 && c3 ? x2 : 0.0f;
+      solved = c2 || c3 || (b.x >= 0.0f && b.y >= 0.0f);
+    }
+    if (solved) {  // no solution: the impulses stay as they are
+      apply_normal_pair(va, wa, vb, wb, mA, iA, mB, iB, normal, r1a, r2a, r1b, r2b, x - aa);
+      lam.x = x.x;
+      lam.z = x.y;
     }
   }
   vA = make_float4(va.x, va.y, wa, 0.0f);
@@ -1348,45 +1323,6 @@ static void launch_worlds_position(World* w, long long items, const int* off, in
 // each thread holds one constraint in registers and the bin's bodies sit in an LDS hash table
 // (body id -> slot), loaded once and written back once. Islands of more than W constraints keep
 // the per-colour launches (their constraints are the last group of every colour).
-static constexpr int kBinHashPerThread = 4;  // body slots per thread (a bin has < 2T bodies)
-
-// slot of body (or island) id `key` in a linear-probing table of H = 2^lg entries (-1 = empty);
-// the table never fills (at most H/2 keys), so the probe ends
-__device__ inline int bin_slot(int* keys, int lg, int key) {
-  const int mask = (1 << lg) - 1;
-  int h = static_cast<int>((static_cast<unsigned>(key) * 2654435761u) >> (32 - lg));
-  for (;;) {
-    const int prev = atomicCAS(&keys[h], -1, key);
-    if (prev == -1 || prev == key) return h;
-    h = (h + 1) & mask;
-  }
-}
-
-// this thread's constraint: the t-th of its bin in colour order (-1: none); rng holds the bin's
-// range per colour
-__device__ inline int bin_constraint(const int2* rng, int ncolors, int t, int* colour) {
-  int base = 0;
-  for (int c = 0; c < ncolors; ++c) {
-    const int2 r = rng[c];
-    const int n = r.y - r.x;
-    if (t >= base && t < base + n) {
-      *colour = c;
-      return r.x + t - base;
-    }
-    base += n;
-  }
-  *colour = -1;
-  return -1;
-}
-
-template <int T>
-__device__ inline void bin_ranges(const int* __restrict__ off, int ng, int ncolors, int2* rng) {
-  const int g = blockIdx.x;
-  for (int c = threadIdx.x; c < ncolors; c += T) rng[c] = make_int2(off[c * ng + g], off[c * ng + g + 1]);
-}
-
-constexpr int ilog2(int x) { return x <= 1 ? 0 : 1 + ilog2(x / 2); }
-
 template <int T>
 __global__ void __launch_bounds__(T) k_solve_bins_velocity(const int* __restrict__ off, int ng, int ncolors, int iters,
                                                            int block_solve, VelArgs a) {
@@ -1908,7 +1844,9 @@ int phase_solve(World* w, float dt, float dt_ratio, int vel_iters, int pos_iters
   const bool bins = !serial && n_small > 0 && (w->island_solve == 1 || n_small >= n_big);
   const int nbins = bins ? (n_small + bin_cap - 1) / bin_cap : 0;
   w->n_bins = nbins;
+  w->solve_groups = bins && n_big == 0 ? nbins + 1 : 0;
   const bool per_world = nc > 0 && want_world && !want_bins && !serial;
+  if (per_world) w->solve_groups = w->n_worlds;
   if (nc > 0) {
     // One launch per non-empty colour, in colour-id order (kept colours can leave gaps).
     // Device copy: launch offsets (kMaxColors + 1, padded with nc), then per colour id its base

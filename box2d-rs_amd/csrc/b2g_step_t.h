@@ -230,45 +230,22 @@ B2G_HD void solve_velocity_t(const TVelC<T>& c, const TContactConst<S>& k, T lam
   TV2<T> b = v2(vn1 - c.bias[0], vn2 - c.bias[1]);
   TV2<T> Ka = v2(c.K[0] * aa.x + c.K[2] * aa.y, c.K[1] * aa.x + c.K[3] * aa.y);
   b = b - Ka;
-  // case 1: vn = 0
+  // case 1: vn = 0; 2: vn1 = 0 and x2 = 0; 3: vn2 = 0 and x1 = 0; 4: x1 = 0 and x2 = 0. The case is
+  // picked first and applied once, so that a wave's lanes apply theirs together.
   TV2<T> x = -v2(c.NM[0] * b.x + c.NM[2] * b.y, c.NM[1] * b.x + c.NM[3] * b.y);
-  if (x.x >= T(0.0) && x.y >= T(0.0)) {
-    apply_normal_pair_t(A, B, k, c, x - aa);
-    lam[0] = x.x;
-    lam[2] = x.y;
-    return;
+  bool solved = x.x >= T(0.0) && x.y >= T(0.0);
+  if (!solved) {
+    const T x1 = -c.nm[0] * b.x, x2 = -c.nm[1] * b.y;
+    const bool c2 = x1 >= T(0.0) && c.K[1] * x1 + b.y >= T(0.0);
+    const bool c3 = x2 >= T(0.0) && c.K[2] * x2 + b.x >= T(0.0);
+    x.x = c2 ? x1 : T(0.0);
+    x.y = !c2 && c3 ? x2 : T(0.0);
+    solved = c2 || c3 || (b.x >= T(0.0) && b.y >= T(0.0));
   }
-  // case 2: vn1 = 0 and x2 = 0
-  x.x = -c.nm[0] * b.x;
-  x.y = T(0.0);
-  vn2 = c.K[1] * x.x + b.y;
-  if (x.x >= T(0.0) && vn2 >= T(0.0)) {
-    apply_normal_pair_t(A, B, k, c, x - aa);
-    lam[0] = x.x;
-    lam[2] = x.y;
-    return;
-  }
-  // case 3: vn2 = 0 and x1 = 0
-  x.x = T(0.0);
-  x.y = -c.nm[1] * b.y;
-  vn1 = c.K[2] * x.y + b.x;
-  if (x.y >= T(0.0) && vn1 >= T(0.0)) {
-    apply_normal_pair_t(A, B, k, c, x - aa);
-    lam[0] = x.x;
-    lam[2] = x.y;
-    return;
-  }
-  // case 4: x1 = 0 and x2 = 0
-  x.x = T(0.0);
-  x.y = T(0.0);
-  vn1 = b.x;
-  vn2 = b.y;
-  if (vn1 >= T(0.0) && vn2 >= T(0.0)) {
-    apply_normal_pair_t(A, B, k, c, x - aa);
-    lam[0] = x.x;
-    lam[2] = x.y;
-  }
-  // no solution: the impulses stay as they are
+  if (!solved) return;  // no solution: the impulses stay as they are
+  apply_normal_pair_t(A, B, k, c, x - aa);
+  lam[0] = x.x;
+  lam[2] = x.y;
 }
 
 // solve_position_constraints for one constraint, point by point; returns the smallest

@@ -1,0 +1,166 @@
+// The hand-written reverse functions of the solve (box2d-rs_amd/csrc/b2g_adjoint_t.h) beside the dual-number
+// vector-Jacobian products of the same functors, in float and double. Test infrastructure only.
+#include "../../box2d-rs_amd/csrc/b2g_adjoint_t.h"
+
+using namespace b2g;
+
+namespace {
+
+// k: type, count, then restitution, threshold, rA, rB, mA, iA, mB, iB, lcA, lcB
+template <class S>
+TContactConst<S> contact(const int* tc, const double* k) {
+  TContactConst<S> c;
+  c.type = tc[0];
+  c.count = tc[1];
+  c.restitution = S(k[0]); c.threshold = S(k[1]);
+  c.rA = S(k[2]); c.rB = S(k[3]);
+  c.mA = S(k[4]); c.iA = S(k[5]); c.mB = S(k[6]); c.iB = S(k[7]);
+  c.lcA[0] = S(k[8]); c.lcA[1] = S(k[9]); c.lcB[0] = S(k[10]); c.lcB[1] = S(k[11]);
+  return c;
+}
+
+// through initialize_velocity_constraints: cotangents of x[10..24) and x[25..31)
+template <class S>
+void init_bar(const TContactConst<S>& k, bool block, const S* x, const TVelC<S>& cb, S* xb) {
+  S xi[kInitIn], yb[kInitOut], xib[kInitIn] = {};
+  for (int i = 0; i < 14; ++i) xi[i] = x[10 + i];
+  for (int i = 0; i < 6; ++i) xi[14 + i] = x[25 + i];
+  InitFn<S>::put_velc(yb, cb);
+  vjp<kInitIn, kInitOut, 4>(xi, yb, xib, InitFn<S>{k, block});
+  for (int i = 0; i < 14; ++i) xb[10 + i] += xib[i];
+  for (int i = 0; i < 6; ++i) xb[25 + i] += xib[14 + i];
+  xb[24] += cb.friction;
+}
+
+// which 0: one velocity iteration (yb 10), 1: warm start (yb 6)
+template <class S>
+void velocity(int which, bool hand, const int* tc, const double* kd, bool block, const double* xd, const double* ybd,
+              double* out) {
+  const TContactConst<S> k = contact<S>(tc, kd);
+  S x[kVelIn], yb[10], xb[kVelIn] = {};
+  for (int i = 0; i < kVelIn; ++i) x[i] = S(xd[i]);
+  for (int i = 0; i < 10; ++i) yb[i] = S(ybd[i]);
+  if (!hand) {
+    if (which == 0) vjp<kVelIn, 10, 8>(x, yb, xb, VelFn<S>{k, block});
+    else vjp<kVelIn, 6, 8>(x, yb, xb, WarmFn<S>{k, block});
+  } else {
+    const TVelC<S> c = velc_of(x, k, block);
+    TVelC<S> cb = zero_velc<S>();
+    TVel<S> Ab = vel_of(yb), Bb = vel_of(yb + 3);
+    S lb[4] = {yb[6], yb[7], yb[8], yb[9]};
+    if (which == 0) {
+      solve_velocity_bar(c, k, x + 6, vel_of(x), vel_of(x + 3), block, Ab, Bb, lb, cb);
+    } else {
+      for (S& l : lb) l = S(0);
+      warm_start_bar(c, k, x + 6, Ab, Bb, lb, cb);
+    }
+    put_vel(xb, Ab);
+    put_vel(xb + 3, Bb);
+    for (int i = 0; i < 4; ++i) xb[6 + i] = lb[i];
+    init_bar(k, block, x, cb, xb);
+  }
+  for (int i = 0; i < kVelIn; ++i) out[i] = double(xb[i]);
+}
+
+template <class S>
+void position(bool hand, const int* tc, const double* kd, const double* xd, const double* ybd, double* out) {
+  const TContactConst<S> k = contact<S>(tc, kd);
+  S x[14], yb[6], xb[14] = {};
+  for (int i = 0; i < 14; ++i) x[i] = S(xd[i]);
+  for (int i = 0; i < 6; ++i) yb[i] = S(ybd[i]);
+  if (!hand) {
+    vjp<14, 6, 7>(x, yb, xb, PosFn<S>{k});
+  } else {
+    TPos<S> Ab = pos_of(yb), Bb = pos_of(yb + 3);
+    S zero[8] = {};
+    TGeom<S> gb = geom_of(zero);
+    solve_position_bar(k, geom_of(x + 6), pos_of(x), pos_of(x + 3), Ab, Bb, gb);
+    put_pos(xb, Ab);
+    put_pos(xb + 3, Bb);
+    xb[6] = gb.ln.x; xb[7] = gb.ln.y; xb[8] = gb.lpt.x; xb[9] = gb.lpt.y;
+    xb[10] = gb.lp[0].x; xb[11] = gb.lp[0].y; xb[12] = gb.lp[1].x; xb[13] = gb.lp[1].y;
+  }
+  for (int i = 0; i < 14; ++i) out[i] = double(xb[i]);
+}
+
+// The warm start and `iters` velocity iterations of one constraint and their reverse, the way the two
+// adjoints walk them: by dual numbers every iteration through the whole functor, or by the reverse functions
+// with the constraint's cotangents summed and taken through its set-up once. The states are those of the float
+// forward run (S decides the reverse's arithmetic only), so the difference between S = float and double is
+// the reverse's rounding alone.
+template <class S>
+void chain(bool hand, const int* tc, const double* kd, bool block, int iters, const double* xd, const double* ybd,
+           double* out) {
+  const TContactConst<float> kf = contact<float>(tc, kd);
+  const TContactConst<S> k = contact<S>(tc, kd);
+  float xf[kVelIn];
+  for (int i = 0; i < kVelIn; ++i) xf[i] = float(xd[i]);
+  const TVelC<float> cf = velc_of(xf, kf, block);
+  float lam[4] = {xf[6], xf[7], xf[8], xf[9]};
+  TVel<float> A = vel_of(xf), B = vel_of(xf + 3);
+  constexpr int kMost = 32;
+  S st[kMost + 1][10];
+  auto keep = [&](int i) {
+    float v[10];
+    put_vel(v, A);
+    put_vel(v + 3, B);
+    for (int j = 0; j < 4; ++j) v[6 + j] = lam[j];
+    for (int j = 0; j < 10; ++j) st[i][j] = S(v[j]);
+  };
+  keep(0);
+  warm_start_t(cf, kf, lam, A, B);
+  for (int it = 0; it < iters; ++it) {
+    keep(1 + it);
+    solve_velocity_t(cf, kf, lam, A, B, block);
+  }
+  S x[kVelIn], yb[10], xb[kVelIn] = {};
+  for (int i = 0; i < kVelIn; ++i) x[i] = S(xf[i]);
+  for (int i = 0; i < 10; ++i) yb[i] = S(float(ybd[i]));
+  if (!hand) {
+    for (int it = iters; it >= 0; --it) {
+      S g[kVelIn] = {};
+      for (int j = 0; j < 10; ++j) x[j] = st[it][j];
+      if (it > 0) vjp<kVelIn, 10, 8>(x, yb, g, VelFn<S>{k, block});
+      else vjp<kVelIn, 6, 8>(x, yb, g, WarmFn<S>{k, block});
+      for (int j = 0; j < 10; ++j) yb[j] = j < 6 || it > 0 ? g[j] : yb[j] + g[j];
+      for (int j = 10; j < kVelIn; ++j) xb[j] += g[j];
+    }
+    for (int j = 0; j < 10; ++j) xb[j] = yb[j];
+  } else {
+    const TVelC<S> c = velc_of(x, k, block);
+    TVelC<S> cb = zero_velc<S>();
+    TVel<S> Ab = vel_of(yb), Bb = vel_of(yb + 3);
+    S lb[4] = {yb[6], yb[7], yb[8], yb[9]};
+    for (int it = iters; it > 0; --it)
+      solve_velocity_bar(c, k, st[it] + 6, vel_of(st[it]), vel_of(st[it] + 3), block, Ab, Bb, lb, cb);
+    warm_start_bar(c, k, st[0] + 6, Ab, Bb, lb, cb);
+    put_vel(xb, Ab);
+    put_vel(xb + 3, Bb);
+    for (int i = 0; i < 4; ++i) xb[6 + i] = lb[i];
+    init_bar(k, block, x, cb, xb);
+  }
+  for (int i = 0; i < kVelIn; ++i) out[i] = double(xb[i]);
+}
+
+}  // namespace
+
+extern "C" {
+
+void vc_chain(int hand, int f64, const int* tc, const double* k, int block, int iters, const double* x,
+              const double* yb, double* xb) {
+  if (f64) chain<double>(hand != 0, tc, k, block != 0, iters, x, yb, xb);
+  else chain<float>(hand != 0, tc, k, block != 0, iters, x, yb, xb);
+}
+
+void vc_velocity(int which, int hand, int f64, const int* tc, const double* k, int block, const double* x,
+                 const double* yb, double* xb) {
+  if (f64) velocity<double>(which, hand != 0, tc, k, block != 0, x, yb, xb);
+  else velocity<float>(which, hand != 0, tc, k, block != 0, x, yb, xb);
+}
+
+void vc_position(int hand, int f64, const int* tc, const double* k, const double* x, const double* yb, double* xb) {
+  if (f64) position<double>(hand != 0, tc, k, x, yb, xb);
+  else position<float>(hand != 0, tc, k, x, yb, xb);
+}
+
+}  // extern "C"
