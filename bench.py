@@ -40,10 +40,10 @@ HBM_PEAK_GBS = 8000.0
 # tangent masses, anchors, bias, block matrix and its inverse, impulses; both bodies' velocities
 # read and written). It is the kernel with the largest share of a step's time; its launches are
 # short (a few microseconds), so it is bound by launch and dependent-load latency more than by
-# bandwidth, which the fraction shows. In steps where small islands hold most constraints the
-# velocity iterations run as one launch of k_solve_bins_velocity (all 8 iterations of every bin of
-# islands); its algorithmic bytes are counted the same way (224 B per constraint-iteration), while
-# its HBM traffic is far lower: it reads each constraint and body once and keeps them on chip
+# bandwidth, which the fraction shows. In steps where every island is small the whole solve (set-up,
+# warm start, velocity and position iterations) runs as one launch of k_solve_groups; the bytes are
+# still those of its velocity iterations (224 B per constraint-iteration), so the fraction understates
+# it, while its HBM traffic is far lower: it reads each constraint and body once and keeps them on chip
 # (registers and LDS) across the iterations.
 # k_collide (--roofline-kernel collide): algorithmic HBM bytes of one narrowphase launch (f32/i32 sizes, each read or written once): per
 # candidate pair 120 B (pair, fixture and body records, the two transforms, the previous
@@ -204,8 +204,8 @@ def solver_kernel_name(kernel):
     if b == 0:
         return "k_" + kernel
     if b == n:
-        return "k_solve_bins_" + kernel.split("_")[1]
-    return "k_%s + k_solve_bins_%s (bins in %d of %d steps)" % (kernel, kernel.split("_")[1], b, n)
+        return "k_solve_groups"
+    return "k_%s + k_solve_groups (bins in %d of %d steps)" % (kernel, b, n)
 
 
 def awake_fraction(w, body_defs):

@@ -142,6 +142,7 @@ struct SolverArrays {
   DevArray<int> isl_count, isl_small, isl_start, croot;
   DevArray<int> touch_flag, touch_scan, touch_list;   // compaction of touching contacts
   DevArray<int> k_contact;   // contact index of constraint
+  DevArray<int4> k_rec;      // grouped solve: contact, bodies and island of constraint (sorted_record)
   DevArray<int2> k_bodies;
   DevArray<int4> k_info;     // manifold type, point count, velocity point count, island
   DevArray<float4> vnf;      // normal.x, normal.y, friction, tangent_speed

@@ -622,13 +622,17 @@ struct InitArgs {
   float2* prad;
 };
 
-__global__ void __launch_bounds__(kBlock) k_init_constraints(InitArgs a) {
-  int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= a.n) return;
-  int j = a.order[i];
-  int k = a.list[j];
-  int2 f = a.ab[k];
-  int bA = a.fbody[f.x], bB = a.fbody[f.y];
+// One constraint as the set-up leaves it.
+struct ConstraintRec {
+  int mtype, mcount, vcount;
+  float4 vnf, vm, r[2], vms, K, NM, lam, plp, pgeo, plc;
+  float2 bias, rad;
+};
+// contact k between fixtures f of bodies bA and bB, whose positions and velocities (of the start of
+// the solve) are given
+__device__ inline ConstraintRec constraint_setup(const InitArgs& a, int k, int2 f, int bA, int bB, float4 pA, float4 pB,
+                                                 float4 vA, float4 vB) {
+  ConstraintRec c;
   float4 matA = a.fmat[f.x], matB = a.fmat[f.y];
   // mixing laws, src/b2_contact.rs:29-46
   float friction = sqrtf(matA.x * matB.x);
@@ -642,10 +646,6 @@ __global__ void __launch_bounds__(kBlock) k_init_constraints(InitArgs a) {
   float4 msA = a.bmass[bA], msB = a.bmass[bB];
   float mA = msA.x, iA = msA.y, mB = msB.x, iB = msB.y;
   V2 lcA = v2(msA.z, msA.w), lcB = v2(msB.z, msB.w);
-  float4 pA = a.bpos[bA], pB = a.bpos[bB];
-  float4 vA = a.bvel[bA], vB = a.bvel[bB];
-  int tA = a.btype[bA], tB = a.btype[bB];
-  int island = tA != 0 ? a.parent[bA] : a.parent[bB];
   float4 lam = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
   if (a.warm) {
     lam.x = a.dt_ratio * p0.z;
@@ -666,13 +666,14 @@ __global__ void __launch_bounds__(kBlock) k_init_constraints(InitArgs a) {
   V2 normal = wm.normal;
   V2 cA = v2(pA.x, pA.y), cB = v2(pB.x, pB.y);
   V2 va = v2(vA.x, vA.y), vb = v2(vB.x, vB.y);
-  float4 r[2];
   float nm[2] = {0.0f, 0.0f}, tm[2] = {0.0f, 0.0f}, bias[2] = {0.0f, 0.0f};
-  r[0] = r[1] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-  for (int p = 0; p < mcount; ++p) {
+  c.r[0] = c.r[1] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+#pragma unroll
+  for (int p = 0; p < 2; ++p) {
+    if (p >= mcount) break;
     V2 ra = wm.points[p] - cA;
     V2 rb = wm.points[p] - cB;
-    r[p] = make_float4(ra.x, ra.y, rb.x, rb.y);
+    c.r[p] = make_float4(ra.x, ra.y, rb.x, rb.y);
     float rnA = cross(ra, normal), rnB = cross(rb, normal);
     float kNormal = mA + mB + iA * rnA * rnA + iB * rnB * rnB;
     nm[p] = kNormal > 0.0f ? 1.0f / kNormal : 0.0f;
@@ -686,7 +687,8 @@ __global__ void __launch_bounds__(kBlock) k_init_constraints(InitArgs a) {
   int vcount = mcount;
   float4 K = make_float4(0.0f, 0.0f, 0.0f, 0.0f), NM = K;
   if (mcount == 2 && a.block_solve) {
-    V2 r1a = v2(r[0].x, r[0].y), r1b = v2(r[0].z, r[0].w), r2a = v2(r[1].x, r[1].y), r2b = v2(r[1].z, r[1].w);
+    V2 r1a = v2(c.r[0].x, c.r[0].y), r1b = v2(c.r[0].z, c.r[0].w), r2a = v2(c.r[1].x, c.r[1].y),
+       r2b = v2(c.r[1].z, c.r[1].w);
     float rn1A = cross(r1a, normal), rn1B = cross(r1b, normal);
     float rn2A = cross(r2a, normal), rn2B = cross(r2b, normal);
     float k11 = mA + mB + iA * rn1A * rn1A + iB * rn1B * rn1B;
@@ -702,22 +704,50 @@ __global__ void __launch_bounds__(kBlock) k_init_constraints(InitArgs a) {
       vcount = 1;
     }
   }
+  c.mtype = mtype;
+  c.mcount = mcount;
+  c.vcount = vcount;
+  c.vnf = make_float4(normal.x, normal.y, friction, tangent_speed);
+  c.vm = make_float4(mA, iA, mB, iB);
+  c.vms = make_float4(nm[0], tm[0], nm[1], tm[1]);
+  c.bias = make_float2(bias[0], bias[1]);
+  c.K = K;
+  c.NM = NM;
+  c.lam = lam;
+  c.plp = make_float4(p0.x, p0.y, p1.x, p1.y);
+  c.pgeo = g;
+  c.plc = make_float4(lcA.x, lcA.y, lcB.x, lcB.y);
+  c.rad = make_float2(rA, rB);
+  return c;
+}
+
+// constraint i (colour order) from contact k, into the solver's arrays
+__device__ inline void init_constraint_one(const InitArgs& a, int i, int k) {
+  const int2 f = a.ab[k];
+  const int bA = a.fbody[f.x], bB = a.fbody[f.y];
+  const int tA = a.btype[bA], tB = a.btype[bB];
+  const int island = tA != 0 ? a.parent[bA] : a.parent[bB];
+  const ConstraintRec c = constraint_setup(a, k, f, bA, bB, a.bpos[bA], a.bpos[bB], a.bvel[bA], a.bvel[bB]);
   a.k_contact[i] = k;
   a.k_bodies[i] = make_int2(bA, bB);
-  a.k_info[i] = make_int4(mtype | ((tA == 2) << 8) | ((tB == 2) << 9), mcount, vcount, island);
-  a.vnf[i] = make_float4(normal.x, normal.y, friction, tangent_speed);
-  a.vm[i] = make_float4(mA, iA, mB, iB);
-  a.vr0[i] = r[0];
-  a.vr1[i] = r[1];
-  a.vms[i] = make_float4(nm[0], tm[0], nm[1], tm[1]);
-  a.vbias[i] = make_float2(bias[0], bias[1]);
-  a.K[i] = K;
-  a.NM[i] = NM;
-  a.lam[i] = lam;
-  a.plp[i] = make_float4(p0.x, p0.y, p1.x, p1.y);
-  a.pgeo[i] = g;
-  a.plc[i] = make_float4(lcA.x, lcA.y, lcB.x, lcB.y);
-  a.prad[i] = make_float2(rA, rB);
+  a.k_info[i] = make_int4(c.mtype | ((tA == 2) << 8) | ((tB == 2) << 9), c.mcount, c.vcount, island);
+  a.vnf[i] = c.vnf;
+  a.vm[i] = c.vm;
+  a.vr0[i] = c.r[0];
+  a.vr1[i] = c.r[1];
+  a.vms[i] = c.vms;
+  a.vbias[i] = c.bias;
+  a.K[i] = c.K;
+  a.NM[i] = c.NM;
+  a.lam[i] = c.lam;
+  a.plp[i] = c.plp;
+  a.pgeo[i] = c.pgeo;
+  a.plc[i] = c.plc;
+  a.prad[i] = c.rad;
+}
+__global__ void __launch_bounds__(kBlock) k_init_constraints(InitArgs a) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < a.n) init_constraint_one(a, i, a.list[a.order[i]]);
 }
 
 // ---- velocity passes --------------------------------------------------------------------------
@@ -1138,11 +1168,16 @@ struct IterationEndArgs {
   int* done;
   const int* isl_awake;
 };
-__global__ void __launch_bounds__(kBlock) k_finalize_end(int nb, const int* __restrict__ btype,
-                                                         const float4* __restrict__ pos, const float4* __restrict__ bmass,
-                                                         float4* __restrict__ xf, IslandView iv, IterationEndArgs e) {
+// free_vel (optional): the bodies without constraints are integrated here (deg: constraints per dynamic
+// body; the others were integrated by their group's workgroup)
+__global__ void __launch_bounds__(kBlock) k_finalize_end(int nb, const int* __restrict__ btype, float4* __restrict__ pos,
+                                                         const float4* __restrict__ bmass, float4* __restrict__ xf,
+                                                         IslandView iv, IterationEndArgs e,
+                                                         float4* __restrict__ free_vel, const int* __restrict__ deg,
+                                                         float h) {
   const int b = blockIdx.x * blockDim.x + threadIdx.x;
   if (b >= nb) return;
+  if (free_vel && deg[b] == 0) integrate_position_one(b, btype, pos, free_vel, h, iv);
   if (e.iteration >= 0) iteration_end_one(b, e.iteration, btype, e.parent, e.violated, e.done, e.isl_awake);
   finalize_one(b, btype, pos, bmass, xf, iv);
 }
@@ -1163,9 +1198,9 @@ __global__ void __launch_bounds__(kBlock) k_position_iteration_end(int nb, int i
 // Within each colour the constraints are grouped by world: cw_off[L * nw + w] is the first
 // constraint of world w in launch colour L (an exclusive scan over (colour, world), colour-major,
 // so cw_off[L * nw] is colour L's first constraint and the order stays colour-major). One
-// workgroup then runs all iterations of its world, colour after colour with a workgroup barrier
-// between colours -- the sequence of the per-colour launches restricted to one world, whose
-// constraints touch no other world's bodies, so the results are the same bit for bit.
+// workgroup then runs the whole solve of its world (k_solve_groups below), colour after colour with a
+// workgroup barrier between colours -- the sequence of the per-colour launches restricted to one
+// world, whose constraints touch no other world's bodies, so the results are the same bit for bit.
 static constexpr int kWorldSolveMin = 16;
 
 __device__ inline int constraint_world(int j, const int* __restrict__ list, const int2* __restrict__ ab,
@@ -1182,135 +1217,40 @@ __global__ void __launch_bounds__(kBlock) k_color_world_hist(int n, const int* _
   block_count_keys(g, count);
 }
 
+// What a group's workgroup starts a constraint from, in one load: contact, bodies (with a bit for a
+// dynamic one) and island.
+constexpr int kDynamicBit = 1 << 30;
+__device__ inline int4 sorted_record(int k, int2 b, bool dA, bool dB, int island) {
+  return make_int4(k, b.x | (dA ? kDynamicBit : 0), b.y | (dB ? kDynamicBit : 0), island);
+}
+
 __global__ void __launch_bounds__(kBlock) k_color_world_scatter(int n, const int* __restrict__ state,
                                                                 const int* __restrict__ launch,
                                                                 const int* __restrict__ list, const int2* __restrict__ ab,
                                                                 const int* __restrict__ fworld, int nw,
                                                                 const int* __restrict__ off, int* __restrict__ cursor,
-                                                                int* __restrict__ order, int* __restrict__ inv_order,
+                                                                const int2* __restrict__ bodies,
+                                                                const int* __restrict__ btype,
+                                                                const int* __restrict__ parent,
+                                                                int* __restrict__ k_contact, int4* __restrict__ k_rec,
                                                                 int* __restrict__ pair_colour) {
   const int j = blockIdx.x * blockDim.x + threadIdx.x;
   const int L = j < n && state[j] >= 0 ? launch[state[j] & 0xff] : -1;
   const int g = L >= 0 ? L * nw + constraint_world(j, list, ab, fworld) : -1;
   const int pos = block_place_keys(g, off, cursor);
   if (g >= 0) {
-    order[pos] = j;
-    inv_order[j] = pos;
-    pair_colour[list[j]] = L;
+    const int k = list[j];
+    const int2 b = bodies[j];
+    const int tA = btype[b.x];
+    k_contact[pos] = k;
+    k_rec[pos] = sorted_record(k, b, tA == 2, btype[b.y] == 2, parent[tA != 0 ? b.x : b.y]);
+    pair_colour[k] = L;
   }
 }
 
 __global__ void __launch_bounds__(kBlock) k_clear_ints(int n, int* __restrict__ a) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) a[i] = 0;
-}
-
-// the world of this workgroup and its constraint range per colour (in LDS)
-template <int B>
-__device__ inline int world_ranges(const int* __restrict__ off, int nw, int ncolors, const int* __restrict__ wlist,
-                                   int wbase, int2* rng) {
-  const int w = wlist[wbase + blockIdx.x];
-  for (int c = threadIdx.x; c < ncolors; c += B) rng[c] = make_int2(off[c * nw + w], off[c * nw + w + 1]);
-  __syncthreads();
-  return w;
-}
-
-template <int B>
-__global__ void __launch_bounds__(B) k_solve_worlds_velocity(const int* __restrict__ off, int nw, int ncolors,
-                                                             int iters, int block_solve, VelArgs a,
-                                                             const int* __restrict__ wlist, int wbase) {
-  __shared__ int2 rng[kMaxColors];
-  world_ranges<B>(off, nw, ncolors, wlist, wbase, rng);
-  for (int it = 0; it < iters; ++it)
-    for (int c = 0; c < ncolors; ++c) {
-      const int2 r = rng[c];
-      if (r.x == r.y) continue;  // uniform across the workgroup
-      for (int i = r.x + threadIdx.x; i < r.y; i += B) solve_velocity_one(i, block_solve, a);
-      __syncthreads();
-    }
-}
-
-// position iterations with the islands' early exit: after every iteration but the last (whose
-// end runs with the copy back), the world's island roots are updated as k_position_iteration_end
-// updates all of them
-template <int B>
-__global__ void __launch_bounds__(B) k_solve_worlds_position(const int* __restrict__ off, int nw, int ncolors,
-                                                             int iters, const int* __restrict__ body_off,
-                                                             const int* __restrict__ btype, PosArgs a,
-                                                             IterationEndArgs e, const int* __restrict__ wlist,
-                                                             int wbase) {
-  __shared__ int2 rng[kMaxColors];
-  const int w = world_ranges<B>(off, nw, ncolors, wlist, wbase, rng);
-  const int b0 = body_off[w], b1 = body_off[w + 1];
-  for (int it = 0; it < iters; ++it) {
-    for (int c = 0; c < ncolors; ++c) {
-      const int2 r = rng[c];
-      if (r.x == r.y) continue;
-      for (int i = r.x + threadIdx.x; i < r.y; i += B) solve_position_one(i, true, r.x, a);
-      __syncthreads();
-    }
-    if (it + 1 < iters) {
-      for (int b = b0 + threadIdx.x; b < b1; b += B)
-        iteration_end_one(b, it, btype, e.parent, e.violated, e.done, e.isl_awake);
-      __syncthreads();
-    }
-  }
-}
-
-// one launch per body-count bucket of worlds, with that bucket's threads per world; a timed launch
-// counts its share of the items by its number of worlds
-static void launch_worlds_velocity(World* w, long long items, const int* off, int ncolors, int iters, int block_solve,
-                                   const VelArgs& a) {
-  const int nw = w->n_worlds;
-  const int* wl = w->s.world_order.p;
-  for (int k = 0; k < 3; ++k) {
-    const int n = w->world_bucket_off[k + 1] - w->world_bucket_off[k], wb = w->world_bucket_off[k];
-    if (n == 0) continue;
-    const long long share = items * n / std::max(nw, 1);
-    const int K = B2G_KERNEL_SOLVE_VELOCITY;
-    switch (w->world_threads[k]) {
-      case 64:
-        launch_timed(w, K, share, k_solve_worlds_velocity<64>, dim3(n), dim3(64), off, nw, ncolors, iters, block_solve, a, wl, wb);
-        break;
-      case 128:
-        launch_timed(w, K, share, k_solve_worlds_velocity<128>, dim3(n), dim3(128), off, nw, ncolors, iters, block_solve, a, wl, wb);
-        break;
-      case 512:
-        launch_timed(w, K, share, k_solve_worlds_velocity<512>, dim3(n), dim3(512), off, nw, ncolors, iters, block_solve, a, wl, wb);
-        break;
-      default:
-        launch_timed(w, K, share, k_solve_worlds_velocity<256>, dim3(n), dim3(256), off, nw, ncolors, iters, block_solve, a, wl, wb);
-        break;
-    }
-  }
-}
-
-static void launch_worlds_position(World* w, long long items, const int* off, int ncolors, int iters,
-                                   const PosArgs& a, const IterationEndArgs& e) {
-  const int nw = w->n_worlds;
-  const int* wl = w->s.world_order.p;
-  const int* bo = w->s.world_body_off.p;
-  const int* bt = w->b.type.p;
-  for (int k = 0; k < 3; ++k) {
-    const int n = w->world_bucket_off[k + 1] - w->world_bucket_off[k], wb = w->world_bucket_off[k];
-    if (n == 0) continue;
-    const long long share = items * n / std::max(nw, 1);
-    const int K = B2G_KERNEL_SOLVE_POSITION;
-    switch (w->world_threads[k]) {
-      case 64:
-        launch_timed(w, K, share, k_solve_worlds_position<64>, dim3(n), dim3(64), off, nw, ncolors, iters, bo, bt, a, e, wl, wb);
-        break;
-      case 128:
-        launch_timed(w, K, share, k_solve_worlds_position<128>, dim3(n), dim3(128), off, nw, ncolors, iters, bo, bt, a, e, wl, wb);
-        break;
-      case 512:
-        launch_timed(w, K, share, k_solve_worlds_position<512>, dim3(n), dim3(512), off, nw, ncolors, iters, bo, bt, a, e, wl, wb);
-        break;
-      default:
-        launch_timed(w, K, share, k_solve_worlds_position<256>, dim3(n), dim3(256), off, nw, ncolors, iters, bo, bt, a, e, wl, wb);
-        break;
-    }
-  }
 }
 
 // ---- island solve (island bins) ---------------------------------------------------------------
@@ -1519,14 +1459,21 @@ __global__ void __launch_bounds__(kBlock) k_color_bin_scatter(int n, const int* 
                                                               const int* __restrict__ isl_start, int cap, int nbins,
                                                               const int* __restrict__ off, int* __restrict__ cursor,
                                                               const int* __restrict__ list, int* __restrict__ order,
-                                                              int* __restrict__ inv_order, int* __restrict__ pair_colour) {
+                                                              int* __restrict__ inv_order,
+                                                              const int2* __restrict__ bodies,
+                                                              const int* __restrict__ btype, int* __restrict__ k_contact,
+                                                              int4* __restrict__ k_rec, int* __restrict__ pair_colour) {
   const int j = blockIdx.x * blockDim.x + threadIdx.x;
   const int g = j < n && state[j] >= 0 ? constraint_group(j, state, launch, croot, isl_count, isl_start, cap, nbins) : -1;
   const int pos = block_place_keys(g, off, cursor);
   if (g >= 0) {
+    const int k = list[j];
     order[pos] = j;
     inv_order[j] = pos;
-    pair_colour[list[j]] = g / (nbins + 1);
+    const int2 b = bodies[j];
+    k_contact[pos] = k;
+    k_rec[pos] = sorted_record(k, b, btype[b.x] == 2, btype[b.y] == 2, croot[j]);
+    pair_colour[k] = g / (nbins + 1);
   }
 }
 
@@ -1589,6 +1536,350 @@ static void launch_bins_position(World* w, long long items, int nbins, const int
     default:
       launch_timed(w, K, items, k_solve_bins_position<256>, dim3(nbins), dim3(256), off, ng, ncolors, iters, a);
       break;
+  }
+}
+
+// ---- the whole solve of a group in one workgroup ---------------------------------------------------
+// A group is a bin of islands or a world of a batch: its dynamic bodies are in no other group. One
+// workgroup takes its constraints from the contacts to the end of the position iterations: set-up, warm
+// start, velocity iterations, impulse store, position integration, position iterations with the
+// islands' early exit. Constraint t + q T of the group (in colour order) is thread t's q-th, in registers
+// (the velocity iterations' record, then the position iterations'); the bodies' velocities and positions
+// sit in LDS, read once and written back once. Bins hold at most T constraints (C = 1) and find their
+// bodies through a hash table; a world's bodies are one index range. The operations on a body, and their
+// order, are those of the per-colour launches (the warm start runs colour by colour, which is the order
+// k_warm_start_bodies applies a body's impulses in), so the results are the same bit for bit.
+//
+// A phase (a colour of an iteration) is one constraint's arithmetic between two barriers: 0.7 us of a
+// velocity and 1.5 us of a position iteration, about 300 and 900 instructions a wave issues whether one
+// or 64 of its lanes hold a constraint of the colour. That times colours times iterations bounds it. As
+// separate launches the set-up, warm start, impulse store and integration read and wrote every record
+// once more, and a world's iterations read their records and bodies from memory in every phase.
+// Per step, 65,536 bodies in free fall (17,000 contacts in bins): 72 us in five launches -> 52 us in one;
+// 1024 worlds of 16-1024 bodies: 504 us in nine launches -> 488 us in three; 192 worlds of 64 bodies:
+// 117 us in five -> 84 us in one.
+struct GroupSolve {
+  InitArgs init;
+  const int4* rec;  // sorted constraints (sorted_record)
+  const int* off;  // [colour * ng + group]: first constraint
+  int ng, ncolors, vel_iters, pos_iters;
+  float dt;
+  PosArgs pos;
+  VelArgs vel;
+  const int* btype;
+  IslandView iv;
+  const int* body_off;  // worlds: first body of each
+  const int* wlist;     // worlds: launch order
+  int wbase;
+};
+
+// an entry's integration (integrate_position_one on records in LDS)
+__device__ inline void integrate_pair(float4& p, float4& v, float h) {
+  V2 tr = h * v2(v.x, v.y);
+  if (dot(tr, tr) > kMaxTranslation * kMaxTranslation) {
+    float ratio = kMaxTranslation / len(tr);
+    v.x *= ratio;
+    v.y *= ratio;
+  }
+  float rotation = h * v.z;
+  if (rotation * rotation > kMaxRotation * kMaxRotation) {
+    float ratio = kMaxRotation / fabsf(rotation);
+    v.z *= ratio;
+  }
+  p.x += h * v.x;
+  p.y += h * v.y;
+  p.z += h * v.z;
+}
+
+// A world with more constraints or bodies than the registers and LDS hold: the same sequence on the
+// solver's arrays in memory.
+template <int T>
+__device__ void solve_world_in_memory(const GroupSolve& a, const int2* rng, int b0, int b1) {
+  auto each_colour = [&](auto&& fn) {
+    for (int c = 0; c < a.ncolors; ++c) {
+      const int2 r = rng[c];
+      if (r.x == r.y) continue;  // uniform across the workgroup
+      for (int i = r.x + threadIdx.x; i < r.y; i += T) fn(i, r.x);
+      __syncthreads();
+    }
+  };
+  each_colour([&](int i, int) { init_constraint_one(a.init, i, a.init.k_contact[i]); });
+  if (a.init.warm)
+    each_colour([&](int i, int) {
+      const int2 bd = a.vel.bodies[i];
+      const int4 info = a.vel.info[i];
+#pragma unroll
+      for (int side = 0; side < 2; ++side) {
+        if (!(info.x & (side ? 0x200 : 0x100))) continue;
+        const int b = side ? bd.y : bd.x;
+        const WarmRec r = warm_load(b, i, a.vel);
+        const float4 vb = a.vel.vel[b];
+        V2 v = v2(vb.x, vb.y);
+        float w = vb.z;
+        warm_apply(r, v, w);
+        a.vel.vel[b] = make_float4(v.x, v.y, w, 0.0f);
+      }
+    });
+  for (int it = 0; it < a.vel_iters; ++it)
+    each_colour([&](int i, int) { solve_velocity_one(i, a.init.block_solve, a.vel); });
+  each_colour([&](int i, int) {
+    store_one(i, a.init.k_contact, a.vel.info, a.vel.lam, const_cast<float4*>(a.init.pt0),
+              const_cast<float4*>(a.init.pt1));
+  });
+  for (int b = b0 + threadIdx.x; b < b1; b += T) integrate_position_one(b, a.btype, a.pos.pos, a.vel.vel, a.dt, a.iv);
+  __syncthreads();
+  for (int it = 0; it < a.pos_iters; ++it) {
+    each_colour([&](int i, int first) { solve_position_one(i, true, first, a.pos); });
+    if (it + 1 < a.pos_iters) {
+      for (int b = b0 + threadIdx.x; b < b1; b += T)
+        iteration_end_one(b, it, a.btype, a.iv.parent, a.pos.violated, a.pos.done, a.iv.isl_awake);
+      __syncthreads();
+    }
+  }
+}
+
+// (at least two waves per SIMD: with four constraints per thread the compiler otherwise takes a few
+// registers more than half of the file)
+template <int T, int C, int NB, bool kWorlds>
+__global__ void __launch_bounds__(T, 2) k_solve_groups(GroupSolve a) {
+  constexpr int H = kWorlds ? NB : kBinHashPerThread * T, LG = kWorlds ? 1 : ilog2(H);
+  constexpr int HR = kWorlds ? NB : 2 * T, LGR = kWorlds ? 1 : ilog2(HR);  // a bin has fewer than T islands
+  __shared__ int2 rng[kMaxColors];
+  __shared__ int keys[kWorlds ? 1 : H], rkeys[kWorlds ? 1 : HR];
+  __shared__ float4 bv[H], bp[H];
+  __shared__ int rdone[HR];
+  __shared__ unsigned char rviol[HR], btype[H];
+  const int t = threadIdx.x;
+  const int g = kWorlds ? a.wlist[a.wbase + blockIdx.x] : blockIdx.x;
+  for (int c = t; c < a.ncolors; c += T) rng[c] = make_int2(a.off[c * a.ng + g], a.off[c * a.ng + g + 1]);
+  if (!kWorlds) {
+    for (int e = t; e < H; e += T) keys[e] = -1;
+    for (int e = t; e < HR; e += T) rkeys[e] = -1;
+  }
+  const int b0 = kWorlds ? a.body_off[g] : 0, nbody = kWorlds ? a.body_off[g + 1] - b0 : 0;
+  __syncthreads();
+  if (kWorlds) {
+    int n = 0;
+    for (int c = 0; c < a.ncolors; ++c) n += rng[c].y - rng[c].x;
+    if (n > T * C || nbody > NB) {  // uniform across the workgroup
+      solve_world_in_memory<T>(a, rng, b0, b0 + nbody);
+      return;
+    }
+  }
+  // the thread's constraints, their bodies and islands
+  int i[C], col[C], k[C], sa[C], sb[C], sr[C];
+  int2 f[C], bd[C];
+  bool dA[C], dB[C];
+#pragma unroll
+  for (int q = 0; q < C; ++q) {
+    i[q] = bin_constraint(rng, a.ncolors, t + q * T, &col[q]);
+    k[q] = sa[q] = sb[q] = sr[q] = 0;
+    f[q] = bd[q] = make_int2(0, 0);
+    dA[q] = dB[q] = false;
+    if (i[q] < 0) continue;
+    const int4 rec = a.rec[i[q]];
+    k[q] = rec.x;
+    f[q] = a.init.ab[k[q]];
+    dA[q] = rec.y & kDynamicBit;
+    dB[q] = rec.z & kDynamicBit;
+    bd[q] = make_int2(rec.y & ~kDynamicBit, rec.z & ~kDynamicBit);
+    const int island = rec.w;
+    if (kWorlds) {
+      sa[q] = bd[q].x - b0;
+      sb[q] = bd[q].y - b0;
+      sr[q] = island - b0;
+    } else {
+      sa[q] = bin_slot(keys, LG, bd[q].x);
+      sb[q] = bin_slot(keys, LG, bd[q].y);
+      sr[q] = bin_slot(rkeys, LGR, island);
+    }
+    a.init.k_bodies[i[q]] = bd[q];
+  }
+  __syncthreads();
+  const int ne = kWorlds ? nbody : H;  // table entries
+  auto body_of = [&](int e) { return kWorlds ? b0 + e : keys[e]; };
+  for (int e = t; e < ne; e += T) {
+    const int b = body_of(e);
+    if (b < 0) continue;
+    bv[e] = a.vel.vel[b];
+    bp[e] = a.pos.pos[b];
+    btype[e] = static_cast<unsigned char>(a.btype[b]);
+  }
+  for (int e = t; e < (kWorlds ? nbody : HR); e += T) {
+    const int r = kWorlds ? b0 + e : rkeys[e];
+    if (r < 0) continue;
+    rdone[e] = a.pos.done[r];
+    rviol[e] = a.pos.violated[r] != 0;
+  }
+  __syncthreads();
+  // set-up
+  float4 m[C], nf[C], lam[C], ms[C], r0[C], r1[C], K[C], NM[C];
+  float2 bias[C];
+  int vcount[C];
+#pragma unroll
+  for (int q = 0; q < C; ++q) {
+    vcount[q] = 0;
+    if (i[q] < 0) continue;
+    const ConstraintRec c = constraint_setup(a.init, k[q], f[q], bd[q].x, bd[q].y, bp[sa[q]], bp[sb[q]], bv[sa[q]],
+                                             bv[sb[q]]);
+    m[q] = c.vm;
+    nf[q] = c.vnf;
+    lam[q] = c.lam;
+    ms[q] = c.vms;
+    r0[q] = c.r[0];
+    r1[q] = c.r[1];
+    K[q] = c.K;
+    NM[q] = c.NM;
+    bias[q] = c.bias;
+    vcount[q] = c.vcount;
+    const int island = kWorlds ? b0 + sr[q] : rkeys[sr[q]];
+    a.init.k_info[i[q]] = make_int4(c.mtype | (dA[q] << 8) | (dB[q] << 9), c.mcount, c.vcount, island);
+  }
+  __syncthreads();  // every set-up has read the velocities
+  for (int it = a.init.warm ? -1 : 0; it < a.vel_iters; ++it)  // -1: the warm start
+    for (int c = 0; c < a.ncolors; ++c) {
+      if (rng[c].x == rng[c].y) continue;  // uniform across the workgroup
+#pragma unroll
+      for (int q = 0; q < C; ++q) {
+        if (col[q] != c) continue;
+        float4 vA = bv[sa[q]], vB = bv[sb[q]];
+        if (it < 0) {
+          WarmRec w{m[q], nf[q], lam[q], r0[q], r1[q], 1, vcount[q]};
+          V2 v = v2(vA.x, vA.y);
+          warm_apply(w, v, vA.z);
+          vA = make_float4(v.x, v.y, vA.z, 0.0f);
+          w.side_a = 0;
+          v = v2(vB.x, vB.y);
+          warm_apply(w, v, vB.z);
+          vB = make_float4(v.x, v.y, vB.z, 0.0f);
+        } else {
+          velocity_core(m[q], nf[q], lam[q], ms[q], r0[q], r1[q], vcount[q], bias[q], a.init.block_solve,
+                        [&](float4& k1, float4& k2) {
+                          k1 = K[q];
+                          k2 = NM[q];
+                        },
+                        vA, vB);
+        }
+        if (dA[q]) bv[sa[q]] = vA;
+        if (dB[q]) bv[sb[q]] = vB;
+      }
+      __syncthreads();
+    }
+  // store_impulses, and the position iterations' records
+  float4 lp[C], pg[C], lc[C];
+  float2 rad[C];
+  int type[C], count[C];
+#pragma unroll
+  for (int q = 0; q < C; ++q) {
+    count[q] = 0;
+    if (i[q] < 0) continue;
+    float4* pt0 = const_cast<float4*>(a.init.pt0) + k[q];
+    float4* pt1 = const_cast<float4*>(a.init.pt1) + k[q];
+    const float4 p0 = *pt0, p1 = *pt1;
+    *pt0 = make_float4(p0.x, p0.y, lam[q].x, lam[q].y);
+    if (vcount[q] > 1) *pt1 = make_float4(p1.x, p1.y, lam[q].z, lam[q].w);
+    const float4 mA = a.init.bmass[bd[q].x], mB = a.init.bmass[bd[q].y];
+    const int h = a.init.hdr[k[q]];
+    type[q] = h & 0xff;
+    count[q] = h >> 8;
+    lp[q] = make_float4(p0.x, p0.y, p1.x, p1.y);
+    pg[q] = a.init.geo[k[q]];
+    lc[q] = make_float4(mA.z, mA.w, mB.z, mB.w);
+    rad[q] = make_float2(__int_as_float(a.init.fshape[f[q].x].z), __int_as_float(a.init.fshape[f[q].y].z));
+  }
+  // position integration of the table's bodies (static ones stay; a kinematic body of a bin moves in
+  // every table that holds it, and in memory with the bodies without constraints)
+  for (int e = t; e < ne; e += T) {
+    const int b = body_of(e);
+    if (b < 0 || btype[e] == 0 || a.iv.asleep(b)) continue;
+    float4 p = bp[e], v = bv[e];
+    integrate_pair(p, v, a.dt);
+    bp[e] = p;
+    bv[e] = v;
+  }
+  __syncthreads();
+  for (int it = 0; it < a.pos_iters; ++it) {
+    for (int c = 0; c < a.ncolors; ++c) {
+      if (rng[c].x == rng[c].y) continue;
+#pragma unroll
+      for (int q = 0; q < C; ++q) {
+        if (col[q] != c || rdone[sr[q]] != 0) continue;
+        float4 PA = bp[sa[q]], PB = bp[sb[q]];
+        const float minSep = position_core(type[q], count[q], m[q], lp[q], pg[q], lc[q], rad[q], PA, PB);
+        if (dA[q]) bp[sa[q]] = PA;
+        if (dB[q]) bp[sb[q]] = PB;
+        if (!(minSep >= -3.0f * kLinearSlop)) rviol[sr[q]] = 1;
+      }
+      __syncthreads();
+    }
+    // the end of an iteration, but for the last (which runs with the copy back)
+    if (it + 1 < a.pos_iters) {
+      for (int e = t; e < (kWorlds ? nbody : HR); e += T)
+        if ((kWorlds || rkeys[e] >= 0) && rdone[e] == 0) {
+          if (!rviol[e]) rdone[e] = it + 1;
+          rviol[e] = 0;
+        }
+      __syncthreads();
+    }
+  }
+  for (int e = t; e < ne; e += T) {
+    const int b = body_of(e);
+    // a world's kinematic bodies are in this table only; those of a bin are written with the free bodies
+    if (b < 0 || btype[e] == 0 || (!kWorlds && btype[e] != 2) || a.iv.asleep(b)) continue;
+    a.vel.vel[b] = bv[e];
+    a.pos.pos[b] = bp[e];
+  }
+  for (int e = t; e < (kWorlds ? nbody : HR); e += T) {
+    const int r = kWorlds ? b0 + e : rkeys[e];
+    if (r < 0) continue;
+    if (kWorlds && (btype[e] == 0 || a.iv.parent[r] != r || a.iv.asleep(r))) continue;
+    a.pos.done[r] = rdone[e];
+    a.pos.violated[r] = rviol[e];
+  }
+}
+
+// Bins: one launch; worlds: one per body-count bucket with that bucket's threads per world, whose LDS
+// holds the bucket's bodies (a world of the largest bucket with more than 1088 runs in memory). Four
+// constraints per thread: up to 2048 with 512 threads. The launch is timed as whichever of the solve's
+// kernels is being timed (it holds them all), a bucket's by its number of worlds.
+template <int T, int NB>
+static void launch_world_bucket(World* w, int kernel, long long items, int n, const GroupSolve& a) {
+  launch_timed(w, kernel, items, k_solve_groups<T, 4, NB, true>, dim3(n), dim3(T), a);
+}
+template <int NB>
+static void launch_world_bucket(World* w, int kernel, long long items, int n, int threads, const GroupSolve& a) {
+  switch (threads) {
+    case 64: launch_world_bucket<64, NB>(w, kernel, items, n, a); break;
+    case 128: launch_world_bucket<128, NB>(w, kernel, items, n, a); break;
+    case 512: launch_world_bucket<512, NB>(w, kernel, items, n, a); break;
+    default: launch_world_bucket<256, NB>(w, kernel, items, n, a); break;
+  }
+}
+static void launch_groups(World* w, int nc, bool worlds, GroupSolve a) {
+  const int kt = w->kt.kernel;
+  const int kernel = kt == B2G_KERNEL_SOLVE_POSITION || kt == B2G_KERNEL_WARM_START || kt == B2G_KERNEL_INIT_CONSTRAINTS
+                         ? kt
+                         : B2G_KERNEL_SOLVE_VELOCITY;
+  const long long items = static_cast<long long>(nc) * (kernel == B2G_KERNEL_SOLVE_VELOCITY ? a.vel_iters
+                                                        : kernel == B2G_KERNEL_SOLVE_POSITION ? a.pos_iters : 1);
+  if (!worlds) {
+    const dim3 grid(a.ng - 1);  // (the last group of a colour holds the large islands' constraints: none here)
+    switch (w->bin_threads) {
+      case 64: launch_timed(w, kernel, items, k_solve_groups<64, 1, 1, false>, grid, dim3(64), a); break;
+      case 128: launch_timed(w, kernel, items, k_solve_groups<128, 1, 1, false>, grid, dim3(128), a); break;
+      case 512: launch_timed(w, kernel, items, k_solve_groups<512, 1, 1, false>, grid, dim3(512), a); break;
+      default: launch_timed(w, kernel, items, k_solve_groups<256, 1, 1, false>, grid, dim3(256), a); break;
+    }
+    return;
+  }
+  for (int k = 0; k < 3; ++k) {
+    const int n = w->world_bucket_off[k + 1] - w->world_bucket_off[k];
+    if (n == 0) continue;
+    a.wbase = w->world_bucket_off[k];
+    const long long share = items * n / std::max(w->n_worlds, 1);
+    if (k == 0) launch_world_bucket<64>(w, kernel, share, n, w->world_threads[k], a);
+    else if (k == 1) launch_world_bucket<256>(w, kernel, share, n, w->world_threads[k], a);
+    else launch_world_bucket<1088>(w, kernel, share, n, w->world_threads[k], a);
   }
 }
 
@@ -1711,7 +2002,7 @@ static int reserve_solver(World* w, int nc) {
       (st = s.vms.reserve(n)) || (st = s.vbias.reserve(n)) || (st = s.K.reserve(n)) || (st = s.NM.reserve(n)) ||
       (st = s.lam.reserve(n)) || (st = s.plp.reserve(n)) || (st = s.pgeo.reserve(n)) || (st = s.plc.reserve(n)) ||
       (st = s.prad.reserve(n)) || (st = s.adj.reserve(2 * n)) || (st = s.color_state.reserve(n)) ||
-      (st = s.order.reserve(n)) || (st = s.inv_order.reserve(n)))
+      (st = s.order.reserve(n)) || (st = s.inv_order.reserve(n)) || (st = s.k_rec.reserve(n)))
     return st;
   return B2G_OK;
 }
@@ -1847,6 +2138,34 @@ int phase_solve(World* w, float dt, float dt_ratio, int vel_iters, int pos_iters
   w->solve_groups = bins && n_big == 0 ? nbins + 1 : 0;
   const bool per_world = nc > 0 && want_world && !want_bins && !serial;
   if (per_world) w->solve_groups = w->n_worlds;
+  // every constraint is in a bin or in a world's group: the whole solve runs in k_solve_groups
+  const bool grouped = w->solve_groups > 0;
+  InitArgs init;
+  init.n = nc;
+  init.order = s.order.p;
+  init.list = s.touch_list.p;
+  init.ab = c.ab.p;
+  init.fbody = w->f.body.p;
+  init.fshape = w->f.shape.p;
+  init.fmat = w->f.mat.p;
+  init.btype = w->b.type.p;
+  init.parent = s.parent.p;
+  init.bpos = w->b.pos.p;
+  init.bvel = w->b.vel.p;
+  init.bmass = w->b.mass.p;
+  init.hdr = c.hdr.p;
+  init.geo = c.geo.p;
+  init.pt0 = c.pt0.p;
+  init.pt1 = c.pt1.p;
+  init.dt_ratio = dt_ratio;
+  init.warm = w->warm_starting;
+  init.block_solve = w->block_solve;
+  init.k_contact = s.k_contact.p;
+  init.k_bodies = s.k_bodies.p;  // overwritten in colour order (the unsorted copy is no longer needed)
+  init.k_info = s.k_info.p;
+  init.vnf = s.vnf.p; init.vm = s.vm.p; init.vr0 = s.vr0.p; init.vr1 = s.vr1.p; init.vms = s.vms.p; init.vbias = s.vbias.p;
+  init.K = s.K.p; init.NM = s.NM.p; init.lam = s.lam.p; init.plp = s.plp.p; init.pgeo = s.pgeo.p; init.plc = s.plc.p;
+  init.prad = s.prad.p;
   if (nc > 0) {
     // One launch per non-empty colour, in colour-id order (kept colours can leave gaps).
     // Device copy: launch offsets (kMaxColors + 1, padded with nc), then per colour id its base
@@ -1884,7 +2203,7 @@ int phase_solve(World* w, float dt, float dt_ratio, int vel_iters, int pos_iters
       if ((st = exclusive_scan(w, s.cw_count.p, s.cw_off.p, ncw, s.cw_off.p + ncw))) return st;
       hipLaunchKernelGGL(k_color_bin_scatter, dim3(blocks_for(n_touching, kBlock)), dim3(kBlock), 0, w->stream,
                          n_touching, s.color_state.p, launch, s.croot.p, s.isl_count.p, s.isl_start.p, bin_cap, nbins,
-                         s.cw_off.p, s.cw_cursor.p, s.touch_list.p, s.order.p, s.inv_order.p, c.colour.p);
+                         s.cw_off.p, s.cw_cursor.p, s.touch_list.p, s.order.p, s.inv_order.p, s.k_bodies.p, w->b.type.p, s.k_contact.p, s.k_rec.p, c.colour.p);
     } else if (per_world) {
       // constraints grouped by world inside each colour (see k_color_world_hist)
       const int nw = w->n_worlds, ncw = ncolors * nw;
@@ -1898,42 +2217,17 @@ int phase_solve(World* w, float dt, float dt_ratio, int vel_iters, int pos_iters
       if ((st = exclusive_scan(w, s.cw_count.p, s.cw_off.p, ncw, s.cw_off.p + ncw))) return st;
       hipLaunchKernelGGL(k_color_world_scatter, dim3(blocks_for(n_touching, kBlock)), dim3(kBlock), 0, w->stream,
                          n_touching, s.color_state.p, launch, s.touch_list.p, c.ab.p, w->f.world.p, nw, s.cw_off.p,
-                         s.cw_cursor.p, s.order.p, s.inv_order.p, c.colour.p);
+                         s.cw_cursor.p, s.k_bodies.p, w->b.type.p, s.parent.p, s.k_contact.p, s.k_rec.p, c.colour.p);
     } else {
       hipLaunchKernelGGL(k_color_scatter, dim3(blocks_for(n_touching, kBlock)), dim3(kBlock), 0, w->stream, n_touching,
                          s.color_state.p, s.color_off.p + kMaxColors + 1, s.color_cursor.p, s.order.p, s.inv_order.p,
                          s.touch_list.p, c.colour.p);
     }
-    InitArgs ia;
-    ia.n = nc;
-    ia.order = s.order.p;
-    ia.list = s.touch_list.p;
-    ia.ab = c.ab.p;
-    ia.fbody = w->f.body.p;
-    ia.fshape = w->f.shape.p;
-    ia.fmat = w->f.mat.p;
-    ia.btype = w->b.type.p;
-    ia.parent = s.parent.p;
-    ia.bpos = w->b.pos.p;
-    ia.bvel = w->b.vel.p;
-    ia.bmass = w->b.mass.p;
-    ia.hdr = c.hdr.p;
-    ia.geo = c.geo.p;
-    ia.pt0 = c.pt0.p;
-    ia.pt1 = c.pt1.p;
-    ia.dt_ratio = dt_ratio;
-    ia.warm = w->warm_starting;
-    ia.block_solve = w->block_solve;
-    ia.k_contact = s.k_contact.p;
-    ia.k_bodies = s.k_bodies.p;  // overwritten in colour order (the unsorted copy is no longer needed)
-    ia.k_info = s.k_info.p;
-    ia.vnf = s.vnf.p; ia.vm = s.vm.p; ia.vr0 = s.vr0.p; ia.vr1 = s.vr1.p; ia.vms = s.vms.p; ia.vbias = s.vbias.p;
-    ia.K = s.K.p; ia.NM = s.NM.p; ia.lam = s.lam.p; ia.plp = s.plp.p; ia.pgeo = s.pgeo.p; ia.plc = s.plc.p;
-    ia.prad = s.prad.p;
-    // k_bodies is both read (colouring, done) and rewritten here in sorted order: the init
-    // kernel recomputes bodies from the contact, so the aliasing is safe.
-    launch_timed(w, B2G_KERNEL_INIT_CONSTRAINTS, nc, k_init_constraints, dim3(blocks_for(nc, kBlock)), dim3(kBlock),
-                 ia);
+    // k_bodies is both read (colouring, done) and rewritten here in sorted order: the set-up
+    // recomputes bodies from the contact, so the aliasing is safe.
+    if (!grouped)
+      launch_timed(w, B2G_KERNEL_INIT_CONSTRAINTS, nc, k_init_constraints, dim3(blocks_for(nc, kBlock)), dim3(kBlock),
+                   init);
   }
   w->n_colors = ncolors;
   if (!reuse && ncolors > 0) {
@@ -1950,7 +2244,7 @@ int phase_solve(World* w, float dt, float dt_ratio, int vel_iters, int pos_iters
   // (graph nodes cannot carry the timing events of a timed solve kernel)
   const bool timed_tail = w->kt.kernel == B2G_KERNEL_WARM_START || w->kt.kernel == B2G_KERNEL_SOLVE_VELOCITY ||
                           w->kt.kernel == B2G_KERNEL_SOLVE_POSITION;
-  if (nc > 0 && w->solver_graphs && !timed_tail && !sleepy && w->nj == 0 && !per_world && !bins && !serial) {
+  if (nc > 0 && w->solver_graphs && !timed_tail && !sleepy && w->nj == 0 && !grouped && !bins && !serial) {
     // one graph launch replaces ~(1 + vel_iters + pos_iters) x colours launches
     int maxc = 0;
     for (int col = 0; col < ncolors; ++col) maxc = std::max(maxc, co[col + 1] - co[col]);
@@ -1980,7 +2274,7 @@ int phase_solve(World* w, float dt, float dt_ratio, int vel_iters, int pos_iters
     w->pos_iters_run = pos_iters;
     return B2G_OK;
   }
-  if (nc > 0 && w->warm_starting)
+  if (nc > 0 && w->warm_starting && !grouped)
     launch_timed(w, B2G_KERNEL_WARM_START, nc, k_warm_start_bodies, dim3(blocks_for(nb, kBlock)), dim3(kBlock), nb,
                  w->b.type.p, s.adj_off.p, s.adj.p, s.inv_order.p, va, iv);
   // joints (b2g_joints.hip): initialised after the contacts' warm start, solved before the
@@ -1990,15 +2284,10 @@ int phase_solve(World* w, float dt, float dt_ratio, int vel_iters, int pos_iters
                      w->j.k3.p,    w->b.type.p,   w->b.pos.p,  w->b.vel.p,  w->b.mass.p, iv,
                      s.isl_violated.p, s.isl_done.p, dt, 1.0f / dt, dt_ratio, int(w->warm_starting)};
   if (w->nj > 0) launch_joint_colours(w, 0, ja);
-  if (per_world) {
-    launch_worlds_velocity(w, static_cast<long long>(nc) * vel_iters, s.cw_off.p, ncolors, vel_iters,
-                           int(w->block_solve), va);
-    hipLaunchKernelGGL(k_store_and_integrate, dim3(blocks_for(std::max(nc, nb), kBlock)), dim3(kBlock), 0, w->stream,
-                       nc, s.k_contact.p, s.k_info.p, s.lam.p, c.pt0.p, c.pt1.p, nb, w->b.type.p, w->b.pos.p,
-                       w->b.vel.p, dt, iv);
-    const IterationEndArgs ends{-1, s.parent.p, s.isl_violated.p, s.isl_done.p, iv.isl_awake};
-    if (pos_iters > 0)
-      launch_worlds_position(w, static_cast<long long>(nc) * pos_iters, s.cw_off.p, ncolors, pos_iters, pa, ends);
+  if (grouped) {
+    const GroupSolve ga{init, s.k_rec.p, s.cw_off.p, w->solve_groups, ncolors, vel_iters, pos_iters, dt, pa, va, w->b.type.p, iv,
+                        s.world_body_off.p, s.world_order.p, 0};
+    launch_groups(w, nc, per_world, ga);
     w->pos_iters_run = pos_iters;
   } else {
   // Per-colour launches: of all constraints, or with island bins of the large islands' (the last
@@ -2073,7 +2362,8 @@ int phase_solve(World* w, float dt, float dt_ratio, int vel_iters, int pos_iters
   }
   const IterationEndArgs last_end{pos_iters - 1, s.parent.p, s.isl_violated.p, s.isl_done.p, iv.isl_awake};
   hipLaunchKernelGGL(k_finalize_end, dim3(blocks_for(nb, kBlock)), dim3(kBlock), 0, w->stream, nb, w->b.type.p,
-                     w->b.pos.p, w->b.mass.p, w->b.xf.p, iv, last_end);
+                     w->b.pos.p, w->b.mass.p, w->b.xf.p, iv, last_end, grouped && !per_world ? w->b.vel.p : nullptr,
+                     s.deg.p, dt);
   if (w->allow_sleep) {
     hipLaunchKernelGGL(k_sleep_time, dim3(blocks_for(nb, kBlock)), dim3(kBlock), 0, w->stream, nb, w->b.type.p,
                        w->b.auto_sleep.p, w->b.vel.p, w->b.sleep_time.p, iv, s.isl_restless.p, dt);
