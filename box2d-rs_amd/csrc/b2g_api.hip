@@ -605,7 +605,8 @@ int b2g_world_create(float gx, float gy, b2g_world** out) {
   w->device = dev;
   if (hipStreamCreateWithFlags(&w->stream, hipStreamNonBlocking) != hipSuccess ||
       w->counters.reserve(4 + 128 + 2) != B2G_OK ||
-      hipHostMalloc(reinterpret_cast<void**>(&w->h_counters), kPinnedInts * sizeof(int), hipHostMallocDefault) !=
+      hipHostMalloc(reinterpret_cast<void**>(&w->h_counters), kPinnedInts * sizeof(int),
+                    hipHostMallocMapped | hipHostMallocCoherent) !=
           hipSuccess) {
     set_error("world allocation failed");
     delete h;
@@ -655,7 +656,7 @@ int b2g_world_destroy(b2g_world* h) {
   BroadphaseArrays& bp = w->bp;
   rel(bp.keys); rel(bp.keys_alt); rel(bp.vals); rel(bp.vals_alt); rel(bp.hist); rel(bp.seg); rel(bp.nodes); rel(bp.nodes4);
   rel(bp.leafrec); rel(bp.count); rel(bp.slots); rel(bp.bounds); rel(bp.scan_tmp); rel(bp.scan_state); rel(bp.scan_ctl); bp.scan_epoch = 0; bp.scan_ctl_ready = false;
-  rel(w->counters);
+  rel(w->counters); rel(w->small_bail);
   if (w->h_counters) (void)hipHostFree(w->h_counters);
   for (int i = 0; i < 8; ++i)
     if (w->ev[i]) (void)hipEventDestroy(w->ev[i]);
@@ -751,7 +752,15 @@ int b2g_world_step(b2g_world* h, float dt, int32_t vi, int32_t pi) {
   if (taping && (st = tape_after_collide(w))) return st;
   (void)hipEventRecord(w->ev[1], w->stream);
   const float dt_ratio = w->inv_dt0 * dt;
-  if (w->step_complete) {
+  bool small = false;
+  if (w->small_holdoff > 0) --w->small_holdoff;
+  if (w->step_complete && dt > 0.0f && small_step_fits(w)) {
+    if ((st = small_step(w, dt, dt_ratio, vi, pi, &small))) return st;
+    if (small) w->inv_dt0 = 1.0f / dt;
+  }
+  if (small) {
+    (void)hipEventRecord(w->ev[2], w->stream);
+  } else if (w->step_complete) {
     if ((st = run_phase(w, B2G_PHASE_SOLVE, dt, vi, pi))) return st;
     if (taping && (st = tape_after_solve(w, dt, dt_ratio, vi, pi))) return st;
     (void)hipEventRecord(w->ev[2], w->stream);

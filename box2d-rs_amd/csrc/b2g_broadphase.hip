@@ -24,21 +24,30 @@ namespace b2g {
 static constexpr int kBlock = 256;
 
 // ---- fixture synchronisation --------------------------------------------------------------
-__global__ void __launch_bounds__(kBlock) k_synchronize(int np, const int* __restrict__ fbody,
-                                                        const ShapeV* __restrict__ shapes,
-                                                        const int* __restrict__ btype, const float4* __restrict__ pos0,
-                                                        const float4* __restrict__ bmass, const float4* __restrict__ bxf,
-                                                        float4* __restrict__ faabb, float4* __restrict__ ffat,
-                                                        int* __restrict__ moved, IslandView iv,
-                                                        int* __restrict__ any_moved) {
-  int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= np) return;
-  int b = fbody[i];
+struct SyncArgs {
+  const int* fbody;
+  const ShapeV* shapes;
+  const int* btype;
+  const float4 *pos0, *bmass, *bxf;
+  float4 *faabb, *ffat;
+  int* moved;
+  IslandView iv;
+};
+__device__ inline void synchronize_one(int i, const SyncArgs& a, int* any_moved) {
+  int b = a.fbody[i];
   // only bodies of this step's islands are synchronised (src/private/dynamics/b2_world.rs:482-500)
-  if (btype[b] == 0 || iv.asleep(b)) { moved[i] = 0; return; }
-  if (!sync_proxy(i, b, shapes[i], pos0, bmass, bxf, faabb, ffat)) { moved[i] = 0; return; }
-  moved[i] = 1;
+  if (a.btype[b] == 0 || a.iv.asleep(b)) { a.moved[i] = 0; return; }
+  if (!sync_proxy(i, b, a.shapes[i], a.pos0, a.bmass, a.bxf, a.faabb, a.ffat)) { a.moved[i] = 0; return; }
+  a.moved[i] = 1;
   if (any_moved) *any_moved = 1;  // every writer stores 1
+}
+__global__ void __launch_bounds__(kBlock) k_synchronize(int np, SyncArgs a, int* __restrict__ any_moved) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < np) synchronize_one(i, a, any_moved);
+}
+static SyncArgs sync_args(World* w, IslandView iv) {
+  return SyncArgs{w->f.body.p, w->f.shapev.p, w->b.type.p, w->b.pos0.p, w->b.mass.p, w->b.xf.p,
+                  w->f.aabb.p, w->f.fat.p,    w->f.moved.p, iv};
 }
 
 // ---- scene bounds and Morton codes ---------------------------------------------------------
@@ -94,6 +103,27 @@ __device__ inline unsigned spread15(unsigned x) {
   return x;
 }
 
+// bits per axis of the Morton codes: the world's number takes the bits above them. 12 bits per axis
+// (4096 cells across the scene's extent, finer than any body on the scenes here; equal keys keep proxy
+// order), fewer for many worlds, so one world sorts in three 8-bit passes
+static int world_bits(const World* w) {
+  int wbits = 0;
+  while ((1 << wbits) < w->n_worlds) ++wbits;
+  return wbits;
+}
+static int morton_bits(const World* w) { return std::min(12, (32 - world_bits(w)) / 2); }
+
+// code of a box's centre in the extent [lx, hx] x [ly, hy]
+__device__ inline unsigned morton_code(float4 a, float lx, float ly, float hx, float hy, int mbits) {
+  const float cells = float((1u << mbits) - 1u);
+  float sx = hx > lx ? cells / (hx - lx) : 0.0f;
+  float sy = hy > ly ? cells / (hy - ly) : 0.0f;
+  float cx = 0.5f * (a.x + a.z), cy = 0.5f * (a.y + a.w);
+  unsigned ux = unsigned(fminf(fmaxf((cx - lx) * sx, 0.0f), cells));
+  unsigned uy = unsigned(fminf(fmaxf((cy - ly) * sy, 0.0f), cells));
+  return spread15(ux) | (spread15(uy) << 1);
+}
+
 // key = world id in the high bits, then a Morton code of `mbits` bits per axis of the fat-AABB
 // centre; sorting by it groups each world's proxies and orders them along a Z curve
 __global__ void __launch_bounds__(kBlock) k_morton(int n, const int* __restrict__ list, const float4* __restrict__ fat,
@@ -109,14 +139,7 @@ __global__ void __launch_bounds__(kBlock) k_morton(int n, const int* __restrict_
   int k = blockIdx.x * blockDim.x + threadIdx.x;
   if (k >= n) return;
   const int i = list[k];
-  const float cells = float((1u << mbits) - 1u);
-  float sx = hx > lx ? cells / (hx - lx) : 0.0f;
-  float sy = hy > ly ? cells / (hy - ly) : 0.0f;
-  float4 a = fat[i];
-  float cx = 0.5f * (a.x + a.z), cy = 0.5f * (a.y + a.w);
-  unsigned ux = unsigned(fminf(fmaxf((cx - lx) * sx, 0.0f), cells));
-  unsigned uy = unsigned(fminf(fmaxf((cy - ly) * sy, 0.0f), cells));
-  unsigned code = spread15(ux) | (spread15(uy) << 1);
+  const unsigned code = morton_code(fat[i], lx, ly, hx, hy, mbits);
   // indexed by list position: the sort runs over the n listed proxies
   keys[k] = (unsigned(world[i]) << (2 * mbits)) | code;
   vals[k] = unsigned(i);
@@ -196,9 +219,10 @@ __global__ void __launch_bounds__(kBlock) k_seg_reduce(Levels lv, int L0, const 
   }
 }
 
-__device__ inline int lbvh_delta(const unsigned* __restrict__ keys, int n, int i, int j) {
+template <class K>
+__device__ inline int lbvh_delta(const K& keys, int n, int i, int j) {
   if (j < 0 || j >= n) return -1;
-  unsigned a = keys[i], b = keys[j];
+  const unsigned a = keys[i], b = keys[j];
   if (a == b) return 32 + __clz(unsigned(i) ^ unsigned(j));
   return __clz(a ^ b);
 }
@@ -208,7 +232,7 @@ __device__ inline void box_union(float4& r, float4 b) {
 }
 
 // union of sorted leaves [a, b): bottom-up segment-tree query
-__device__ inline float4 seg_range(const float4* __restrict__ seg, const Levels& lv, int a, int b) {
+__device__ inline float4 seg_range(const float4* seg, const Levels& lv, int a, int b) {
   float4 r = make_float4(kMaxFloat, kMaxFloat, -kMaxFloat, -kMaxFloat);
   for (int L = 0; a < b; ++L) {
     if (a & 1) box_union(r, seg[lv.off[L] + a++]);
@@ -219,12 +243,9 @@ __device__ inline float4 seg_range(const float4* __restrict__ seg, const Levels&
   return r;
 }
 
-// Karras 2012 internal node i: split and children, then each child's box (a leaf's own box,
-// or a segment-tree query over the child's leaf range) and world range
-__global__ void __launch_bounds__(kBlock) k_lbvh_build(int n, const unsigned* __restrict__ keys, int wshift, Levels lv,
-                                                       const float4* __restrict__ seg, BvhNode* __restrict__ nodes) {
-  int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n - 1) return;
+// Karras 2012 internal node i: its range of sorted leaves [lo, hi] and its split gamma
+template <class K>
+__device__ inline void lbvh_node(const K& keys, int n, int i, int& lo, int& hi, int& gamma) {
   int d = (lbvh_delta(keys, n, i, i + 1) - lbvh_delta(keys, n, i, i - 1)) >= 0 ? 1 : -1;
   int dmin = lbvh_delta(keys, n, i, i - d);
   int lmax = 2;
@@ -240,8 +261,19 @@ __global__ void __launch_bounds__(kBlock) k_lbvh_build(int n, const unsigned* __
     t = (t + 1) >> 1;
     if (lbvh_delta(keys, n, i, i + (s + t) * d) > dnode) s += t;
   } while (t > 1);
-  int gamma = i + s * d + (d < 0 ? -1 : 0);
-  int lo = i < j ? i : j, hi = i < j ? j : i;
+  gamma = i + s * d + (d < 0 ? -1 : 0);
+  lo = i < j ? i : j;
+  hi = i < j ? j : i;
+}
+
+// internal node i: split and children, then each child's box (a leaf's own box, or a segment-tree
+// query over the child's leaf range) and world range
+__global__ void __launch_bounds__(kBlock) k_lbvh_build(int n, const unsigned* __restrict__ keys, int wshift, Levels lv,
+                                                       const float4* __restrict__ seg, BvhNode* __restrict__ nodes) {
+  int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n - 1) return;
+  int lo, hi, gamma;
+  lbvh_node(keys, n, i, lo, hi, gamma);
   const bool left_leaf = lo == gamma, right_leaf = hi == gamma + 1;
   BvhNode nd;
   nd.box[0] = left_leaf ? seg[gamma] : seg_range(seg, lv, lo, gamma + 1);
@@ -347,7 +379,9 @@ template <bool OVERFLOW_PASS>
 __global__ void __launch_bounds__(kTravBlock) k_traverse(int nq, const float4* __restrict__ fat, TreeView tv,
                                                          PairFilter pf, int* __restrict__ count,
                                                          int* __restrict__ slots, const int* __restrict__ off,
-                                                         int2* __restrict__ pairs, int* __restrict__ flags) {
+                                                         int2* __restrict__ pairs, int* __restrict__ flags,
+                                                         const int* __restrict__ skip) {
+  if (skip && *skip) return;
   __shared__ int stack[kStack][kTravQueries];
   const int k = (blockIdx.x * blockDim.x + threadIdx.x) / kTravLanes;
   const int g = threadIdx.x / kTravLanes;  // the query's stack column (and lane group of the wave)
@@ -495,12 +529,7 @@ static int find_pairs(World* w, const float4* fat, int np, ContactArrays& dst, i
   float4* partial = bp.bounds.p + 1;
   const int* scan_ctl = static_cast<const int*>(bp.scan_ctl.p);
   if (nt == 0) hipLaunchKernelGGL(k_pair_flags_init, dim3(1), dim3(1), 0, w->stream, flags, scan_ctl);
-  // world bits above Morton bits: 12 bits per axis (4096 cells across the scene's extent, finer
-  // than any body on the scenes here; equal keys keep proxy order), fewer for many worlds, so one
-  // world sorts in three 8-bit passes
-  int wbits = 0;
-  while ((1 << wbits) < w->n_worlds) ++wbits;
-  const int mbits = std::min(12, (32 - wbits) / 2);
+  const int wbits = world_bits(w), mbits = morton_bits(w);
   const int key_bits = wbits + 2 * mbits;
   const bool nc = w->n_nocollide > 0;
   const LeafInputs li{w->f.body.p, w->b.type.p, w->f.filter.p, w->f.shape.p, nc ? w->j.nc_flag.p : nullptr};
@@ -530,7 +559,7 @@ static int find_pairs(World* w, const float4* fat, int np, ContactArrays& dst, i
   if (nt > 0) {
     launch_timed(w, B2G_KERNEL_TRAVERSE, nt, k_traverse<false>, dim3(blocks_for(nt * kTravLanes, kTravBlock)),
                  dim3(kTravBlock),
-                 nt, fat, tv, pf, bp.count.p, bp.slots.p, nullptr, nullptr, flags);
+                 nt, fat, tv, pf, bp.count.p, bp.slots.p, nullptr, nullptr, flags, nullptr);
   }
   // the pair total also lands beside the flags (flags[3]), so one read-back brings both
   if ((st = exclusive_scan(w, bp.count.p, dst.off.p, np, dst.off.p + np, flags + 3))) return st;
@@ -556,7 +585,7 @@ static int find_pairs(World* w, const float4* fat, int np, ContactArrays& dst, i
                        bp.leafrec.p, bp.count.p, bp.slots.p, dst.off.p, dst.pair.p);
   if (h[2] > 0)
     hipLaunchKernelGGL(k_traverse<true>, dim3(blocks_for(nt * kTravLanes, kTravBlock)), dim3(kTravBlock), 0, w->stream, nt, fat,
-                       tv, pf, bp.count.p, bp.slots.p, dst.off.p, dst.pair.p, flags);
+                       tv, pf, bp.count.p, bp.slots.p, dst.off.p, dst.pair.p, flags, nullptr);
   B2G_HIP(hipGetLastError());
   *npairs = total;
   return B2G_OK;
@@ -574,9 +603,8 @@ static int reserve_contacts(World* w, ContactArrays& c, int pairs) {
 
 int phase_synchronize_view(World* w, IslandView iv, int* any_moved) {
   if (w->np == 0) return B2G_OK;
-  hipLaunchKernelGGL(k_synchronize, dim3(blocks_for(w->np, kBlock)), dim3(kBlock), 0, w->stream, w->np, w->f.body.p,
-                     w->f.shapev.p, w->b.type.p, w->b.pos0.p, w->b.mass.p, w->b.xf.p, w->f.aabb.p,
-                     w->f.fat.p, w->f.moved.p, iv, any_moved);
+  hipLaunchKernelGGL(k_synchronize, dim3(blocks_for(w->np, kBlock)), dim3(kBlock), 0, w->stream, w->np,
+                     sync_args(w, iv), any_moved);
   B2G_HIP(hipGetLastError());
   return B2G_OK;
 }
@@ -589,6 +617,11 @@ int phase_synchronize(World* w) {
 // New contact set from the current fat AABBs; becomes the current set, the old one is kept
 // (its manifolds feed warm starting).
 int phase_broadphase(World* w) {
+  if (small_find_fits(w)) return small_find(w, false, IslandView{nullptr, nullptr}, nullptr);
+  return phase_broadphase_general(w);
+}
+
+int phase_broadphase_general(World* w) {
   int next = 1 - w->cur;
   ContactArrays& dst = w->c[next];
   ContactArrays& old = w->c[w->cur];
@@ -642,6 +675,309 @@ int broadphase_pairs_for(World* w, const float* fat_host, int64_t cap, int32_t* 
   tmp.off.release();
   fat.release();
   return st;
+}
+
+// ---- small worlds -------------------------------------------------------------------------------
+// find_new_contacts of a single world with at most kSmallTree proxies in the tree and kSmallProxies in
+// all: one workgroup synchronises the proxies, sorts them (by the same Morton key, then by proxy, which is
+// the order the stable radix sort leaves), and builds the same tree in LDS; the walk is the grid's; one
+// workgroup turns its counts into the pair list with predecessors. Three launches and no read-back
+// in between, where the launches above are seventeen and each costs 3 us of host time.
+constexpr int kSmallBlock = 1024;
+
+struct SmallFind {
+  int np, nt, mbits;
+  int sync;         // synchronise the proxies first
+  const int* bail;  // set: the solve before did nothing, and neither does this
+  SyncArgs s;
+  const int* list;  // proxies in the tree
+  Levels lv;
+  LeafInputs li;
+  int4* leafrec;
+  Bvh4Node* nodes;
+  int* flags;
+  const int* scan_ctl;
+  // pairs
+  int* count;
+  const int* slots;
+  int* off;
+  int2* pairs;
+  int cap;  // pairs the new set's arrays hold
+  int old_np;
+  const int* old_off;
+  const int2* old_pairs;
+  int* old_index;
+  int* colour;
+  int* host;  // pinned: [0] published, [1..3] flags, [4] pairs
+  int epoch;
+};
+
+struct SmallTree {
+  unsigned long long key[kSmallTree];  // Morton code << 32 | proxy
+  float4 seg[2 * kSmallTree + 32];
+  unsigned short lo[kSmallTree], hi[kSmallTree], split[kSmallTree];
+};
+struct SmallKeys {  // the sorted codes as lbvh_delta reads them
+  const unsigned long long* key;
+  __device__ unsigned operator[](int i) const { return static_cast<unsigned>(key[i] >> 32); }
+};
+
+__global__ void __launch_bounds__(kSmallBlock) k_small_build(SmallFind a) {
+  __shared__ SmallTree s;
+  __shared__ float red[4][kSmallBlock / 64];
+  const int t = threadIdx.x, lane = t & 63, wid = t >> 6;
+  if (a.bail && *a.bail) return;
+  if (t == 0) pair_flags_init(a.flags, a.scan_ctl);
+  if (a.sync)
+    for (int i = t; i < a.np; i += kSmallBlock) synchronize_one(i, a.s, nullptr);
+  __syncthreads();
+  // bounds of the fat-AABB centres, then the codes (k_bounds and k_morton)
+  float lx = kMaxFloat, ly = kMaxFloat, hx = -kMaxFloat, hy = -kMaxFloat;
+  for (int i = t; i < a.nt; i += kSmallBlock) {
+    const float4 f = a.s.ffat[a.list[i]];
+    const float cx = 0.5f * (f.x + f.z), cy = 0.5f * (f.y + f.w);
+    lx = fminf(lx, cx); ly = fminf(ly, cy); hx = fmaxf(hx, cx); hy = fmaxf(hy, cy);
+  }
+  for (int d = 32; d >= 1; d >>= 1) {
+    lx = fminf(lx, __shfl_xor(lx, d, 64));
+    ly = fminf(ly, __shfl_xor(ly, d, 64));
+    hx = fmaxf(hx, __shfl_xor(hx, d, 64));
+    hy = fmaxf(hy, __shfl_xor(hy, d, 64));
+  }
+  if (lane == 0) { red[0][wid] = lx; red[1][wid] = ly; red[2][wid] = hx; red[3][wid] = hy; }
+  __syncthreads();
+  for (int w = 0; w < kSmallBlock / 64; ++w) {
+    lx = fminf(lx, red[0][w]); ly = fminf(ly, red[1][w]); hx = fmaxf(hx, red[2][w]); hy = fmaxf(hy, red[3][w]);
+  }
+  int m = 64;  // elements sorted: a power of two
+  while (m < a.nt) m <<= 1;
+  for (int i = t; i < m; i += kSmallBlock) {
+    unsigned long long key = ~0ull;
+    if (i < a.nt) {
+      const int p = a.list[i];
+      key = (static_cast<unsigned long long>(morton_code(a.s.ffat[p], lx, ly, hx, hy, a.mbits)) << 32) | unsigned(p);
+    }
+    s.key[i] = key;
+  }
+  __syncthreads();
+  for (int size = 2; size <= m; size <<= 1)
+    for (int step = size >> 1; step > 0; step >>= 1) {
+      for (int i = t; i < m / 2; i += kSmallBlock) {
+        const int lo = 2 * i - (i & (step - 1)), hi = lo + step;
+        const unsigned long long x = s.key[lo], y = s.key[hi];
+        if ((x > y) == ((lo & size) == 0)) {
+          s.key[lo] = y;
+          s.key[hi] = x;
+        }
+      }
+      __syncthreads();
+    }
+  // leaf boxes and records, then the segment tree level by level
+  for (int i = t; i < a.nt; i += kSmallBlock) {
+    const int p = static_cast<int>(s.key[i] & 0xffffffffu);
+    s.seg[i] = a.s.ffat[p];
+    a.leafrec[i] = leaf_record(p, a.li);
+  }
+  __syncthreads();
+  for (int L = 1; L < a.lv.count; ++L) {
+    const int below = a.lv.size[L - 1];
+    for (int i = t; i < a.lv.size[L]; i += kSmallBlock) {
+      float4 r = s.seg[a.lv.off[L - 1] + 2 * i];
+      box_union(r, 2 * i + 1 < below ? s.seg[a.lv.off[L - 1] + 2 * i + 1]
+                                     : make_float4(kMaxFloat, kMaxFloat, -kMaxFloat, -kMaxFloat));
+      s.seg[a.lv.off[L] + i] = r;
+    }
+    __syncthreads();
+  }
+  const SmallKeys keys{s.key};
+  for (int i = t; i < a.nt - 1; i += kSmallBlock) {
+    int lo, hi, gamma;
+    lbvh_node(keys, a.nt, i, lo, hi, gamma);
+    s.lo[i] = static_cast<unsigned short>(lo);
+    s.hi[i] = static_cast<unsigned short>(hi);
+    s.split[i] = static_cast<unsigned short>(gamma);
+  }
+  __syncthreads();
+  // the 4-wide nodes (k_lbvh_build and k_bvh4_collapse): slots of node i are its children, an internal
+  // child replaced by its own two
+  for (int i = t; i < a.nt - 1; i += kSmallBlock) {
+    Bvh4Node out;
+    auto put = [&](int slot, int lo, int hi, int link) {
+      out.box[slot] = link < 0 ? s.seg[~link] : seg_range(s.seg, a.lv, lo, hi + 1);
+      out.link[slot] = link;
+      out.last[slot] = hi;
+      out.wlo[slot] = out.whi[slot] = 0;  // one world
+    };
+    const int g = s.split[i];
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+      const int lo = c ? g + 1 : s.lo[i], hi = c ? s.hi[i] : g, node = g + c;
+      if (lo == hi) {
+        put(2 * c, lo, hi, ~node);
+        out.box[2 * c + 1] = make_float4(kMaxFloat, kMaxFloat, -kMaxFloat, -kMaxFloat);
+        out.link[2 * c + 1] = 0;
+        out.last[2 * c + 1] = -1;
+        out.wlo[2 * c + 1] = 1;
+        out.whi[2 * c + 1] = 0;
+      } else {
+        const int gc = s.split[node];
+        put(2 * c, lo, gc, lo == gc ? ~gc : gc);
+        put(2 * c + 1, gc + 1, hi, hi == gc + 1 ? ~(gc + 1) : gc + 1);
+      }
+    }
+    a.nodes[i] = out;
+  }
+}
+
+// The pair counts' scan, and, unless the host has to step in (a walk that overflowed its stack or its
+// slots, more pairs than the arrays hold), the pairs with their predecessors.
+__global__ void __launch_bounds__(kSmallBlock) k_small_pairs(SmallFind a) {
+  __shared__ int wsum[kSmallBlock / 64];
+  __shared__ int ok;
+  const int t = threadIdx.x, lane = t & 63, wid = t >> 6;
+  const bool idle = a.bail && *a.bail;
+  int total = 0;
+  if (!idle) {
+    const int chunk = (a.np + kSmallBlock - 1) / kSmallBlock, i0 = min(a.np, t * chunk), i1 = min(a.np, i0 + chunk);
+    int sum = 0;
+    for (int i = i0; i < i1; ++i) sum += a.count[i];
+    int inc = sum;
+    for (int d = 1; d < 64; d <<= 1) {
+      const int y = __shfl_up(inc, d, 64);
+      if (lane >= d) inc += y;
+    }
+    if (lane == 63) wsum[wid] = inc;
+    __syncthreads();
+    int ex = inc - sum;
+    for (int w = 0; w < kSmallBlock / 64; ++w) {
+      if (w < wid) ex += wsum[w];
+      total += wsum[w];
+    }
+    for (int i = i0; i < i1; ++i) {
+      const int c = a.count[i];
+      a.off[i] = ex;
+      ex += c;
+    }
+    if (t == 0) {
+      a.off[a.np] = total;
+      ok = a.flags[0] == 0 && a.flags[1] == 0 && total <= a.cap;
+    }
+    __syncthreads();
+    if (ok) {
+      for (int k = t; k < a.nt; k += kSmallBlock) {
+        const int q = a.leafrec[k].x, c = a.count[q], o = a.off[q];
+        for (int j = 0; j < c; ++j) a.pairs[o + j] = make_int2(q, a.slots[size_t(j) * a.nt + k]);
+      }
+      __syncthreads();
+      for (int k = t; k < total; k += kSmallBlock) {
+        const int2 pr = a.pairs[k];
+        int found = find_in_segment(pr.x, pr.y, a.old_np, a.old_off, a.old_pairs);
+        if (found < 0) found = find_in_segment(pr.y, pr.x, a.old_np, a.old_off, a.old_pairs);
+        a.old_index[k] = found;
+        a.colour[k] = -1;
+      }
+    }
+  }
+  if (t == 0) {
+    a.host[1] = idle ? 0 : a.flags[0];
+    a.host[2] = idle ? 0 : a.flags[1];
+    a.host[3] = idle ? 0 : a.flags[2];
+    a.host[4] = total;
+    __threadfence_system();
+    __hip_atomic_store(a.host, a.epoch, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+  }
+}
+
+bool small_find_fits(const World* w) {
+  return w->n_worlds == 1 && w->n_tree > 0 && w->n_tree <= kSmallTree && w->np <= kSmallProxies && !w->dirty &&
+         w->kt.kernel == B2G_KERNEL_NONE;
+}
+
+// phase_synchronize (sync) and phase_broadphase for a world that small_find_fits accepts; with *bail set
+// on the device the kernels do nothing and the new set is empty (the caller then takes the step back)
+int small_find(World* w, bool sync, IslandView iv, const int* bail) {
+  BroadphaseArrays& bp = w->bp;
+  const int next = 1 - w->cur, np = w->np, nt = w->n_tree;
+  ContactArrays& dst = w->c[next];
+  ContactArrays& old = w->c[w->cur];
+  int st;
+  SmallFind a;
+  a.lv.count = 0;
+  int total_nodes = 0;
+  for (int sz = nt;; sz = (sz + 1) / 2) {
+    a.lv.size[a.lv.count] = sz;
+    a.lv.off[a.lv.count] = total_nodes;
+    total_nodes += sz;
+    ++a.lv.count;
+    if (sz <= 1) break;
+  }
+  static_assert(sizeof(SmallTree) + 1024 <= 160 * 1024, "LDS of a workgroup");
+  if ((st = bp.nodes4.reserve(nt)) || (st = bp.leafrec.reserve(nt)) || (st = bp.count.reserve(np + 1)) ||
+      (st = bp.slots.reserve(size_t(np) * kSlots)) || (st = dst.off.reserve(np + 1)) ||
+      (st = bp.bounds.reserve(1 + kBoundsBlocks)) || (st = reserve_contacts(w, dst, 0)))
+    return st;
+  const bool nc = w->n_nocollide > 0;
+  a.np = np;
+  a.nt = nt;
+  a.mbits = morton_bits(w);
+  a.sync = sync;
+  a.bail = bail;
+  a.s = sync_args(w, iv);
+  a.list = w->f.tree_list.p;
+  a.li = LeafInputs{w->f.body.p, w->b.type.p, w->f.filter.p, w->f.shape.p, nc ? w->j.nc_flag.p : nullptr};
+  a.leafrec = bp.leafrec.p;
+  a.nodes = bp.nodes4.p;
+  a.flags = reinterpret_cast<int*>(bp.bounds.p);
+  a.scan_ctl = static_cast<const int*>(bp.scan_ctl.p);
+  a.count = bp.count.p;
+  a.slots = bp.slots.p;
+  a.off = dst.off.p;
+  a.pairs = dst.pair.p;
+  a.cap = static_cast<int>(dst.colour.cap);  // (the arrays of a set are reserved together)
+  a.old_np = w->set_np[w->cur];
+  a.old_off = old.off.p;
+  a.old_pairs = old.pair.p;
+  a.old_index = dst.old_index.p;
+  a.colour = dst.colour.p;
+  a.host = w->h_counters + kPinnedFind;
+  static_assert(kPinnedFind + 5 <= kPinnedInts, "pinned pair-search counters");
+  a.epoch = ++w->publish_epoch;
+  hipLaunchKernelGGL(k_small_build, dim3(1), dim3(kSmallBlock), 0, w->stream, a);
+  PairFilter pf{w->f.body.p, w->b.type.p, w->f.filter.p, w->f.shape.p, w->f.world.p, nc ? w->j.nc_off.p : nullptr,
+                nc ? w->j.nc_list.p : nullptr};
+  TreeView tv{nt, bp.nodes4.p, bp.leafrec.p, w->f.loose_off.p, w->f.loose.p, np - nt, 0};
+  hipLaunchKernelGGL(k_traverse<false>, dim3(blocks_for(nt * kTravLanes, kTravBlock)), dim3(kTravBlock), 0, w->stream,
+                     nt, w->f.fat.p, tv, pf, bp.count.p, bp.slots.p, nullptr, nullptr, a.flags, bail);
+  hipLaunchKernelGGL(k_small_pairs, dim3(1), dim3(kSmallBlock), 0, w->stream, a);
+  B2G_HIP(hipGetLastError());
+  if ((st = wait_published(w, a.host, a.epoch))) return st;
+  if (a.host[1]) {
+    set_error("broadphase: BVH traversal stack overflow");
+    return B2G_ERR_CAPACITY;
+  }
+  if (a.host[3]) {
+    set_error("device scan: a tile waited too long for its predecessor");
+    return B2G_ERR_DEVICE;
+  }
+  const int total = a.host[4];
+  if (a.host[2] > 0 || total > a.cap) {
+    // the pairs and their predecessors by the launches (a walk overflowed its slots, or the set outgrew
+    // its arrays)
+    if ((st = reserve_contacts(w, dst, total))) return st;
+    hipLaunchKernelGGL(k_pairs_from_slots, dim3(blocks_for(nt, kBlock)), dim3(kBlock), 0, w->stream, nt, bp.leafrec.p,
+                       bp.count.p, bp.slots.p, dst.off.p, dst.pair.p);
+    if (a.host[2] > 0)
+      hipLaunchKernelGGL(k_traverse<true>, dim3(blocks_for(nt * kTravLanes, kTravBlock)), dim3(kTravBlock), 0, w->stream,
+                         nt, w->f.fat.p, tv, pf, bp.count.p, bp.slots.p, dst.off.p, dst.pair.p, a.flags, nullptr);
+    hipLaunchKernelGGL(k_merge, dim3(blocks_for(total, kBlock)), dim3(kBlock), 0, w->stream, total, dst.pair.p,
+                       a.old_np, old.off.p, old.pair.p, dst.old_index.p, dst.colour.p);
+    B2G_HIP(hipGetLastError());
+  }
+  w->set_np[next] = np;
+  w->cur = next;
+  w->n_pairs_old = w->n_pairs;
+  w->n_pairs = total;
+  return B2G_OK;
 }
 
 }  // namespace b2g

@@ -378,11 +378,13 @@ struct World {
   int set_np[2] = {0, 0};  // proxy count when each contact set was built (0: never built)
   SolverArrays s;
   BroadphaseArrays bp;
+  DevArray<int> small_bail;  // the small-world solve did nothing: the kernels after it do nothing either
   DevArray<int> counters;   // small device counters: 4 solver counters, then the colour histogram
   // pinned host memory (kPinnedInts ints): [0, 134) the solver's counters read back after the
   // colouring (4 counters, 128 colour counts, last round, large-island constraints),
   // [kPinnedPairFlags, +4) the pair search's flags and total, [kPinnedColourOffsets, +385) the
-  // colour offsets uploaded for the solve, [kPinnedToi, +4) the counters of a separable TOI pass
+  // colour offsets uploaded for the solve, [kPinnedToi, +8) the counters of a separable TOI pass,
+  // [kPinnedSmall, +134) and [kPinnedFind, +6) what the small-world kernels publish
   int* h_counters = nullptr;
   int n_touch = 0, n_colors = 0, n_islands = 0;
   int color_rounds = 16;       // colouring rounds launched before the first readback
@@ -402,6 +404,8 @@ struct World {
   int island_solve = -1;
   int bin_threads = 256;
   int n_bins = 0;  // bins of the last solve
+  int publish_epoch = 0;   // value of the last published word (pinned memory)
+  int small_holdoff = 0;   // steps for which the small-world kernels are left alone after a world outgrew them
   int solve_groups = 0;  // groups per colour of the last solve's constraints (s.cw_off); 0: not grouped
   bool worlds_contiguous = false;         // every world's bodies are one index range (set at upload)
   std::vector<int> h_world_body_off;      // n_worlds + 1 (when contiguous)
@@ -431,7 +435,8 @@ struct World {
   JointArrays j;
 };
 
-constexpr int kPinnedInts = 1024, kPinnedPairFlags = 192, kPinnedColourOffsets = 256, kPinnedToi = 768;
+constexpr int kPinnedInts = 1024, kPinnedPairFlags = 192, kPinnedColourOffsets = 256, kPinnedToi = 768,
+              kPinnedSmall = 800, kPinnedFind = 944;
 
 // Capacity floor of the arrays sized by the contact set (the pairs, and the solver's arrays,
 // which the pairs bound): reserving for a multiple of the proxy count from the first step keeps a
@@ -524,10 +529,21 @@ int kt_harvest(World* w);
 
 // phase drivers (each returns a B2G_* status)
 int upload_world(World* w);
+int phase_broadphase_general(World* w);
 int phase_broadphase(World* w);  // fat AABBs -> next contact set (pairs + old indices)
 int phase_collide(World* w);     // narrowphase on the current contact set
 int phase_solve(World* w, float dt, float dt_ratio, int vel_iters, int pos_iters);
 int phase_synchronize(World* w); // swept + fat AABBs of non-static proxies
+struct IslandView;
+// Small worlds (b2g_world_step): a step's solve in one launch and its pair search in three
+constexpr int kSmallBodies = 2048, kSmallTree = 2048, kSmallProxies = 4096, kSmallPairs = 4096, kSmallTouch = 2048;
+bool small_step_fits(const World* w);
+// runs the solve and find_new_contacts; *done false: the world did not fit after all and nothing was done
+int small_step(World* w, float dt, float dt_ratio, int vel_iters, int pos_iters, bool* done);
+bool small_find_fits(const World* w);
+int small_find(World* w, bool sync, IslandView iv, const int* bail);
+// waits until the word at `flag` (pinned, written by a kernel) is `value`
+int wait_published(World* w, const int* flag, int value);
 int phase_toi(World* w, float dt, int vi);  // continuous collision after the solve
 void toi_note_bodies(World* w);             // has_kinematic, has_bullet and statics_still from the host mirrors
 int toi_carry_state(World* w);              // TOI state of the previous contact set onto the current one

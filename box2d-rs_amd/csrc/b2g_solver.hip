@@ -119,12 +119,10 @@ __global__ void __launch_bounds__(kBlock) k_finalize(int nb, const int* __restri
 // of awake islands: each body's sleep time is reset when it may not sleep or moves faster than
 // the tolerances, else advanced by h; an island whose bodies all reached kTimeToSleep (no body
 // marks it restless) and whose position iterations converged goes to sleep.
-__global__ void __launch_bounds__(kBlock) k_sleep_time(int nb, const int* __restrict__ btype,
-                                                       const int* __restrict__ auto_sleep, const float4* __restrict__ vel,
-                                                       float* __restrict__ sleep_time, IslandView iv,
-                                                       int* __restrict__ restless, float h) {
-  const int b = blockIdx.x * blockDim.x + threadIdx.x;
-  if (b >= nb || btype[b] == 0 || iv.asleep(b)) return;
+__device__ inline void sleep_time_one(int b, const int* __restrict__ btype, const int* __restrict__ auto_sleep,
+                                      const float4* __restrict__ vel, float* __restrict__ sleep_time, const IslandView& iv,
+                                      int* __restrict__ restless, float h) {
+  if (btype[b] == 0 || iv.asleep(b)) return;
   const float lin_tol_sqr = kLinearSleepTolerance * kLinearSleepTolerance;
   const float ang_tol_sqr = kAngularSleepTolerance * kAngularSleepTolerance;
   const float4 v = vel[b];
@@ -137,12 +135,11 @@ __global__ void __launch_bounds__(kBlock) k_sleep_time(int nb, const int* __rest
   sleep_time[b] = t;
   if (!(t >= kTimeToSleep)) restless[iv.parent[b]] = 1;
 }
-__global__ void __launch_bounds__(kBlock) k_sleep_apply(int nb, const int* __restrict__ btype, IslandView iv,
-                                                        const int* __restrict__ restless, const int* __restrict__ done,
-                                                        int* __restrict__ awake, float* __restrict__ sleep_time,
-                                                        float4* __restrict__ vel, float4* __restrict__ force) {
-  const int b = blockIdx.x * blockDim.x + threadIdx.x;
-  if (b >= nb || btype[b] == 0 || iv.asleep(b)) return;
+__device__ inline void sleep_apply_one(int b, const int* __restrict__ btype, const IslandView& iv,
+                                       const int* __restrict__ restless, const int* __restrict__ done,
+                                       int* __restrict__ awake, float* __restrict__ sleep_time, float4* __restrict__ vel,
+                                       float4* __restrict__ force) {
+  if (btype[b] == 0 || iv.asleep(b)) return;
   const int r = iv.parent[b];
   if (restless[r] || !done[r]) return;
   // B2body::set_awake(false)
@@ -150,6 +147,20 @@ __global__ void __launch_bounds__(kBlock) k_sleep_apply(int nb, const int* __res
   sleep_time[b] = 0.0f;
   vel[b] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
   force[b] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+}
+__global__ void __launch_bounds__(kBlock) k_sleep_time(int nb, const int* __restrict__ btype,
+                                                       const int* __restrict__ auto_sleep, const float4* __restrict__ vel,
+                                                       float* __restrict__ sleep_time, IslandView iv,
+                                                       int* __restrict__ restless, float h) {
+  const int b = blockIdx.x * blockDim.x + threadIdx.x;
+  if (b < nb) sleep_time_one(b, btype, auto_sleep, vel, sleep_time, iv, restless, h);
+}
+__global__ void __launch_bounds__(kBlock) k_sleep_apply(int nb, const int* __restrict__ btype, IslandView iv,
+                                                        const int* __restrict__ restless, const int* __restrict__ done,
+                                                        int* __restrict__ awake, float* __restrict__ sleep_time,
+                                                        float4* __restrict__ vel, float4* __restrict__ force) {
+  const int b = blockIdx.x * blockDim.x + threadIdx.x;
+  if (b < nb) sleep_apply_one(b, btype, iv, restless, done, awake, sleep_time, vel, force);
 }
 
 // ---- touching contacts, islands, colouring -----------------------------------------------------
@@ -1638,41 +1649,35 @@ __device__ void solve_world_in_memory(const GroupSolve& a, const int2* rng, int 
   }
 }
 
-// (at least two waves per SIMD: with four constraints per thread the compiler otherwise takes a few
-// registers more than half of the file)
+template <int T, int NB, bool kWorlds>
+struct GroupStore {
+  static constexpr int H = kWorlds ? NB : kBinHashPerThread * T, LG = kWorlds ? 1 : ilog2(H);
+  static constexpr int HR = kWorlds ? NB : 2 * T, LGR = kWorlds ? 1 : ilog2(HR);  // a bin has fewer than T islands
+  int2 rng[kMaxColors];  // the group's constraints of each colour
+  int keys[kWorlds ? 1 : H], rkeys[kWorlds ? 1 : HR];
+  float4 bv[H], bp[H];
+  int rdone[HR];
+  unsigned char rviol[HR], btype[H];
+};
+
+// The group's solve by a workgroup of T threads; s.rng is filled (and, for a bin, the tables are
+// empty), worlds: bodies [b0, b0 + nbody).
 template <int T, int C, int NB, bool kWorlds>
-__global__ void __launch_bounds__(T, 2) k_solve_groups(GroupSolve a) {
-  constexpr int H = kWorlds ? NB : kBinHashPerThread * T, LG = kWorlds ? 1 : ilog2(H);
-  constexpr int HR = kWorlds ? NB : 2 * T, LGR = kWorlds ? 1 : ilog2(HR);  // a bin has fewer than T islands
-  __shared__ int2 rng[kMaxColors];
-  __shared__ int keys[kWorlds ? 1 : H], rkeys[kWorlds ? 1 : HR];
-  __shared__ float4 bv[H], bp[H];
-  __shared__ int rdone[HR];
-  __shared__ unsigned char rviol[HR], btype[H];
+__device__ void solve_group(const GroupSolve& a, GroupStore<T, NB, kWorlds>& s, int ncolors, int b0, int nbody) {
+  constexpr int H = GroupStore<T, NB, kWorlds>::H, LG = GroupStore<T, NB, kWorlds>::LG;
+  constexpr int HR = GroupStore<T, NB, kWorlds>::HR, LGR = GroupStore<T, NB, kWorlds>::LGR;
+  int2* rng = s.rng;
+  int *keys = s.keys, *rkeys = s.rkeys, *rdone = s.rdone;
+  float4 *bv = s.bv, *bp = s.bp;
+  unsigned char *rviol = s.rviol, *btype = s.btype;
   const int t = threadIdx.x;
-  const int g = kWorlds ? a.wlist[a.wbase + blockIdx.x] : blockIdx.x;
-  for (int c = t; c < a.ncolors; c += T) rng[c] = make_int2(a.off[c * a.ng + g], a.off[c * a.ng + g + 1]);
-  if (!kWorlds) {
-    for (int e = t; e < H; e += T) keys[e] = -1;
-    for (int e = t; e < HR; e += T) rkeys[e] = -1;
-  }
-  const int b0 = kWorlds ? a.body_off[g] : 0, nbody = kWorlds ? a.body_off[g + 1] - b0 : 0;
-  __syncthreads();
-  if (kWorlds) {
-    int n = 0;
-    for (int c = 0; c < a.ncolors; ++c) n += rng[c].y - rng[c].x;
-    if (n > T * C || nbody > NB) {  // uniform across the workgroup
-      solve_world_in_memory<T>(a, rng, b0, b0 + nbody);
-      return;
-    }
-  }
   // the thread's constraints, their bodies and islands
   int i[C], col[C], k[C], sa[C], sb[C], sr[C];
   int2 f[C], bd[C];
   bool dA[C], dB[C];
 #pragma unroll
   for (int q = 0; q < C; ++q) {
-    i[q] = bin_constraint(rng, a.ncolors, t + q * T, &col[q]);
+    i[q] = bin_constraint(rng, ncolors, t + q * T, &col[q]);
     k[q] = sa[q] = sb[q] = sr[q] = 0;
     f[q] = bd[q] = make_int2(0, 0);
     dA[q] = dB[q] = false;
@@ -1737,7 +1742,7 @@ __global__ void __launch_bounds__(T, 2) k_solve_groups(GroupSolve a) {
   }
   __syncthreads();  // every set-up has read the velocities
   for (int it = a.init.warm ? -1 : 0; it < a.vel_iters; ++it)  // -1: the warm start
-    for (int c = 0; c < a.ncolors; ++c) {
+    for (int c = 0; c < ncolors; ++c) {
       if (rng[c].x == rng[c].y) continue;  // uniform across the workgroup
 #pragma unroll
       for (int q = 0; q < C; ++q) {
@@ -1799,7 +1804,7 @@ __global__ void __launch_bounds__(T, 2) k_solve_groups(GroupSolve a) {
   }
   __syncthreads();
   for (int it = 0; it < a.pos_iters; ++it) {
-    for (int c = 0; c < a.ncolors; ++c) {
+    for (int c = 0; c < ncolors; ++c) {
       if (rng[c].x == rng[c].y) continue;
 #pragma unroll
       for (int q = 0; q < C; ++q) {
@@ -1836,6 +1841,31 @@ __global__ void __launch_bounds__(T, 2) k_solve_groups(GroupSolve a) {
     a.pos.done[r] = rdone[e];
     a.pos.violated[r] = rviol[e];
   }
+}
+
+// (at least two waves per SIMD: with four constraints per thread the compiler otherwise takes a few
+// registers more than half of the file)
+template <int T, int C, int NB, bool kWorlds>
+__global__ void __launch_bounds__(T, 2) k_solve_groups(GroupSolve a) {
+  __shared__ GroupStore<T, NB, kWorlds> s;
+  const int t = threadIdx.x;
+  const int g = kWorlds ? a.wlist[a.wbase + blockIdx.x] : blockIdx.x;
+  for (int c = t; c < a.ncolors; c += T) s.rng[c] = make_int2(a.off[c * a.ng + g], a.off[c * a.ng + g + 1]);
+  if (!kWorlds) {
+    for (int e = t; e < s.H; e += T) s.keys[e] = -1;
+    for (int e = t; e < s.HR; e += T) s.rkeys[e] = -1;
+  }
+  const int b0 = kWorlds ? a.body_off[g] : 0, nbody = kWorlds ? a.body_off[g + 1] - b0 : 0;
+  __syncthreads();
+  if (kWorlds) {
+    int n = 0;
+    for (int c = 0; c < a.ncolors; ++c) n += s.rng[c].y - s.rng[c].x;
+    if (n > T * C || nbody > NB) {  // uniform across the workgroup
+      solve_world_in_memory<T>(a, s.rng, b0, b0 + nbody);
+      return;
+    }
+  }
+  solve_group<T, C, NB, kWorlds>(a, s, a.ncolors, b0, nbody);
 }
 
 // Bins: one launch; worlds: one per body-count bucket with that bucket's threads per world, whose LDS
@@ -1880,6 +1910,312 @@ static void launch_groups(World* w, int nc, bool worlds, GroupSolve a) {
     if (k == 0) launch_world_bucket<64>(w, kernel, share, n, w->world_threads[k], a);
     else if (k == 1) launch_world_bucket<256>(w, kernel, share, n, w->world_threads[k], a);
     else launch_world_bucket<1088>(w, kernel, share, n, w->world_threads[k], a);
+  }
+}
+
+// ---- small worlds: a step's whole solve in one workgroup ------------------------------------------
+// A single world of at most kSmallBodies bodies and kSmallTouch touching contacts spends its step on
+// launches and on the host's wait for the colour counts, not on work: the 210-box pyramid's solve was
+// 45 launches at 3 us of host time each. One workgroup instead compacts the touching contacts, finds the
+// islands (union-find in LDS), colours the constraints (the rounds of k_color_keep and k_color_round, with a
+// barrier for the launch boundary, until none is left), sorts them by colour and runs the group solve with
+// the world as its group, then the end of the last position iteration, the transforms and the sleep rules.
+// The constraint numbers, priorities, colours and operations are those of the launches it replaces, so the
+// results are the same bit for bit. A world with more touching contacts or with a body of more than 127
+// (whose last colour is solved serially) is left untouched (*bail) and stepped by those launches.
+// A frame (step and states) of one box on the ground: 290 us -> 203 us; of the pyramid: 403 us -> 288 us;
+// 40 steps of 1531 stacked boxes: 20.8 ms -> 17.9 ms (one workgroup then is slower than the bins' many by 50 us
+// a step, the launches were 120 us).
+constexpr int kSmallThreads = 512;
+static_assert(kSmallThreads >= kMaxColors, "a thread per colour");
+
+struct SmallArgs {
+  GroupSolve g;  // (off, ng and ncolors unused)
+  int nb, n_pairs;
+  const int* touch_flag;
+  const int* old_index;
+  const int* old_colour;  // null: colours are not reused
+  int colour_cap;         // kept colours are below it
+  int* parent;
+  int *violated, *done, *isl_awake, *restless;  // isl_awake null: no sleeping
+  int* awake;
+  IntegrateArgs integrate;
+  int4* rec;
+  int* k_contact;
+  int* pair_colour;
+  int* color_off;  // [ncolors + 1], and the same as the group offsets of one group
+  int* cw_off;
+  // the end of the step
+  float4* xf;
+  int allow_sleep;
+  const int* auto_sleep;
+  float* sleep_time;
+  float4* force;
+  int* bail;
+  int* host;  // pinned: [0] published, [1] bail, [2] touching, [3] solved, [4] colours, [5] last round, [6..] counts
+  int epoch;
+};
+
+struct SmallSetup {
+  int parent[kSmallBodies];
+  int off[kSmallBodies + 1];
+  int cursor[kSmallBodies];
+  unsigned short adj[2 * kSmallTouch];
+  int contact[kSmallTouch];
+  unsigned short bodyA[kSmallTouch], bodyB[kSmallTouch];
+  int state[kSmallTouch];
+  short prev[kSmallTouch];
+  unsigned char type[kSmallBodies];
+};
+static_assert(kSmallBodies <= 65536 && kSmallTouch <= 65536, "16-bit body and constraint numbers");
+
+__global__ void __launch_bounds__(kSmallThreads, 2) k_small_solve(SmallArgs a) {
+  constexpr int T = kSmallThreads;
+  using Store = GroupStore<T, kSmallBodies, true>;
+  __shared__ __align__(16) unsigned char raw[sizeof(Store) > sizeof(SmallSetup) ? sizeof(Store) : sizeof(SmallSetup)];
+  __shared__ int wsum[T / 64], count[kMaxColors], launch[kMaxColors], base[kMaxColors + 1], cursor[kMaxColors];
+  __shared__ int n_touch, left, last_round, overflow, ncolors, nsolved;
+  SmallSetup& s = *reinterpret_cast<SmallSetup*>(raw);
+  const int t = threadIdx.x, lane = t & 63, wid = t >> 6;
+  // exclusive scan over the threads' values; every thread gets its prefix, *total the sum
+  auto scan = [&](int x, int* total) {
+    int inc = x;
+    for (int d = 1; d < 64; d <<= 1) {
+      const int y = __shfl_up(inc, d, 64);
+      if (lane >= d) inc += y;
+    }
+    if (lane == 63) wsum[wid] = inc;
+    __syncthreads();
+    int before = 0, sum = 0;
+    for (int w = 0; w < T / 64; ++w) {
+      if (w < wid) before += wsum[w];
+      sum += wsum[w];
+    }
+    __syncthreads();
+    *total = sum;
+    return before + inc - x;
+  };
+  if (t == 0) left = last_round = overflow = 0;
+  for (int c = t; c < kMaxColors; c += T) count[c] = cursor[c] = 0;
+  // touching contacts in pair order: constraint j = its rank among them
+  {
+    const int chunk = (a.n_pairs + T - 1) / T, k0 = min(a.n_pairs, t * chunk), k1 = min(a.n_pairs, k0 + chunk);
+    int n = 0, total;
+    for (int k = k0; k < k1; ++k) n += a.touch_flag[k] != 0;
+    int j = scan(n, &total);
+    if (t == 0) n_touch = total;
+    if (total <= kSmallTouch)
+      for (int k = k0; k < k1; ++k)
+        if (a.touch_flag[k]) s.contact[j++] = k;
+  }
+  for (int b = t; b < a.nb; b += T) {
+    s.parent[b] = b;
+    s.off[b] = 0;
+    s.cursor[b] = 0;
+    s.type[b] = static_cast<unsigned char>(a.g.btype[b]);
+  }
+  if (t == 0) s.off[a.nb] = 0;
+  __syncthreads();
+  const int nt = n_touch;
+  auto parent_of = [&](int x) {
+    return __hip_atomic_load(&s.parent[x], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+  };
+  auto bail_out = [&] {
+    if (t == 0) {
+      *a.bail = 1;
+      a.host[1] = 1;
+      __threadfence_system();
+      __hip_atomic_store(a.host, a.epoch, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+  };
+  if (nt > kSmallTouch) {  // uniform
+    bail_out();
+    return;
+  }
+  // bodies, degrees (dynamic bodies only), previous colours; islands
+  for (int j = t; j < nt; j += T) {
+    const int k = s.contact[j];
+    const int2 f = a.g.init.ab[k];
+    const int bA = a.g.init.fbody[f.x], bB = a.g.init.fbody[f.y];
+    s.bodyA[j] = static_cast<unsigned short>(bA);
+    s.bodyB[j] = static_cast<unsigned short>(bB);
+    if (s.type[bA] == 2) atomicAdd(&s.off[bA], 1);
+    if (s.type[bB] == 2) atomicAdd(&s.off[bB], 1);
+    int pc = -1;
+    if (a.old_colour) {
+      const int o = a.old_index[k];
+      if (o >= 0) pc = a.old_colour[o];
+    }
+    s.prev[j] = static_cast<short>(pc >= 0 && pc < kMaxColors ? pc : -1);
+    if (s.type[bA] != 0 && s.type[bB] != 0) {
+      // union_bodies on the LDS array (a CAS there sees every link, so a failed one climbs from it)
+      int x = bA, y = bB;
+      for (;;) {
+        for (int p = parent_of(x); p != x; p = parent_of(x)) x = p;
+        for (int p = parent_of(y); p != y; p = parent_of(y)) y = p;
+        if (x == y) break;
+        const bool x_low = uf_below(x, y);
+        const int lo = x_low ? x : y, hi = x_low ? y : x;
+        if (atomicCAS(&s.parent[lo], lo, hi) == lo) break;
+      }
+    }
+  }
+  __syncthreads();
+  // island roots to memory, with the islands' flags; the degrees' scan
+  for (int b = t; b < a.nb; b += T) {
+    int r = b;
+    for (int p = s.parent[r]; p != r; p = s.parent[r]) r = p;
+    a.parent[b] = r;
+    a.violated[b] = 0;
+    a.done[b] = 0;
+    if (a.isl_awake) {
+      a.isl_awake[b] = 0;
+      a.restless[b] = 0;
+    }
+  }
+  {
+    const int n = a.nb + 1, chunk = (n + T - 1) / T, i0 = min(n, t * chunk), i1 = min(n, i0 + chunk);
+    int sum = 0, total;
+    for (int i = i0; i < i1; ++i) sum += s.off[i];
+    int ex = scan(sum, &total);
+    for (int i = i0; i < i1; ++i) {
+      const int v = s.off[i];
+      s.off[i] = ex;
+      ex += v;
+    }
+  }
+  __syncthreads();
+  const IslandView iv{a.parent, a.isl_awake};
+  if (a.isl_awake)
+    for (int b = t; b < a.nb; b += T)
+      if (s.type[b] != 0 && a.awake[b]) a.isl_awake[a.parent[b]] = 1;
+  for (int j = t; j < nt; j += T) {
+    const int bA = s.bodyA[j], bB = s.bodyB[j];
+    if (s.type[bA] == 2) s.adj[s.off[bA] + atomicAdd(&s.cursor[bA], 1)] = static_cast<unsigned short>(j);
+    if (s.type[bB] == 2) s.adj[s.off[bB] + atomicAdd(&s.cursor[bB], 1)] = static_cast<unsigned short>(j);
+  }
+  __syncthreads();
+  // neighbours of constraint j: fn(o) for every other constraint on one of its dynamic bodies
+  auto neighbours = [&](int j, auto&& fn) {
+    for (int side = 0; side < 2; ++side) {
+      const int b = side ? s.bodyB[j] : s.bodyA[j];
+      if (s.type[b] != 2) continue;
+      for (int e = s.off[b]; e < s.off[b + 1]; ++e)
+        if (s.adj[e] != j) fn(int(s.adj[e]));
+    }
+  };
+  // round 0 (k_color_keep): a kept colour, -1, or -2 for a sleeping island's constraint
+  for (int j = t; j < nt; j += T) {
+    const int bA = s.bodyA[j], bB = s.bodyB[j];
+    int st = -1;
+    if (iv.asleep(s.type[bA] != 0 ? bA : bB)) {
+      st = -2;
+    } else if (s.prev[j] >= 0 && s.prev[j] < a.colour_cap) {
+      const unsigned long long pj = priority(j);
+      bool kept = true;
+      neighbours(j, [&](int o) {
+        if (s.prev[o] == s.prev[j] && priority(o) > pj) kept = false;
+      });
+      if (kept) st = s.prev[j];
+    }
+    s.state[j] = st;
+    if (st == -1) left = 1;  // every writer stores 1
+  }
+  __syncthreads();
+  // Jones-Plassmann-Luby rounds (k_color_round): each colours at least the uncoloured constraint of
+  // highest priority, so at most nt of them run
+  for (int round = 1; left; ++round) {
+    __syncthreads();
+    if (t == 0) left = 0;
+    __syncthreads();
+    for (int j = t; j < nt; j += T) {
+      if (s.state[j] != -1) continue;
+      const unsigned long long pj = priority(j);
+      unsigned long long used0 = 0, used1 = 0;
+      bool lose = false;
+      neighbours(j, [&](int o) {
+        color_look(o, __hip_atomic_load(&s.state[o], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP), round, pj, lose,
+                   used0, used1);
+      });
+      int c = -1;
+      if (!lose) c = ~used0 ? __ffsll(static_cast<long long>(~used0)) - 1
+                            : ~used1 ? 64 + __ffsll(static_cast<long long>(~used1)) - 1 : kMaxColors - 1;
+      if (c < 0) {
+        left = 1;
+        continue;
+      }
+      __hip_atomic_store(&s.state[j], (round << 8) | c, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+      last_round = round;
+    }
+    __syncthreads();
+  }
+  // colour counts; a constraint of the highest colour means a body with more contacts than the masks hold
+  for (int j = t; j < nt; j += T)
+    if (s.state[j] >= 0) atomicAdd(&count[s.state[j] & 0xff], 1);
+  __syncthreads();
+  if (count[kMaxColors - 1] > 0) {  // uniform
+    bail_out();
+    return;
+  }
+  if (t == 0) {
+    int n = 0, nc = 0;
+    for (int c = 0; c < kMaxColors; ++c) {
+      launch[c] = nc;
+      if (count[c] == 0) continue;
+      base[nc++] = n;
+      n += count[c];
+    }
+    base[nc] = n;
+    ncolors = nc;
+    nsolved = n;
+  }
+  __syncthreads();
+  const int nc = ncolors;
+  for (int j = t; j < nt; j += T) {
+    if (s.state[j] < 0) continue;
+    const int L = launch[s.state[j] & 0xff], k = s.contact[j], bA = s.bodyA[j], bB = s.bodyB[j];
+    const int pos = base[L] + atomicAdd(&cursor[L], 1);
+    a.k_contact[pos] = k;
+    a.rec[pos] = sorted_record(k, make_int2(bA, bB), s.type[bA] == 2, s.type[bB] == 2,
+                               a.parent[s.type[bA] != 0 ? bA : bB]);
+    a.pair_colour[k] = L;
+  }
+  for (int c = t; c <= nc; c += T) a.color_off[c] = a.cw_off[c] = base[c];
+  // the host's copy of all this
+  if (t < kMaxColors) a.host[6 + t] = count[t];
+  if (t == 0) {
+    a.host[1] = 0;
+    a.host[2] = nt;
+    a.host[3] = nsolved;
+    a.host[4] = nc;
+    a.host[5] = last_round;
+    *a.bail = 0;
+  }
+  if (t < kMaxColors) __threadfence_system();  // (published at the end)
+  // velocity integration of the awake islands' bodies
+  for (int b = t; b < a.nb; b += T) integrate_velocity_one(b, a.integrate, iv, a.isl_awake ? a.awake : nullptr);
+  __syncthreads();
+  Store& g = *reinterpret_cast<Store*>(raw);
+  for (int c = t; c < nc; c += T) g.rng[c] = make_int2(base[c], base[c + 1]);
+  __syncthreads();
+  solve_group<T, 4, kSmallBodies, true>(a.g, g, nc, 0, a.nb);
+  __syncthreads();
+  // the last position iteration's end, the transforms, and the islands' sleep
+  for (int b = t; b < a.nb; b += T) {
+    if (a.g.pos_iters > 0)
+      iteration_end_one(b, a.g.pos_iters - 1, a.g.btype, a.parent, a.violated, a.done, a.isl_awake);
+    finalize_one(b, a.g.btype, a.g.pos.pos, a.g.init.bmass, a.xf, iv);
+    if (a.allow_sleep)
+      sleep_time_one(b, a.g.btype, a.auto_sleep, a.g.vel.vel, a.sleep_time, iv, a.restless, a.g.dt);
+  }
+  if (a.allow_sleep) {
+    __syncthreads();
+    for (int b = t; b < a.nb; b += T)
+      sleep_apply_one(b, a.g.btype, iv, a.restless, a.done, a.awake, a.sleep_time, a.g.vel.vel, a.force);
+  }
+  if (t == 0) {
+    __threadfence_system();
+    __hip_atomic_store(a.host, a.epoch, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
   }
 }
 
@@ -2007,6 +2343,58 @@ static int reserve_solver(World* w, int nc) {
   return B2G_OK;
 }
 
+// Colour reuse (persisting contacts keep their colour) lets the colour count creep up as new
+// contacts take first-fit colours around kept ones; the step colours from scratch again once
+// the count exceeds the last from-scratch count by kColorSlack, and at least every
+// kColorRefresh steps (which keeps that count, the cap on kept colours, current).
+static bool reuse_colours(const World* w) {
+  constexpr int kColorSlack = 2, kColorRefresh = 32;
+  return w->color_reuse && w->scratch_colors > 0 && w->n_colors <= w->scratch_colors + kColorSlack &&
+         w->steps_since_scratch < kColorRefresh;
+}
+// after a step's colouring (w->n_colors)
+static void note_colours(World* w, bool reuse) {
+  if (!reuse && w->n_colors > 0) {
+    w->scratch_colors = w->n_colors;
+    w->steps_since_scratch = 0;
+  } else {
+    ++w->steps_since_scratch;
+  }
+}
+
+// the constraint set-up's arguments for the current contact set
+static InitArgs init_args(World* w, int nc, float dt_ratio) {
+  SolverArrays& s = w->s;
+  ContactArrays& c = w->c[w->cur];
+  InitArgs init;
+  init.n = nc;
+  init.order = s.order.p;
+  init.list = s.touch_list.p;
+  init.ab = c.ab.p;
+  init.fbody = w->f.body.p;
+  init.fshape = w->f.shape.p;
+  init.fmat = w->f.mat.p;
+  init.btype = w->b.type.p;
+  init.parent = s.parent.p;
+  init.bpos = w->b.pos.p;
+  init.bvel = w->b.vel.p;
+  init.bmass = w->b.mass.p;
+  init.hdr = c.hdr.p;
+  init.geo = c.geo.p;
+  init.pt0 = c.pt0.p;
+  init.pt1 = c.pt1.p;
+  init.dt_ratio = dt_ratio;
+  init.warm = w->warm_starting;
+  init.block_solve = w->block_solve;
+  init.k_contact = s.k_contact.p;
+  init.k_bodies = s.k_bodies.p;  // overwritten in colour order (the unsorted copy is no longer needed)
+  init.k_info = s.k_info.p;
+  init.vnf = s.vnf.p; init.vm = s.vm.p; init.vr0 = s.vr0.p; init.vr1 = s.vr1.p; init.vms = s.vms.p; init.vbias = s.vbias.p;
+  init.K = s.K.p; init.NM = s.NM.p; init.lam = s.lam.p; init.plp = s.plp.p; init.pgeo = s.pgeo.p; init.plc = s.plc.p;
+  init.prad = s.prad.p;
+  return init;
+}
+
 int phase_solve(World* w, float dt, float dt_ratio, int vel_iters, int pos_iters) {
   const int nb = w->nb;
   if (nb == 0) return B2G_OK;
@@ -2044,13 +2432,7 @@ int phase_solve(World* w, float dt, float dt_ratio, int vel_iters, int pos_iters
   if (n_pairs == 0)
     hipLaunchKernelGGL(k_solver_counters_init, dim3(1), dim3(kBlock), 0, w->stream, cnt, s.color_cursor.p);
   const int gp = blocks_for(std::max(n_pairs, 1), kBlock);
-  // Colour reuse (persisting contacts keep their colour) lets the colour count creep up as new
-  // contacts take first-fit colours around kept ones; the step colours from scratch again once
-  // the count exceeds the last from-scratch count by kColorSlack, and at least every
-  // kColorRefresh steps (which keeps that count, the cap on kept colours, current).
-  constexpr int kColorSlack = 2, kColorRefresh = 32;
-  const bool reuse = w->color_reuse && w->scratch_colors > 0 && w->n_colors <= w->scratch_colors + kColorSlack &&
-                     w->steps_since_scratch < kColorRefresh;
+  const bool reuse = reuse_colours(w);
   // constraints (touching contacts): list, bodies, degrees, previous colours; then islands
   if (n_pairs > 0) {
     // colours of the previous step's contacts (the old set's solve wrote them)
@@ -2140,32 +2522,7 @@ int phase_solve(World* w, float dt, float dt_ratio, int vel_iters, int pos_iters
   if (per_world) w->solve_groups = w->n_worlds;
   // every constraint is in a bin or in a world's group: the whole solve runs in k_solve_groups
   const bool grouped = w->solve_groups > 0;
-  InitArgs init;
-  init.n = nc;
-  init.order = s.order.p;
-  init.list = s.touch_list.p;
-  init.ab = c.ab.p;
-  init.fbody = w->f.body.p;
-  init.fshape = w->f.shape.p;
-  init.fmat = w->f.mat.p;
-  init.btype = w->b.type.p;
-  init.parent = s.parent.p;
-  init.bpos = w->b.pos.p;
-  init.bvel = w->b.vel.p;
-  init.bmass = w->b.mass.p;
-  init.hdr = c.hdr.p;
-  init.geo = c.geo.p;
-  init.pt0 = c.pt0.p;
-  init.pt1 = c.pt1.p;
-  init.dt_ratio = dt_ratio;
-  init.warm = w->warm_starting;
-  init.block_solve = w->block_solve;
-  init.k_contact = s.k_contact.p;
-  init.k_bodies = s.k_bodies.p;  // overwritten in colour order (the unsorted copy is no longer needed)
-  init.k_info = s.k_info.p;
-  init.vnf = s.vnf.p; init.vm = s.vm.p; init.vr0 = s.vr0.p; init.vr1 = s.vr1.p; init.vms = s.vms.p; init.vbias = s.vbias.p;
-  init.K = s.K.p; init.NM = s.NM.p; init.lam = s.lam.p; init.plp = s.plp.p; init.pgeo = s.pgeo.p; init.plc = s.plc.p;
-  init.prad = s.prad.p;
+  const InitArgs init = init_args(w, nc, dt_ratio);
   if (nc > 0) {
     // One launch per non-empty colour, in colour-id order (kept colours can leave gaps).
     // Device copy: launch offsets (kMaxColors + 1, padded with nc), then per colour id its base
@@ -2230,12 +2587,7 @@ int phase_solve(World* w, float dt, float dt_ratio, int vel_iters, int pos_iters
                    init);
   }
   w->n_colors = ncolors;
-  if (!reuse && ncolors > 0) {
-    w->scratch_colors = ncolors;
-    w->steps_since_scratch = 0;
-  } else {
-    ++w->steps_since_scratch;
-  }
+  note_colours(w, reuse);
   VelArgs va{s.k_bodies.p, s.k_info.p, s.vnf.p, s.vm.p, s.vr0.p, s.vr1.p, s.vms.p, s.vbias.p, s.K.p, s.NM.p, s.lam.p,
              w->b.vel.p};
   PosArgs pa{s.k_bodies.p, s.k_info.p, s.vm.p, s.plp.p, s.pgeo.p, s.plc.p, s.prad.p, w->b.pos.p, s.isl_violated.p,
@@ -2371,6 +2723,110 @@ int phase_solve(World* w, float dt, float dt_ratio, int vel_iters, int pos_iters
                        s.isl_restless.p, s.isl_done.p, w->b.awake.p, w->b.sleep_time.p, w->b.vel.p, w->b.force.p);
   }
   B2G_HIP(hipGetLastError());
+  return B2G_OK;
+}
+
+// The word a kernel publishes in pinned memory is seen a few microseconds before the stream's own
+// completion would be (a copy and a stream wait cost 13 us more than this). The stream is asked now and
+// then, so that the wait also ends when a launch failed and nothing will be published.
+int wait_published(World* w, const int* flag, int value) {
+  for (long long spin = 1;; ++spin) {
+    if (__atomic_load_n(flag, __ATOMIC_ACQUIRE) == value) return B2G_OK;
+    if ((spin & 0xfffff) != 0) continue;
+    const hipError_t e = hipStreamQuery(w->stream);
+    if (e == hipErrorNotReady) continue;
+    if (e == hipSuccess && __atomic_load_n(flag, __ATOMIC_ACQUIRE) == value) return B2G_OK;
+    set_error(std::string("a small-world kernel did not publish its result: ") + hipGetErrorString(e));
+    return B2G_ERR_DEVICE;
+  }
+}
+
+// Single worlds within the small kernels' limits, stepped with the solve's settings at their defaults (a
+// timed kernel, forced bins and solver graphs mean the launches they name) and without joints or a tape.
+bool small_step_fits(const World* w) {
+  return w->nb > 0 && w->nb <= kSmallBodies && w->n_pairs <= kSmallPairs && w->n_worlds == 1 && w->nj == 0 &&
+         !w->tape.active && w->island_solve == -1 && !w->solver_graphs && w->kt.kernel == B2G_KERNEL_NONE &&
+         w->small_holdoff == 0 && small_find_fits(w);
+}
+
+int small_step(World* w, float dt, float dt_ratio, int vel_iters, int pos_iters, bool* done) {
+  *done = false;
+  SolverArrays& s = w->s;
+  ContactArrays& c = w->c[w->cur];
+  const int nb = w->nb;
+  const bool sleepy = w->sleep_possible();
+  int st;
+  if ((st = reserve_solver(w, w->n_pairs)) || (st = s.touch_flag.reserve(pair_capacity(w, w->n_pairs))) ||
+      (st = s.parent.reserve(nb)) || (st = s.isl_violated.reserve(nb)) || (st = s.isl_done.reserve(nb)) ||
+      (st = s.isl_awake.reserve(nb)) || (st = s.isl_restless.reserve(nb)) ||
+      (st = s.color_off.reserve(3 * kMaxColors + 1)) || (st = s.cw_off.reserve(kMaxColors + 1)) ||
+      (st = w->small_bail.reserve(1)))
+    return st;
+  const bool reuse = reuse_colours(w);
+  const IslandView iv{s.parent.p, sleepy ? s.isl_awake.p : nullptr};
+  VelArgs va{s.k_bodies.p, s.k_info.p, s.vnf.p, s.vm.p, s.vr0.p, s.vr1.p, s.vms.p, s.vbias.p, s.K.p, s.NM.p, s.lam.p,
+             w->b.vel.p};
+  PosArgs pa{s.k_bodies.p, s.k_info.p, s.vm.p, s.plp.p, s.pgeo.p, s.plc.p, s.prad.p, w->b.pos.p, s.isl_violated.p,
+             s.isl_done.p};
+  SmallArgs a;
+  a.g = GroupSolve{init_args(w, 0, dt_ratio), s.k_rec.p, s.cw_off.p, 1, 0, vel_iters, pos_iters, dt, pa, va,
+                   w->b.type.p, iv, nullptr, nullptr, 0};
+  a.nb = nb;
+  a.n_pairs = w->n_pairs;
+  a.touch_flag = s.touch_flag.p;
+  a.old_index = c.old_index.p;
+  a.old_colour = reuse ? w->c[1 - w->cur].colour.p : nullptr;
+  a.colour_cap = w->scratch_colors;
+  a.parent = s.parent.p;
+  a.violated = s.isl_violated.p;
+  a.done = s.isl_done.p;
+  a.isl_awake = sleepy ? s.isl_awake.p : nullptr;
+  a.restless = s.isl_restless.p;
+  a.awake = w->b.awake.p;
+  a.integrate = IntegrateArgs{w->b.type.p, w->b.pos.p, w->b.vel.p, w->b.pos0.p, w->b.props.p, w->b.mass.p, w->b.force.p,
+                              w->gravity.x, w->gravity.y, dt};
+  a.rec = s.k_rec.p;
+  a.k_contact = s.k_contact.p;
+  a.pair_colour = c.colour.p;
+  a.color_off = s.color_off.p;
+  a.cw_off = s.cw_off.p;
+  a.xf = w->b.xf.p;
+  a.allow_sleep = w->allow_sleep;
+  a.auto_sleep = w->b.auto_sleep.p;
+  a.sleep_time = w->b.sleep_time.p;
+  a.force = w->b.force.p;
+  a.bail = w->small_bail.p;
+  a.host = w->h_counters + kPinnedSmall;
+  static_assert(kPinnedSmall + 6 + kMaxColors <= kPinnedFind, "pinned small-world counters");
+  a.epoch = ++w->publish_epoch;
+  hipLaunchKernelGGL(k_small_solve, dim3(1), dim3(kSmallThreads), 0, w->stream, a);
+  B2G_HIP(hipGetLastError());
+  const int cur = w->cur, n_pairs = w->n_pairs, n_old = w->n_pairs_old;
+  if ((st = small_find(w, true, iv, w->small_bail.p))) return st;
+  if ((st = wait_published(w, a.host, a.epoch))) return st;
+  if (a.host[1]) {
+    // outgrown: nothing was done; the launches take this step and the next ones
+    w->cur = cur;
+    w->n_pairs = n_pairs;
+    w->n_pairs_old = n_old;
+    w->small_holdoff = 64;
+    return B2G_OK;
+  }
+  const int* counts = a.host + 6;
+  w->n_touch = a.host[3];
+  w->n_colors = a.host[4];
+  w->h_color_off.assign(1, 0);
+  for (int i = 0; i < kMaxColors; ++i)
+    if (counts[i]) w->h_color_off.push_back(w->h_color_off.back() + counts[i]);
+  if (reuse) w->reuse_rounds = a.host[5];
+  w->color_rounds_used = a.host[5];
+  note_colours(w, reuse);
+  w->n_bins = 0;
+  w->solve_groups = w->n_touch > 0 ? 1 : 0;
+  w->pos_iters_run = pos_iters;
+  w->manifolds_valid[w->cur] = false;
+  w->collide_pending = true;
+  *done = true;
   return B2G_OK;
 }
 

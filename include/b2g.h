@@ -153,7 +153,8 @@ typedef struct b2g_profile {
   float step, collide, solve, broadphase; /* milliseconds, device time */
   int32_t pairs, touching, colours, islands, position_iterations;
   int32_t toi_events; /* continuous collision: TOI events solved in the step */
-  int32_t island_bins; /* island solve: bins of the last solve (0: per-colour or per-world launches) */
+  int32_t island_bins; /* island solve: bins of the last solve (0: per-colour or per-world launches, or a
+                         small world solved as one group) */
   int32_t pad;
 } b2g_profile;
 
