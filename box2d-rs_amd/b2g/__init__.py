@@ -497,10 +497,13 @@ class World:
     def broadphase_pairs(self, fat):
         fat = np.ascontiguousarray(fat, np.float32).reshape(-1, 4)
         cnt = ctypes.c_int64()
-        _check(_lib.b2g_broadphase_pairs(self._h, _ptr(fat), 0, None, ctypes.byref(cnt)))
-        out = np.zeros((max(cnt.value, 1), 2), np.int32)
-        _check(_lib.b2g_broadphase_pairs(self._h, _ptr(fat), cnt.value, _ptr(out), ctypes.byref(cnt)))
-        return out[:cnt.value]
+        # one search where its pairs fit into eight per proxy (a packed heap has three to four)
+        out = np.empty((max(8 * len(fat), 1), 2), np.int32)
+        _check(_lib.b2g_broadphase_pairs(self._h, _ptr(fat), len(out), _ptr(out), ctypes.byref(cnt)))
+        if cnt.value > len(out):
+            out = np.empty((cnt.value, 2), np.int32)
+            _check(_lib.b2g_broadphase_pairs(self._h, _ptr(fat), cnt.value, _ptr(out), ctypes.byref(cnt)))
+        return out[:cnt.value].copy()
 
 
 # ---- reference-style API ---------------------------------------------------------------------

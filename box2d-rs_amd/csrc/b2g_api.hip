@@ -235,6 +235,7 @@ static int add_items(World* w, int nbn, const b2g_body_def* bodies, const int32_
     if (fixtures[k].is_sensor) ++w->n_sensors;
     w->h_fshape.push_back(
         make_int4(s.type | (s.count << 8) | (s.one_sided << 16), 0, radius_bits, fixtures[k].is_sensor ? 1 : 0));
+    w->h_ftype.push_back(static_cast<unsigned char>(w->h_fshape.back().x & 0xff));
     w->h_fmat.push_back(make_float4(fd.friction, fd.restitution, fd.restitution_threshold, 0.0f));
     w->h_ffilter.push_back(make_int2(int(fd.category_bits) | (int(fd.mask_bits) << 16), fd.group_index));
     w->h_fworld.push_back(w->h_bworld[b]);
@@ -274,6 +275,64 @@ static int down(std::vector<T>& h, const DevArray<T>& d, size_t n, hipStream_t s
   h.resize(n);
   if (n) B2G_HIP(hipMemcpyAsync(h.data(), d.p, sizeof(T) * n, hipMemcpyDeviceToHost, s));
   return B2G_OK;
+}
+
+// ---- staged transfers --------------------------------------------------------------------------
+int stage_reserve(World* w) {
+  int st;
+  if (w->stage) return B2G_OK;
+  if ((st = w->stage_done.reserve(2))) return st;
+  B2G_HIP(hipMemsetAsync(w->stage_done.p, 0, 2 * sizeof(int), w->stream));
+  B2G_HIP(hipHostMalloc(reinterpret_cast<void**>(&w->stage), 2 * kStageBytes, hipHostMallocMapped | hipHostMallocCoherent));
+  return B2G_OK;
+}
+void stage_release(World* w) {
+  if (w->stage) (void)hipHostFree(w->stage);
+  w->stage = nullptr;
+  w->stage_done.release();
+}
+
+// The bodies' arrays and b2g_body_state records, four float4 each. A block's records go through LDS, so
+// that the accesses over the bus are whole lines (it bounds these kernels: 64 bytes a body).
+struct StateArrays {
+  float4 *xf, *pos, *vel, *pos0;
+  int* awake;
+  float* sleep_time;
+  const int* type;
+};
+static_assert(sizeof(b2g_body_state) == 4 * sizeof(float4), "a body state is four float4");
+__global__ void __launch_bounds__(kBlock) k_pack_states(int b0, int n, StateArrays s, float4* __restrict__ out,
+                                                        StagePub pub) {
+  __shared__ float4 rec[4 * kBlock];
+  const int t = threadIdx.x, first = blockIdx.x * kBlock, m = min(kBlock, n - first), b = b0 + first + t;
+  if (t < m) {
+    const float4 p = s.pos[b], v = s.vel[b], p0 = s.pos0[b];
+    rec[4 * t] = s.xf[b];
+    rec[4 * t + 1] = make_float4(p.x, p.y, p.z, v.x);
+    rec[4 * t + 2] = make_float4(v.y, v.z, p0.x, p0.y);
+    rec[4 * t + 3] = make_float4(p0.z, s.sleep_time[b], s.awake[b] ? 1.0f : 0.0f, 0.0f);
+  }
+  __syncthreads();
+  for (int e = t; e < 4 * m; e += kBlock) out[4 * first + e] = rec[e];
+  stage_publish(pub);
+}
+__global__ void __launch_bounds__(kBlock) k_unpack_states(int b0, int n, const float4* __restrict__ in, StateArrays s,
+                                                          StagePub pub) {
+  __shared__ float4 rec[4 * kBlock];
+  const int t = threadIdx.x, first = blockIdx.x * kBlock, m = min(kBlock, n - first), b = b0 + first + t;
+  for (int e = t; e < 4 * m; e += kBlock) rec[e] = in[4 * first + e];
+  __syncthreads();
+  if (t < m) {
+    const float4 q1 = rec[4 * t + 1], q2 = rec[4 * t + 2], q3 = rec[4 * t + 3];
+    s.xf[b] = rec[4 * t];
+    s.pos[b] = make_float4(q1.x, q1.y, q1.z, 0.0f);
+    s.vel[b] = make_float4(q1.w, q2.x, q2.y, 0.0f);
+    s.pos0[b] = make_float4(q2.z, q2.w, q3.x, 0.0f);
+    const bool dynamic = s.type[b] != B2G_STATIC;
+    s.awake[b] = dynamic && q3.z != 0.0f ? 1 : 0;
+    s.sleep_time[b] = dynamic ? q3.y : 0.0f;
+  }
+  stage_publish(pub);
 }
 
 // pulls the device-owned dynamic state into the host mirrors
@@ -657,6 +716,8 @@ int b2g_world_destroy(b2g_world* h) {
   rel(bp.keys); rel(bp.keys_alt); rel(bp.vals); rel(bp.vals_alt); rel(bp.hist); rel(bp.seg); rel(bp.nodes); rel(bp.nodes4);
   rel(bp.leafrec); rel(bp.count); rel(bp.slots); rel(bp.bounds); rel(bp.scan_tmp); rel(bp.scan_state); rel(bp.scan_ctl); bp.scan_epoch = 0; bp.scan_ctl_ready = false;
   rel(w->counters); rel(w->small_bail);
+  stage_release(w);
+  rel(w->query_fat); rel(w->query_set.pair); rel(w->query_set.off);
   if (w->h_counters) (void)hipHostFree(w->h_counters);
   for (int i = 0; i < 8; ++i)
     if (w->ev[i]) (void)hipEventDestroy(w->ev[i]);
@@ -813,58 +874,47 @@ int b2g_world_get_body_states(b2g_world* h, b2g_body_state* out, int32_t n) {
   World* w = &h->w;
   int st;
   if ((st = ensure_uploaded(w))) return st;
-  std::vector<float4> pos, vel, pos0, xf;
-  std::vector<int> awake;
-  std::vector<float> sleep_time;
-  if ((st = down(pos, w->b.pos, n, w->stream)) || (st = down(vel, w->b.vel, n, w->stream)) ||
-      (st = down(pos0, w->b.pos0, n, w->stream)) || (st = down(xf, w->b.xf, n, w->stream)) ||
-      (st = down(awake, w->b.awake, n, w->stream)) || (st = down(sleep_time, w->b.sleep_time, n, w->stream)))
-    return st;
-  B2G_HIP(hipStreamSynchronize(w->stream));
-  for (int i = 0; i < n; ++i) {
-    b2g_body_state& s = out[i];
-    s.p[0] = xf[i].x; s.p[1] = xf[i].y; s.q[0] = xf[i].z; s.q[1] = xf[i].w;
-    s.c[0] = pos[i].x; s.c[1] = pos[i].y; s.a = pos[i].z;
-    s.v[0] = vel[i].x; s.v[1] = vel[i].y; s.w = vel[i].z;
-    s.c0[0] = pos0[i].x; s.c0[1] = pos0[i].y; s.a0 = pos0[i].z;
-    s.sleep_time = sleep_time[i];
-    s.awake = awake[i] ? 1.0f : 0.0f;
-    s.pad = 0.0f;
-  }
-  return B2G_OK;
+  const StateArrays s{w->b.xf.p, w->b.pos.p, w->b.vel.p, w->b.pos0.p, w->b.awake.p, w->b.sleep_time.p, w->b.type.p};
+  return staged(
+      w, n, kStageBytes / sizeof(b2g_body_state), [](size_t, size_t, unsigned char*) {},
+      [&](int i0, int m, unsigned char* buf, const StagePub& pub) {
+        hipLaunchKernelGGL(k_pack_states, dim3(blocks_for(m, kBlock)), dim3(kBlock), 0, w->stream, i0, m, s,
+                           reinterpret_cast<float4*>(buf), pub);
+      },
+      [&](size_t i0, size_t m, unsigned char* buf) { std::memcpy(out + i0, buf, m * sizeof(b2g_body_state)); });
 }
 
+// (The host copies of the bodies' states are brought up to date from the device before they are read, except for
+// static bodies', which toi_note_statics looks at.)
 int b2g_world_set_body_states(b2g_world* h, const b2g_body_state* in, int32_t n) {
   if (!h || !in || n != h->w.nb) { set_error("b2g_world_set_body_states: invalid argument"); return B2G_ERR_INVALID_ARGUMENT; }
   World* w = &h->w;
   int st;
   if ((st = ensure_uploaded(w))) return st;
-  std::vector<float4> pos(n), vel(n), pos0(n), xf(n);
-  std::vector<int> awake(n);
-  std::vector<float> sleep_time(n);
-  for (int i = 0; i < n; ++i) {
-    const b2g_body_state& s = in[i];
-    pos[i] = make_float4(s.c[0], s.c[1], s.a, 0.0f);
-    vel[i] = make_float4(s.v[0], s.v[1], s.w, 0.0f);
-    pos0[i] = make_float4(s.c0[0], s.c0[1], s.a0, 0.0f);
-    xf[i] = make_float4(s.p[0], s.p[1], s.q[0], s.q[1]);
-    const bool non_static = w->host_type[i] != B2G_STATIC;
-    awake[i] = non_static && s.awake != 0.0f ? 1 : 0;
-    sleep_time[i] = non_static ? s.sleep_time : 0.0f;
-    if (non_static && !awake[i]) w->created_asleep = true;
+  const StateArrays s{w->b.xf.p, w->b.pos.p, w->b.vel.p, w->b.pos0.p, w->b.awake.p, w->b.sleep_time.p, w->b.type.p};
+  bool asleep = false;
+  st = staged(
+      w, n, kStageBytes / sizeof(b2g_body_state),
+      [&](size_t i0, size_t m, unsigned char* buf) {
+        std::memcpy(buf, in + i0, m * sizeof(b2g_body_state));
+        const b2g_body_state* r = in + i0;
+        const int* type = w->host_type.data() + i0;
+        for (size_t i = 0; i < m; ++i) asleep |= type[i] != B2G_STATIC && !(r[i].awake != 0.0f);
+      },
+      [&](int i0, int m, unsigned char* buf, const StagePub& pub) {
+        hipLaunchKernelGGL(k_unpack_states, dim3(blocks_for(m, kBlock)), dim3(kBlock), 0, w->stream, i0, m,
+                           reinterpret_cast<const float4*>(buf), s, pub);
+      },
+      [](size_t, size_t, unsigned char*) {});
+  if (st) return st;
+  if (asleep) w->created_asleep = true;
+  for (int b : w->static_bodies) {
+    w->h_pos[b] = make_float4(in[b].c[0], in[b].c[1], in[b].a, 0.0f);
+    w->h_vel[b] = make_float4(in[b].v[0], in[b].v[1], in[b].w, 0.0f);
+    w->h_pos0[b] = make_float4(in[b].c0[0], in[b].c0[1], in[b].a0, 0.0f);
+    w->h_xf[b] = make_float4(in[b].p[0], in[b].p[1], in[b].q[0], in[b].q[1]);
   }
-  if ((st = up(w->b.pos, pos, w->stream)) || (st = up(w->b.vel, vel, w->stream)) ||
-      (st = up(w->b.pos0, pos0, w->stream)) || (st = up(w->b.xf, xf, w->stream)) ||
-      (st = up(w->b.awake, awake, w->stream)) || (st = up(w->b.sleep_time, sleep_time, w->stream)))
-    return st;
-  B2G_HIP(hipStreamSynchronize(w->stream));
-  w->h_pos = pos;
-  w->h_vel = vel;
-  w->h_pos0 = pos0;
-  w->h_xf = xf;
-  w->h_awake = awake;
-  w->h_sleep_time = sleep_time;
-  toi_note_bodies(w);
+  toi_note_statics(w);
   return B2G_OK;
 }
 

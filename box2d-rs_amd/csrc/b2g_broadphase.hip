@@ -17,6 +17,8 @@
 // grouped by emitter and deterministic; each new pair finds its predecessor in the previous
 // step's segment of either of its proxies (the emitter of a pair changes when the two proxies
 // swap places in the Morton order). Pairs are stored as (emitter, other).
+#include <cstring>
+
 #include "b2g_internal.h"
 
 namespace b2g {
@@ -648,33 +650,32 @@ int phase_broadphase_general(World* w) {
   return B2G_OK;
 }
 
-int broadphase_pairs_for(World* w, const float* fat_host, int64_t cap, int32_t* out, int64_t* count) {
-  int np = w->np;
-  DevArray<float4> fat;
-  int st;
-  if ((st = fat.reserve(std::max(np, 1)))) return st;
-  B2G_HIP(hipMemcpyAsync(fat.p, fat_host, sizeof(float4) * np, hipMemcpyHostToDevice, w->stream));
-  ContactArrays tmp;
-  int n = 0;
-  st = find_pairs(w, fat.p, np, tmp, &n);
-  if (st == B2G_OK) {
-    *count = n;
-    int64_t m = std::min<int64_t>(cap, n);
-    if (m > 0) {
-      if (hipMemcpyAsync(out, tmp.pair.p, sizeof(int2) * m, hipMemcpyDeviceToHost, w->stream) != hipSuccess ||
-          hipStreamSynchronize(w->stream) != hipSuccess) {
-        set_error("broadphase pair readback failed");
-        st = B2G_ERR_DEVICE;
-      } else {
-        for (int64_t i = 0; i < m; ++i)  // report as (lower, higher) fixture index
-          if (out[2 * i] > out[2 * i + 1]) std::swap(out[2 * i], out[2 * i + 1]);
-      }
-    }
+// pairs as (lower, higher) fixture index, to a stage
+__global__ void __launch_bounds__(kBlock) k_ordered_pairs(int n, const int2* __restrict__ pairs, int2* __restrict__ out,
+                                                          StagePub pub) {
+  const int k = blockIdx.x * kBlock + threadIdx.x;
+  if (k < n) {
+    const int2 p = pairs[k];
+    out[k] = make_int2(min(p.x, p.y), max(p.x, p.y));
   }
-  tmp.pair.release();
-  tmp.off.release();
-  fat.release();
-  return st;
+  stage_publish(pub);
+}
+
+int broadphase_pairs_for(World* w, const float* fat_host, int64_t cap, int32_t* out, int64_t* count) {
+  const int np = w->np;
+  int n = 0, st;
+  if ((st = w->query_fat.reserve(std::max(np, 1)))) return st;
+  B2G_HIP(hipMemcpyAsync(w->query_fat.p, fat_host, sizeof(float4) * np, hipMemcpyHostToDevice, w->stream));
+  if ((st = find_pairs(w, w->query_fat.p, np, w->query_set, &n))) return st;
+  *count = n;
+  return staged(
+      w, static_cast<size_t>(std::min<int64_t>(cap, n)), kStageBytes / sizeof(int2),
+      [](size_t, size_t, unsigned char*) {},
+      [&](int i0, int m, unsigned char* buf, const StagePub& pub) {
+        hipLaunchKernelGGL(k_ordered_pairs, dim3(blocks_for(m, kBlock)), dim3(kBlock), 0, w->stream, m,
+                           w->query_set.pair.p + i0, reinterpret_cast<int2*>(buf), pub);
+      },
+      [&](size_t i0, size_t m, unsigned char* buf) { std::memcpy(out + 2 * i0, buf, sizeof(int2) * m); });
 }
 
 // ---- small worlds -------------------------------------------------------------------------------

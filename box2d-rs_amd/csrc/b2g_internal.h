@@ -326,6 +326,7 @@ struct World {
   std::vector<int> h_fbody;
   std::vector<float> h_fdensity;
   std::vector<int4> h_fshape;
+  std::vector<unsigned char> h_ftype;  // the shape types of h_fshape alone (check_given_pairs)
   std::vector<float4> h_fmat, h_ffat, h_faabb;
   std::vector<int2> h_ffilter;
   std::vector<int> h_bworld, h_fworld;  // world id per body / per proxy
@@ -384,7 +385,8 @@ struct World {
   // colouring (4 counters, 128 colour counts, last round, large-island constraints),
   // [kPinnedPairFlags, +4) the pair search's flags and total, [kPinnedColourOffsets, +385) the
   // colour offsets uploaded for the solve, [kPinnedToi, +8) the counters of a separable TOI pass,
-  // [kPinnedSmall, +134) and [kPinnedFind, +6) what the small-world kernels publish
+  // [kPinnedSmall, +134) and [kPinnedFind, +6) what the small-world kernels publish,
+  // [kPinnedStage, +2) the last transfer through each half of the stage
   int* h_counters = nullptr;
   int n_touch = 0, n_colors = 0, n_islands = 0;
   int color_rounds = 16;       // colouring rounds launched before the first readback
@@ -404,6 +406,13 @@ struct World {
   int island_solve = -1;
   int bin_threads = 256;
   int n_bins = 0;  // bins of the last solve
+  // staged transfers (staged()): two pinned halves of kStageBytes, and the blocks done with each
+  unsigned char* stage = nullptr;
+  DevArray<int> stage_done;
+  // b2g_broadphase_pairs' boxes and pair list
+  DevArray<float4> query_fat;
+  ContactArrays query_set;
+  std::vector<int> static_bodies;  // (toi_note_bodies)
   int publish_epoch = 0;   // value of the last published word (pinned memory)
   int small_holdoff = 0;   // steps for which the small-world kernels are left alone after a world outgrew them
   int solve_groups = 0;  // groups per colour of the last solve's constraints (s.cw_off); 0: not grouped
@@ -436,7 +445,7 @@ struct World {
 };
 
 constexpr int kPinnedInts = 1024, kPinnedPairFlags = 192, kPinnedColourOffsets = 256, kPinnedToi = 768,
-              kPinnedSmall = 800, kPinnedFind = 944;
+              kPinnedSmall = 800, kPinnedFind = 944, kPinnedStage = 960;
 
 // Capacity floor of the arrays sized by the contact set (the pairs, and the solver's arrays,
 // which the pairs bound): reserving for a multiple of the proxy count from the first step keeps a
@@ -544,8 +553,60 @@ bool small_find_fits(const World* w);
 int small_find(World* w, bool sync, IslandView iv, const int* bail);
 // waits until the word at `flag` (pinned, written by a kernel) is `value`
 int wait_published(World* w, const int* flag, int value);
+// Host transfers without pageable copies: pinned staging memory that kernels read and write themselves,
+// packing and unpacking the caller's records on the way. A copy of pageable memory costs the
+// runtime 15 us and an allocation as much again, and six arrays were six of them: the states of two bodies
+// took 79 us, of 393,216 3.6 ms (with the host's loop over them); now 12 us and 1.5 ms. (A
+// single large array that needs no packing is copied as fast by the runtime.)
+constexpr size_t kStageBytes = size_t(1) << 20;  // a half; small enough that the host's copy of one
+                                                 // half and the kernel on the other overlap
+struct StagePub {  // the kernel's last block publishes `epoch`
+  int* done;
+  int* flag;
+  int epoch;
+};
+#ifdef __HIPCC__
+__device__ inline void stage_publish(const StagePub& p) {
+  __threadfence_system();
+  __syncthreads();
+  if (threadIdx.x == 0 && atomicAdd(p.done, 1) == static_cast<int>(gridDim.x) - 1) {
+    *p.done = 0;
+    __threadfence_system();
+    __hip_atomic_store(p.flag, p.epoch, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+  }
+}
+#endif
+int stage_reserve(World* w);
+void stage_release(World* w);
+// `items` in chunks of `per` (their records fit in kStageBytes): fill(i0, n, half) on the host, then
+// launch(i0, n, half, pub), which ends with stage_publish, then drain(i0, n, half) on the host
+template <class Fill, class Launch, class Drain>
+int staged(World* w, size_t items, size_t per, Fill&& fill, Launch&& launch, Drain&& drain) {
+  int st;
+  if ((st = stage_reserve(w))) return st;
+  int epoch[2] = {0, 0};
+  const size_t chunks = (items + per - 1) / per;
+  for (size_t c = 0; c < chunks + 2; ++c) {
+    const int half = static_cast<int>(c & 1);
+    unsigned char* buf = w->stage + half * kStageBytes;
+    int* flag = w->h_counters + kPinnedStage + half;
+    if (c >= 2 && c - 2 < chunks) {
+      if ((st = wait_published(w, flag, epoch[half]))) return st;
+      const size_t i0 = (c - 2) * per;
+      drain(i0, std::min(per, items - i0), buf);
+    }
+    if (c >= chunks) continue;
+    const size_t i0 = c * per, n = std::min(per, items - i0);
+    fill(i0, n, buf);
+    epoch[half] = ++w->publish_epoch;
+    launch(static_cast<int>(i0), static_cast<int>(n), buf, StagePub{w->stage_done.p + half, flag, epoch[half]});
+    B2G_HIP(hipGetLastError());
+  }
+  return B2G_OK;
+}
 int phase_toi(World* w, float dt, int vi);  // continuous collision after the solve
 void toi_note_bodies(World* w);             // has_kinematic, has_bullet and statics_still from the host mirrors
+void toi_note_statics(World* w);  // after the static bodies' states changed
 int toi_carry_state(World* w);              // TOI state of the previous contact set onto the current one
 void release_solve_graphs(World* w);
 // primitives

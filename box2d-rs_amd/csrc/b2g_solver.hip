@@ -2736,7 +2736,7 @@ int wait_published(World* w, const int* flag, int value) {
     const hipError_t e = hipStreamQuery(w->stream);
     if (e == hipErrorNotReady) continue;
     if (e == hipSuccess && __atomic_load_n(flag, __ATOMIC_ACQUIRE) == value) return B2G_OK;
-    set_error(std::string("a small-world kernel did not publish its result: ") + hipGetErrorString(e));
+    set_error(std::string("a kernel did not publish its result: ") + hipGetErrorString(e));
     return B2G_ERR_DEVICE;
   }
 }

@@ -1630,11 +1630,18 @@ int toi_carry_state(World* w) {
 
 void toi_note_bodies(World* w) {
   w->has_kinematic = w->has_bullet = false;
-  w->statics_still = true;
+  w->static_bodies.clear();
   for (int b = 0; b < w->nb; ++b) {
     w->has_bullet = w->has_bullet || w->h_bullet[b] != 0;
     if (w->host_type[b] == B2G_KINEMATIC) w->has_kinematic = true;
-    if (w->host_type[b] != B2G_STATIC) continue;
+    if (w->host_type[b] == B2G_STATIC) w->static_bodies.push_back(b);
+  }
+  toi_note_statics(w);
+}
+
+void toi_note_statics(World* w) {
+  w->statics_still = true;
+  for (int b : w->static_bodies) {
     const float4 p = w->h_pos[b], p0 = w->h_pos0[b], v = w->h_vel[b], m = w->h_mass[b];
     w->statics_still = w->statics_still && p.x == p0.x && p.y == p0.y && p.z == p0.z && v.x == 0.0f && v.y == 0.0f &&
                        v.z == 0.0f && m.x == 0.0f && m.y == 0.0f;

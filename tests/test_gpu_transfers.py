@@ -1,0 +1,87 @@
+"""Staged transfers (pinned memory that kernels read and write in chunks of 1 MiB): body states (and boxes)
+come back as they were set, at one record, a block and a chunk of records and one to each side of them, over
+several chunks; manifolds of given pairs equal those of the entry point without staging, byte for byte;
+pair lists of several chunks equal the pairs found on the host.
+"""
+import numpy as np
+import pytest
+
+import b2g
+
+pytestmark = pytest.mark.gpu
+
+STATES = 16384  # records of a chunk
+PAIRS = 9216
+
+
+def _world(n, circles=True):
+    rng = np.random.default_rng(n)
+    bd = np.zeros(n, b2g.BODY_DEF)
+    bd["type"] = rng.choice([0, 1, 2, 2], n)
+    bd["awake"] = bd["allow_sleep"] = 1
+    bd["position"][:, 0] = np.arange(n)
+    sd = np.zeros(n, b2g.SHAPE_DEF)
+    sd["radius"] = 0.4
+    if not circles:
+        sd["type"] = b2g.SHAPE_BOX
+        sd["radius"] = 0.0
+        sd["params"][:, :2] = rng.uniform(0.2, 0.5, (n, 2))
+    fd = np.zeros(n, b2g.FIXTURE_DEF)
+    fd["density"], fd["category"], fd["mask"] = 1.0, 1, 0xFFFF
+    w = b2g.World()
+    w.add(bd, np.arange(n, dtype=np.int32), sd, fd)
+    return w, bd, rng
+
+
+@pytest.mark.parametrize("n", [1, 255, 256, 257, STATES - 1, STATES, STATES + 1, 3 * STATES + 7])
+def test_states_and_boxes_come_back_as_set(n):
+    w, bd, rng = _world(n)
+    for _ in range(2):  # the second call over the first's chunks
+        st = w.body_states()
+        for name in ("p", "q", "c", "a", "v", "w", "c0", "a0", "sleep_time"):
+            st[name] = rng.normal(size=st[name].shape)
+        st["awake"] = rng.integers(0, 2, n)
+        w.set_body_states(st)
+        static = bd["type"] == 0
+        st["sleep_time"][static] = 0.0
+        st["awake"][static] = 0.0
+        assert w.body_states().tobytes() == st.tobytes()
+        fat = rng.normal(size=(n, 4)).astype(np.float32)
+        w.set_fat_aabbs(fat)
+        assert w.fat_aabbs().tobytes() == fat.tobytes()
+    w.close()
+
+
+@pytest.mark.parametrize("n", [1, 257, PAIRS - 1, PAIRS, PAIRS + 1, 2 * PAIRS + 300])
+def test_given_pairs_match_the_entry_point_without_staging(n):
+    w, bd, rng = _world(500, circles=False)
+    w.body_states()
+    pairs = rng.integers(0, 500, (n, 2)).astype(np.int32)
+    xf = []
+    for _ in range(2):
+        a = rng.uniform(-3.0, 3.0, n)
+        xf.append(np.stack([rng.uniform(0.0, 0.6, n), rng.uniform(0.0, 0.6, n), np.sin(a), np.cos(a)], 1).astype(np.float32))
+    got = w.collide_pairs(pairs, *xf)
+    ref = np.concatenate([w.collide_pairs_noalloc(pairs[i:i + 4000], xf[0][i:i + 4000], xf[1][i:i + 4000])
+                          for i in range(0, n, 4000)])
+    assert (got["point_count"] > 0).any()
+    assert got.tobytes() == ref.tobytes()
+    w.close()
+
+
+@pytest.mark.parametrize("n,close", [(2, 3.0), (600, 400.0), (5000, 60.0)])
+def test_pair_lists_match_the_host(n, close):
+    """close: pairs per proxy, up to more than eight per proxy (a second search) and several chunks of pairs."""
+    w, bd, rng = _world(n)
+    side = max(1.0, np.sqrt(4.0 * n / close))
+    c = rng.uniform(0.0, side, (n, 2)) if n > 2 else np.zeros((n, 2))
+    fat = np.concatenate([c - 1.0, c + 1.0], 1).astype(np.float32)
+    i, j = np.triu_indices(n, 1)
+    hit = ((fat[i, :2] <= fat[j, 2:]) & (fat[j, :2] <= fat[i, 2:])).all(1)
+    hit &= (bd["type"][i] == 2) | (bd["type"][j] == 2)
+    want = np.stack([i[hit], j[hit]], 1)
+    got = w.broadphase_pairs(fat)
+    assert (got[:, 0] < got[:, 1]).all()
+    got = got[np.lexsort((got[:, 1], got[:, 0]))]
+    assert np.array_equal(got, want)
+    w.close()
