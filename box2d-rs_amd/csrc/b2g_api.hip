@@ -724,6 +724,7 @@ int b2g_world_destroy(b2g_world* h) {
   for (hipEvent_t e : w->kt.ev) (void)hipEventDestroy(e);
   tape_release(w);
   release_solve_graphs(w);
+  release_side_streams(w);
   if (w->stream) (void)hipStreamDestroy(w->stream);
   delete h;
   return B2G_OK;

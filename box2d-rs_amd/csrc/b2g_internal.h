@@ -400,7 +400,9 @@ struct World {
   // world_solve: -1 auto (on when the batch has at least kWorldSolveMin worlds), 0 off, 1 on.
   // world_threads[k]: threads per world for the worlds of body-count bucket k (see world_bucket).
   int world_solve = -1;
-  int world_threads[3] = {64, 128, 256};
+  int world_threads[3] = {64, 256, 512};
+  hipStream_t side[2] = {nullptr, nullptr};  // the smaller buckets' (fork_buckets)
+  hipEvent_t side_fork = nullptr, side_join[2] = {nullptr, nullptr};
   // island_solve: -1 auto (on unless the per-world solve is), 0 off, 1 on; bin_threads: threads per
   // bin (islands of at most bin_threads / 2 constraints are binned)
   int island_solve = -1;
@@ -546,6 +548,7 @@ int phase_synchronize(World* w); // swept + fat AABBs of non-static proxies
 struct IslandView;
 // Small worlds (b2g_world_step): a step's solve in one launch and its pair search in three
 constexpr int kSmallBodies = 2048, kSmallTree = 2048, kSmallProxies = 4096, kSmallPairs = 4096, kSmallTouch = 2048;
+void release_side_streams(World* w);
 bool small_step_fits(const World* w);
 // runs the solve and find_new_contacts; *done false: the world did not fit after all and nothing was done
 int small_step(World* w, float dt, float dt_ratio, int vel_iters, int pos_iters, bool* done);

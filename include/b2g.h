@@ -401,15 +401,15 @@ enum {
  *                           deterministic; the colour order it gives is the Gauss-Seidel order.
  *   B2G_TUNE_WORLD_SOLVE    batched worlds (b2g_world_add_batched): 1 solves the velocity and the
  *                           position iterations of each world in one workgroup per world, colour
- *                           after colour with workgroup barriers (two launches per step instead of
- *                           one per colour and iteration); 0 launches per colour; -1 (default) is 1
+ *                           after colour with workgroup barriers (a launch per size of worlds
+ *                           instead of one per colour and iteration); 0 launches per colour; -1 (default) is 1
  *                           for batches of at least 16 worlds whose bodies are contiguous per world
  *                           and that have no joints. The constraint order is the colour order
  *                           either way, so the results are the same bit for bit.
  *   B2G_TUNE_WORLD_THREADS_SMALL / _MEDIUM / _LARGE
  *                           threads per world (64, 128, 256 or 512) in that solve for worlds of
- *                           fewer than 64 bodies / 64-255 bodies / 256 or more (defaults 64, 128,
- *                           256; box2d-rs_amd/b2g/autotune.py sweeps them).
+ *                           fewer than 64 bodies / 64-255 bodies / 256 or more (defaults 64, 256,
+ *                           512; box2d-rs_amd/b2g/autotune.py sweeps them).
  *   B2G_TUNE_ISLAND_SOLVE   1: islands of at most B2G_TUNE_ISLAND_THREADS / 2 constraints are packed
  *                           into bins, and one workgroup per bin runs all velocity (and all position)
  *                           iterations of its islands, colour after colour with workgroup barriers,
