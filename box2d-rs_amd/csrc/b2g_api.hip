@@ -525,7 +525,9 @@ int upload_world(World* w) {
     w->n_tree = int(tree.size());
     w->tree_statics = false;
     for (int f : tree) w->tree_statics = w->tree_statics || host_is_static(w, f);
-    if ((st = up(w->f.tree_list, tree, w->stream)) || (st = up(w->f.loose_off, loose_off, w->stream)) ||
+    w->h_in_tree.assign(w->np, 0);
+    for (int f : tree) w->h_in_tree[f] = 1;
+    if ((st = up(w->f.in_tree, w->h_in_tree, w->stream)) || (st = up(w->f.tree_list, tree, w->stream)) || (st = up(w->f.loose_off, loose_off, w->stream)) ||
         (st = up(w->f.loose, loose, w->stream)))
       return st;
   }
@@ -606,9 +608,8 @@ static int run_phase(World* w, int phase, float dt, int vi, int pi) {
   }
   if (phase == B2G_PHASE_FIND) {
     if (dt > 0.0f) {
-      if ((st = phase_synchronize(w))) return st;
       if ((st = carry_manifolds(w))) return st;
-      if ((st = phase_broadphase(w))) return st;
+      if ((st = phase_find(w))) return st;
       w->manifolds_valid[w->cur] = false;
       w->collide_pending = true;
       w->inv_dt0 = 1.0f / dt;
@@ -685,7 +686,7 @@ int b2g_world_destroy(b2g_world* h) {
   rel(w->b.pos); rel(w->b.vel); rel(w->b.pos0); rel(w->b.xf); rel(w->b.mass); rel(w->b.props); rel(w->b.force); rel(w->b.awake); rel(w->b.sleep_time); rel(w->b.auto_sleep); rel(w->b.wake);
   rel(w->b.type); rel(w->b.bullet);
   rel(w->f.body); rel(w->f.shape); rel(w->f.mat); rel(w->f.filter); rel(w->f.aabb); rel(w->f.fat); rel(w->f.moved);
-  rel(w->f.shapev); rel(w->f.world); rel(w->f.tree_list); rel(w->f.loose_off); rel(w->f.loose);
+  rel(w->f.shapev); rel(w->f.world); rel(w->f.tree_list); rel(w->f.in_tree); rel(w->f.loose_off); rel(w->f.loose);
   for (auto& c : w->c) {
     rel(c.pair); rel(c.off); rel(c.old_index); rel(c.ab); rel(c.hdr); rel(c.geo); rel(c.pt0); rel(c.pt1); rel(c.ids); rel(c.colour);
   }

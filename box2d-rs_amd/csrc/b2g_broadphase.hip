@@ -35,17 +35,12 @@ struct SyncArgs {
   int* moved;
   IslandView iv;
 };
-__device__ inline void synchronize_one(int i, const SyncArgs& a, int* any_moved) {
+__device__ inline void synchronize_one(int i, const SyncArgs& a) {
   int b = a.fbody[i];
   // only bodies of this step's islands are synchronised (src/private/dynamics/b2_world.rs:482-500)
   if (a.btype[b] == 0 || a.iv.asleep(b)) { a.moved[i] = 0; return; }
   if (!sync_proxy(i, b, a.shapes[i], a.pos0, a.bmass, a.bxf, a.faabb, a.ffat)) { a.moved[i] = 0; return; }
   a.moved[i] = 1;
-  if (any_moved) *any_moved = 1;  // every writer stores 1
-}
-__global__ void __launch_bounds__(kBlock) k_synchronize(int np, SyncArgs a, int* __restrict__ any_moved) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < np) synchronize_one(i, a, any_moved);
 }
 static SyncArgs sync_args(World* w, IslandView iv) {
   return SyncArgs{w->f.body.p, w->f.shapev.p, w->b.type.p, w->b.pos0.p, w->b.mass.p, w->b.xf.p,
@@ -53,11 +48,12 @@ static SyncArgs sync_args(World* w, IslandView iv) {
 }
 
 // ---- scene bounds and Morton codes ---------------------------------------------------------
-// The scene's extent for the Morton codes, in two steps without atomics: each block of k_bounds
-// writes the box of its proxies' fat-AABB centres to partial[block], and every block of k_morton
-// reduces those partial boxes itself before coding its proxies (min and max are exact, so the
-// result does not depend on the order). Block 0 also clears the pair search's flags.
-static constexpr int kBoundsBlocks = 256;  // most partial boxes (one per k_bounds block)
+// The scene's extent for the Morton codes, in two steps without atomics: each block of k_bounds (of
+// k_sync_bounds, which synchronises the proxies first) writes the box of its proxies' fat-AABB centres
+// to partial[block], and every block of k_morton reduces those partial boxes itself before coding its
+// proxies (min and max are exact, so the result does not depend on the order). Block 0 also clears the
+// pair search's flags.
+static constexpr int kBoundsBlocks = 2048;  // most partial boxes (32 KB, eight per thread of k_morton)
 __device__ inline void pair_flags_init(int* flags, const int* scan_ctl) {
   flags[0] = 0;                           // traversal stack overflow
   flags[1] = 0;                           // proxies whose pairs overflow their slots
@@ -86,6 +82,24 @@ __global__ void __launch_bounds__(kBlock) k_bounds(int n, const int* __restrict_
   for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
     float4 a = fat[list[i]];
     float cx = 0.5f * (a.x + a.z), cy = 0.5f * (a.y + a.w);
+    lx = fminf(lx, cx); ly = fminf(ly, cy); hx = fmaxf(hx, cx); hy = fmaxf(hy, cy);
+  }
+  block_box(lx, ly, hx, hy);
+  if (threadIdx.x == 0) partial[blockIdx.x] = make_float4(lx, ly, hx, hy);
+  if (blockIdx.x == 0 && threadIdx.x == 0) pair_flags_init(flags, scan_ctl);
+}
+
+// One proxy per thread (bound by the memory it touches: its body's state and its shape). The bounds in the
+// same launch: 65,536 proxies 7.9 + 4.9 us -> 9.0 us, 393,216 31.3 + 6.4 -> 33.1 us.
+__global__ void __launch_bounds__(kBlock) k_sync_bounds(int np, SyncArgs a, const unsigned char* __restrict__ in_tree,
+                                                        float4* __restrict__ partial, int* __restrict__ flags,
+                                                        const int* __restrict__ scan_ctl) {
+  float lx = kMaxFloat, ly = kMaxFloat, hx = -kMaxFloat, hy = -kMaxFloat;
+  for (int i = blockIdx.x * kBlock + threadIdx.x; i < np; i += gridDim.x * kBlock) {
+    synchronize_one(i, a);
+    if (!in_tree[i]) continue;
+    const float4 f = a.ffat[i];
+    const float cx = 0.5f * (f.x + f.z), cy = 0.5f * (f.y + f.w);
     lx = fminf(lx, cx); ly = fminf(ly, cy); hx = fmaxf(hx, cx); hy = fmaxf(hy, cy);
   }
   block_box(lx, ly, hx, hy);
@@ -127,24 +141,36 @@ __device__ inline unsigned morton_code(float4 a, float lx, float ly, float hx, f
 }
 
 // key = world id in the high bits, then a Morton code of `mbits` bits per axis of the fat-AABB
-// centre; sorting by it groups each world's proxies and orders them along a Z curve
-__global__ void __launch_bounds__(kBlock) k_morton(int n, const int* __restrict__ list, const float4* __restrict__ fat,
-                                                   const float4* __restrict__ partial, int nparts,
-                                                   const int* __restrict__ world, int mbits, unsigned* __restrict__ keys,
-                                                   unsigned* __restrict__ vals) {
+// centre; sorting by it groups each world's proxies and orders them along a Z curve. A block codes a
+// tile of the sort and counts the low digit's values on the way (the sort's first histogram).
+__global__ void __launch_bounds__(kSortBlock) k_morton(int n, const int* __restrict__ list,
+                                                       const float4* __restrict__ fat,
+                                                       const float4* __restrict__ partial, int nparts,
+                                                       const int* __restrict__ world, int mbits,
+                                                       unsigned* __restrict__ keys, unsigned* __restrict__ vals,
+                                                       unsigned* __restrict__ hist) {
+  static_assert(kSortBlock == kBlock && kSortBlock == kRadix, "one thread per digit");
+  __shared__ unsigned h[kRadix];
+  h[threadIdx.x] = 0;
   float lx = kMaxFloat, ly = kMaxFloat, hx = -kMaxFloat, hy = -kMaxFloat;
   for (int p = threadIdx.x; p < nparts; p += blockDim.x) {
     const float4 b = partial[p];
     lx = fminf(lx, b.x); ly = fminf(ly, b.y); hx = fmaxf(hx, b.z); hy = fmaxf(hy, b.w);
   }
-  block_box(lx, ly, hx, hy);
-  int k = blockIdx.x * blockDim.x + threadIdx.x;
-  if (k >= n) return;
-  const int i = list[k];
-  const unsigned code = morton_code(fat[i], lx, ly, hx, hy, mbits);
-  // indexed by list position: the sort runs over the n listed proxies
-  keys[k] = (unsigned(world[i]) << (2 * mbits)) | code;
-  vals[k] = unsigned(i);
+  block_box(lx, ly, hx, hy);  // (a barrier: h is clear)
+#pragma unroll
+  for (int e = 0; e < kSortItems; ++e) {
+    const int k = blockIdx.x * kSortTile + e * kSortBlock + threadIdx.x;
+    if (k >= n) break;
+    const int i = list[k];
+    const unsigned key = (unsigned(world[i]) << (2 * mbits)) | morton_code(fat[i], lx, ly, hx, hy, mbits);
+    // indexed by list position: the sort runs over the n listed proxies
+    keys[k] = key;
+    vals[k] = unsigned(i);
+    atomicAdd(&h[key & 0xffu], 1u);
+  }
+  __syncthreads();
+  hist[threadIdx.x * gridDim.x + blockIdx.x] = h[threadIdx.x];
 }
 
 // ---- BVH -------------------------------------------------------------------------------------
@@ -466,18 +492,6 @@ __global__ void __launch_bounds__(kTravBlock) k_traverse(int nq, const float4* _
   }
 }
 
-__global__ void __launch_bounds__(kBlock) k_pairs_from_slots(int nq, const int4* __restrict__ leafrec,
-                                                             const int* __restrict__ count,
-                                                             const int* __restrict__ slots, const int* __restrict__ off,
-                                                             int2* __restrict__ pairs) {
-  const int k = blockIdx.x * blockDim.x + threadIdx.x;
-  if (k >= nq) return;
-  const int q = leafrec[k].x;
-  const int c = min(count[q], kSlots);
-  const int o = off[q];
-  for (int j = 0; j < c; ++j) pairs[o + j] = make_int2(q, slots[size_t(j) * nq + k]);
-}
-
 // predecessor of each new pair in the previous contact set: the pair sits in the old segment of
 // one of its two proxies (its emitter then)
 __device__ inline int find_in_segment(int a, int b, int old_np, const int* __restrict__ old_off,
@@ -487,23 +501,93 @@ __device__ inline int find_in_segment(int a, int b, int old_np, const int* __res
     if (old_pairs[i].y == b) return i;
   return -1;
 }
-// (also clears the new set's solve colours: the solve of this set writes those of its touching
-// contacts)
-__global__ void __launch_bounds__(kBlock) k_merge(int n, const int2* __restrict__ pairs, int old_np,
-                                                  const int* __restrict__ old_off, const int2* __restrict__ old_pairs,
-                                                  int* __restrict__ old_index, int* __restrict__ colour) {
-  int k = blockIdx.x * blockDim.x + threadIdx.x;
-  if (k >= n) return;
-  colour[k] = -1;
-  int2 pr = pairs[k];
-  int found = find_in_segment(pr.x, pr.y, old_np, old_off, old_pairs);
-  if (found < 0) found = find_in_segment(pr.y, pr.x, old_np, old_off, old_pairs);
-  old_index[k] = found;
+// what the pairs of a new set are written to; old_index null: no predecessors (and no colours)
+struct PairOut {
+  int2* pairs;
+  int cap;
+  int* old_index;
+  int* colour;  // cleared: the solve of this set writes those of its touching contacts
+  int old_np;   // proxies when the old set was built (0: no old set)
+  const int* old_off;
+  const int2* old_pairs;
+};
+__device__ inline void pair_predecessor(int k, int2 pr, const PairOut& o) {
+  o.colour[k] = -1;
+  int found = find_in_segment(pr.x, pr.y, o.old_np, o.old_off, o.old_pairs);
+  if (found < 0) found = find_in_segment(pr.y, pr.x, o.old_np, o.old_off, o.old_pairs);
+  o.old_index[k] = found;
+}
+// The pairs from the walk's slots, a thread per query (slots are read whole lines at a time), then their
+// predecessors, a thread per pair: pairs are grouped by emitter, so neighbouring threads look at neighbouring
+// segments and write neighbouring words (one kernel by query for both: 15.2 -> 21.5 us at 393,216 proxies).
+// The host learns the total from the first thread while the kernels run (a copy and a wait less: 20 us a
+// step), so they only write if the set's arrays hold the pairs and no walk overflowed (flags[0], [1]) and
+// no scan failed ([2]); otherwise the host does what is left. `host` null: it is doing that.
+__device__ inline bool pairs_held(const int* __restrict__ flags, const PairOut& o) {
+  return flags[0] == 0 && flags[1] == 0 && flags[2] == 0 && flags[3] <= o.cap;
+}
+__global__ void __launch_bounds__(kBlock) k_emit_pairs(int nq, const int4* __restrict__ leafrec,
+                                                       const int* __restrict__ count, const int* __restrict__ slots,
+                                                       const int* __restrict__ off, PairOut o,
+                                                       const int* __restrict__ flags, int* host, int epoch) {
+  const int k = blockIdx.x * kBlock + threadIdx.x;
+  if (host && k == 0) {
+    for (int e = 0; e < 4; ++e) host[1 + e] = flags[e];
+    __threadfence_system();
+    __hip_atomic_store(host, epoch, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+  }
+  if (k >= nq || (host && !pairs_held(flags, o))) return;
+  const int q = leafrec[k].x, c = min(count[q], kSlots), first = off[q];
+  for (int j = 0; j < c; ++j) o.pairs[first + j] = make_int2(q, slots[size_t(j) * nq + k]);
+}
+__global__ void __launch_bounds__(kBlock) k_merge(PairOut o, const int* __restrict__ flags, int n) {
+  if (n < 0) {  // the host does not know the total yet
+    if (!pairs_held(flags, o)) return;
+    n = flags[3];
+  }
+  for (int k = blockIdx.x * kBlock + threadIdx.x; k < n; k += gridDim.x * kBlock) pair_predecessor(k, o.pairs[k], o);
 }
 
-// Pair search over the proxies' fat AABBs into contact set `dst` (pairs, offsets); returns the
-// pair count in *npairs. Does not touch manifolds.
-static int find_pairs(World* w, const float4* fat, int np, ContactArrays& dst, int* npairs) {
+static int reserve_contacts(World* w, ContactArrays& c, int pairs) {
+  int st;
+  const size_t n = pair_capacity(w, pairs);
+  if ((st = c.pair.reserve(n)) || (st = c.old_index.reserve(n)) || (st = c.ab.reserve(n)) || (st = c.hdr.reserve(n)) ||
+      (st = c.geo.reserve(n)) || (st = c.pt0.reserve(n)) || (st = c.pt1.reserve(n)) || (st = c.ids.reserve(n)) ||
+      (st = c.colour.reserve(n)))
+    return st;
+  return B2G_OK;
+}
+
+// where a search into `dst` writes its pairs; old: the set their predecessors are in (null: none wanted)
+static PairOut pair_out(World* w, ContactArrays& dst, const ContactArrays* old) {
+  return PairOut{dst.pair.p,
+                 static_cast<int>(old ? dst.colour.cap : dst.pair.cap),  // (a set's arrays are reserved together)
+                 old ? dst.old_index.p : nullptr, dst.colour.p, old ? w->set_np[w->cur] : 0, old ? old->off.p : nullptr,
+                 old ? old->pair.p : nullptr};
+}
+
+// what k_emit_pairs left to the host: a set that outgrew its arrays, or walks that overflowed their slots
+static int finish_pairs(World* w, const float4* fat, const TreeView& tv, const PairFilter& pf, ContactArrays& dst,
+                        const ContactArrays* old, int total, bool overflow, int* flags) {
+  BroadphaseArrays& bp = w->bp;
+  int st;
+  if ((st = old ? reserve_contacts(w, dst, total) : dst.pair.reserve(pair_capacity(w, total)))) return st;
+  const PairOut o = pair_out(w, dst, old);
+  const int nt = tv.n;
+  hipLaunchKernelGGL(k_emit_pairs, dim3(blocks_for(nt, kBlock)), dim3(kBlock), 0, w->stream, nt, bp.leafrec.p,
+                     bp.count.p, bp.slots.p, dst.off.p, o, flags, nullptr, 0);
+  if (overflow)
+    hipLaunchKernelGGL(k_traverse<true>, dim3(blocks_for(nt * kTravLanes, kTravBlock)), dim3(kTravBlock), 0, w->stream,
+                       nt, fat, tv, pf, bp.count.p, bp.slots.p, dst.off.p, dst.pair.p, flags, nullptr);
+  if (old) hipLaunchKernelGGL(k_merge, dim3(blocks_for(total, kBlock)), dim3(kBlock), 0, w->stream, o, flags, total);
+  B2G_HIP(hipGetLastError());
+  return B2G_OK;
+}
+
+// Pair search over the proxies' fat AABBs (after `sync`, if given) into contact set `dst` (pairs, offsets,
+// and with `old` their predecessors in that set); returns the pair count in *npairs. Does not touch manifolds.
+static int find_pairs(World* w, const float4* fat, int np, const SyncArgs* sync, ContactArrays& dst,
+                      const ContactArrays* old, int* npairs) {
   BroadphaseArrays& bp = w->bp;
   const int nt = w->n_tree;  // proxies in the tree (the others are big statics, tested directly)
   int st;
@@ -523,25 +607,30 @@ static int find_pairs(World* w, const float4* fat, int np, ContactArrays& dst, i
       (st = bp.nodes4.reserve(std::max(nt, 1))) ||
       (st = bp.leafrec.reserve(std::max(nt, 1))) ||
       (st = bp.count.reserve(np + 1)) || (st = bp.slots.reserve(size_t(np) * kSlots)) ||
-      (st = dst.off.reserve(np + 1)) || (st = bp.bounds.reserve(1 + kBoundsBlocks)))
+      (st = dst.off.reserve(np + 1)) || (st = bp.bounds.reserve(1 + kBoundsBlocks)) || (st = radix_reserve(w, std::max(nt, 1))) ||
+      (st = old ? reserve_contacts(w, dst, 0) : dst.pair.reserve(pair_capacity(w, 0))))
     return st;
   // bounds[0]: the pair search's flags ([0] stack overflow, [1] proxies with more pairs than
   // slots, [2] scan error, [3] pair total); bounds[1..]: k_bounds' partial boxes
   int* flags = reinterpret_cast<int*>(bp.bounds.p);
   float4* partial = bp.bounds.p + 1;
   const int* scan_ctl = static_cast<const int*>(bp.scan_ctl.p);
-  if (nt == 0) hipLaunchKernelGGL(k_pair_flags_init, dim3(1), dim3(1), 0, w->stream, flags, scan_ctl);
+  if (sync)
+    hipLaunchKernelGGL(k_sync_bounds, dim3(std::min(blocks_for(np, kBlock), kBoundsBlocks)), dim3(kBlock), 0, w->stream,
+                       np, *sync, w->f.in_tree.p, partial, flags, scan_ctl);
+  else if (nt == 0) hipLaunchKernelGGL(k_pair_flags_init, dim3(1), dim3(1), 0, w->stream, flags, scan_ctl);
   const int wbits = world_bits(w), mbits = morton_bits(w);
   const int key_bits = wbits + 2 * mbits;
   const bool nc = w->n_nocollide > 0;
   const LeafInputs li{w->f.body.p, w->b.type.p, w->f.filter.p, w->f.shape.p, nc ? w->j.nc_flag.p : nullptr};
   if (nt > 0) {
-    const int gb = std::min(blocks_for(nt, kBlock), kBoundsBlocks);
-    hipLaunchKernelGGL(k_bounds, dim3(gb), dim3(kBlock), 0, w->stream, nt, w->f.tree_list.p, fat, partial, flags,
-                       scan_ctl);
-    hipLaunchKernelGGL(k_morton, dim3(blocks_for(nt, kBlock)), dim3(kBlock), 0, w->stream, nt, w->f.tree_list.p, fat,
-                       partial, gb, w->f.world.p, mbits, bp.keys.p, bp.vals.p);
-    if ((st = radix_sort_pairs(w, bp.keys.p, bp.vals.p, nt, key_bits))) return st;
+    const int gb = std::min(blocks_for(sync ? np : nt, kBlock), kBoundsBlocks);
+    if (!sync)
+      hipLaunchKernelGGL(k_bounds, dim3(gb), dim3(kBlock), 0, w->stream, nt, w->f.tree_list.p, fat, partial, flags,
+                         scan_ctl);
+    hipLaunchKernelGGL(k_morton, dim3(blocks_for(nt, kSortTile)), dim3(kSortBlock), 0, w->stream, nt, w->f.tree_list.p,
+                       fat, partial, gb, w->f.world.p, mbits, bp.keys.p, bp.vals.p, bp.hist.p);
+    if ((st = radix_sort_pairs(w, bp.keys.p, bp.vals.p, nt, key_bits, true))) return st;
     for (int L0 = 0; L0 == 0 || L0 < lv.count - 1; L0 += kReduceLevels)
       hipLaunchKernelGGL(k_seg_reduce, dim3(blocks_for(lv.size[L0], kBlock)), dim3(kBlock), 0, w->stream, lv, L0,
                          bp.vals.p, fat, bp.seg.p, li, bp.leafrec.p);
@@ -565,89 +654,64 @@ static int find_pairs(World* w, const float4* fat, int np, ContactArrays& dst, i
   }
   // the pair total also lands beside the flags (flags[3]), so one read-back brings both
   if ((st = exclusive_scan(w, bp.count.p, dst.off.p, np, dst.off.p + np, flags + 3))) return st;
-  // flags: [0] stack overflow, [1] slot overflow, [2] scan error, [3] pair total
-  int* f = w->h_counters + kPinnedPairFlags;  // pinned
-  B2G_HIP(hipMemcpyAsync(f, flags, 4 * sizeof(int), hipMemcpyDeviceToHost, w->stream));
-  B2G_HIP(hipStreamSynchronize(w->stream));
-  const int h[4] = {f[3], f[0], f[1], f[2]};
+  int* host = w->h_counters + kPinnedFind;
+  const int epoch = ++w->publish_epoch;
+  const PairOut out = pair_out(w, dst, old);
+  hipLaunchKernelGGL(k_emit_pairs, dim3(std::max(1, blocks_for(nt, kBlock))), dim3(kBlock), 0, w->stream, nt,
+                     bp.leafrec.p, bp.count.p, bp.slots.p, dst.off.p, out, flags, host, epoch);
+  if (old)  // (about as many pairs as in the old set; more take another round of the grid)
+    hipLaunchKernelGGL(k_merge, dim3(blocks_for(std::max(w->n_pairs + w->n_pairs / 8, 4096), kBlock)), dim3(kBlock), 0,
+                       w->stream, out, flags, -1);
+  B2G_HIP(hipGetLastError());
+  if ((st = wait_published(w, host, epoch))) return st;
+  // [1] stack overflow, [2] slot overflow, [3] scan error, [4] pair total
+  const int stack = host[1], overflow = host[2], scan = host[3], total = host[4];
   if ((st = kt_harvest(w))) return st;
-  if (h[1]) {
+  if (stack) {
     set_error("broadphase: BVH traversal stack overflow");
     return B2G_ERR_CAPACITY;
   }
-  if (h[3]) {
+  if (scan) {
     set_error("device scan: a tile waited too long for its predecessor");
     return B2G_ERR_DEVICE;
   }
-  int total = h[0];
   kt_aux(w, B2G_KERNEL_TRAVERSE, total);
-  if ((st = dst.pair.reserve(pair_capacity(w, total)))) return st;
-  if (nt > 0)
-    hipLaunchKernelGGL(k_pairs_from_slots, dim3(blocks_for(nt, kBlock)), dim3(kBlock), 0, w->stream, nt,
-                       bp.leafrec.p, bp.count.p, bp.slots.p, dst.off.p, dst.pair.p);
-  if (h[2] > 0)
-    hipLaunchKernelGGL(k_traverse<true>, dim3(blocks_for(nt * kTravLanes, kTravBlock)), dim3(kTravBlock), 0, w->stream, nt, fat,
-                       tv, pf, bp.count.p, bp.slots.p, dst.off.p, dst.pair.p, flags, nullptr);
-  B2G_HIP(hipGetLastError());
+  if ((overflow || total > out.cap) &&
+      (st = finish_pairs(w, fat, tv, pf, dst, old, total, overflow != 0, flags)))
+    return st;
   *npairs = total;
   return B2G_OK;
 }
 
-static int reserve_contacts(World* w, ContactArrays& c, int pairs) {
-  int st;
-  const size_t n = pair_capacity(w, pairs);
-  if ((st = c.pair.reserve(n)) || (st = c.old_index.reserve(n)) || (st = c.ab.reserve(n)) || (st = c.hdr.reserve(n)) ||
-      (st = c.geo.reserve(n)) || (st = c.pt0.reserve(n)) || (st = c.pt1.reserve(n)) || (st = c.ids.reserve(n)) ||
-      (st = c.colour.reserve(n)))
-    return st;
-  return B2G_OK;
-}
-
-int phase_synchronize_view(World* w, IslandView iv, int* any_moved) {
-  if (w->np == 0) return B2G_OK;
-  hipLaunchKernelGGL(k_synchronize, dim3(blocks_for(w->np, kBlock)), dim3(kBlock), 0, w->stream, w->np,
-                     sync_args(w, iv), any_moved);
-  B2G_HIP(hipGetLastError());
-  return B2G_OK;
-}
-
-int phase_synchronize(World* w) {
-  return phase_synchronize_view(w, IslandView{w->s.parent.p, w->sleep_possible() ? w->s.isl_awake.p : nullptr},
-                                nullptr);
-}
-
-// New contact set from the current fat AABBs; becomes the current set, the old one is kept
+// New contact set from the current fat AABBs (after `sync`); becomes the current set, the old one is kept
 // (its manifolds feed warm starting).
-int phase_broadphase(World* w) {
-  if (small_find_fits(w)) return small_find(w, false, IslandView{nullptr, nullptr}, nullptr);
-  return phase_broadphase_general(w);
-}
-
-int phase_broadphase_general(World* w) {
-  int next = 1 - w->cur;
-  ContactArrays& dst = w->c[next];
-  ContactArrays& old = w->c[w->cur];
-  int n = 0;
-  int st;
-  if (w->np == 0) {
-    w->cur = next;
-    w->n_pairs_old = w->n_pairs;
-    w->n_pairs = 0;
-    return B2G_OK;
+static int broadphase(World* w, const SyncArgs* sync) {
+  const int next = 1 - w->cur;
+  int n = 0, st;
+  if (w->np > 0) {
+    if ((st = find_pairs(w, w->f.fat.p, w->np, sync, w->c[next], &w->c[w->cur], &n))) return st;
+    w->set_np[next] = w->np;
+    // A solve of a launch per colour and iteration leaves a hundred launches or more: asked about the stream, the
+    // runtime retires those that are done, and without that each launch takes 0.4 us longer (20 steps of 1024
+    // chains, 180 launches each: 17.5 -> 19.4 ms). After few launches the question costs more than it gives.
+    if (w->solve_groups == 0 && w->n_touch > 0) (void)hipStreamQuery(w->stream);
   }
-  if ((st = find_pairs(w, w->f.fat.p, w->np, dst, &n))) return st;
-  if ((st = reserve_contacts(w, dst, n))) return st;
-  if (n > 0) {
-    int old_np = w->set_np[w->cur];  // proxies when the old set was built (0: no old set)
-    hipLaunchKernelGGL(k_merge, dim3(blocks_for(n, kBlock)), dim3(kBlock), 0, w->stream, n, dst.pair.p, old_np,
-                       old.off.p, old.pair.p, dst.old_index.p, dst.colour.p);
-    B2G_HIP(hipGetLastError());
-  }
-  w->set_np[next] = w->np;
   w->cur = next;
   w->n_pairs_old = w->n_pairs;
   w->n_pairs = n;
   return B2G_OK;
+}
+
+int phase_broadphase(World* w) {
+  if (small_find_fits(w)) return small_find(w, false, IslandView{nullptr, nullptr}, nullptr);
+  return broadphase(w, nullptr);
+}
+
+int phase_find(World* w) {
+  const IslandView iv{w->s.parent.p, w->sleep_possible() ? w->s.isl_awake.p : nullptr};
+  if (small_find_fits(w)) return small_find(w, true, iv, nullptr);
+  const SyncArgs sync = sync_args(w, iv);
+  return broadphase(w, &sync);
 }
 
 // pairs as (lower, higher) fixture index, to a stage
@@ -666,7 +730,7 @@ int broadphase_pairs_for(World* w, const float* fat_host, int64_t cap, int32_t* 
   int n = 0, st;
   if ((st = w->query_fat.reserve(std::max(np, 1)))) return st;
   B2G_HIP(hipMemcpyAsync(w->query_fat.p, fat_host, sizeof(float4) * np, hipMemcpyHostToDevice, w->stream));
-  if ((st = find_pairs(w, w->query_fat.p, np, w->query_set, &n))) return st;
+  if ((st = find_pairs(w, w->query_fat.p, np, nullptr, w->query_set, nullptr, &n))) return st;
   *count = n;
   return staged(
       w, static_cast<size_t>(std::min<int64_t>(cap, n)), kStageBytes / sizeof(int2),
@@ -702,13 +766,7 @@ struct SmallFind {
   int* count;
   const int* slots;
   int* off;
-  int2* pairs;
-  int cap;  // pairs the new set's arrays hold
-  int old_np;
-  const int* old_off;
-  const int2* old_pairs;
-  int* old_index;
-  int* colour;
+  PairOut out;
   int* host;  // pinned: [0] published, [1..3] flags, [4] pairs
   int epoch;
 };
@@ -730,7 +788,7 @@ __global__ void __launch_bounds__(kSmallBlock) k_small_build(SmallFind a) {
   if (a.bail && *a.bail) return;
   if (t == 0) pair_flags_init(a.flags, a.scan_ctl);
   if (a.sync)
-    for (int i = t; i < a.np; i += kSmallBlock) synchronize_one(i, a.s, nullptr);
+    for (int i = t; i < a.np; i += kSmallBlock) synchronize_one(i, a.s);
   __syncthreads();
   // bounds of the fat-AABB centres, then the codes (k_bounds and k_morton)
   float lx = kMaxFloat, ly = kMaxFloat, hx = -kMaxFloat, hy = -kMaxFloat;
@@ -861,22 +919,16 @@ __global__ void __launch_bounds__(kSmallBlock) k_small_pairs(SmallFind a) {
     }
     if (t == 0) {
       a.off[a.np] = total;
-      ok = a.flags[0] == 0 && a.flags[1] == 0 && total <= a.cap;
+      ok = a.flags[0] == 0 && a.flags[1] == 0 && total <= a.out.cap;
     }
     __syncthreads();
     if (ok) {
       for (int k = t; k < a.nt; k += kSmallBlock) {
         const int q = a.leafrec[k].x, c = a.count[q], o = a.off[q];
-        for (int j = 0; j < c; ++j) a.pairs[o + j] = make_int2(q, a.slots[size_t(j) * a.nt + k]);
+        for (int j = 0; j < c; ++j) a.out.pairs[o + j] = make_int2(q, a.slots[size_t(j) * a.nt + k]);
       }
       __syncthreads();
-      for (int k = t; k < total; k += kSmallBlock) {
-        const int2 pr = a.pairs[k];
-        int found = find_in_segment(pr.x, pr.y, a.old_np, a.old_off, a.old_pairs);
-        if (found < 0) found = find_in_segment(pr.y, pr.x, a.old_np, a.old_off, a.old_pairs);
-        a.old_index[k] = found;
-        a.colour[k] = -1;
-      }
+      for (int k = t; k < total; k += kSmallBlock) pair_predecessor(k, a.out.pairs[k], a.out);
     }
   }
   if (t == 0) {
@@ -933,15 +985,9 @@ int small_find(World* w, bool sync, IslandView iv, const int* bail) {
   a.count = bp.count.p;
   a.slots = bp.slots.p;
   a.off = dst.off.p;
-  a.pairs = dst.pair.p;
-  a.cap = static_cast<int>(dst.colour.cap);  // (the arrays of a set are reserved together)
-  a.old_np = w->set_np[w->cur];
-  a.old_off = old.off.p;
-  a.old_pairs = old.pair.p;
-  a.old_index = dst.old_index.p;
-  a.colour = dst.colour.p;
+  a.out = pair_out(w, dst, &old);
   a.host = w->h_counters + kPinnedFind;
-  static_assert(kPinnedFind + 5 <= kPinnedInts, "pinned pair-search counters");
+  static_assert(kPinnedFind + 5 <= kPinnedStage, "pinned pair-search counters");
   a.epoch = ++w->publish_epoch;
   hipLaunchKernelGGL(k_small_build, dim3(1), dim3(kSmallBlock), 0, w->stream, a);
   PairFilter pf{w->f.body.p, w->b.type.p, w->f.filter.p, w->f.shape.p, w->f.world.p, nc ? w->j.nc_off.p : nullptr,
@@ -961,19 +1007,9 @@ int small_find(World* w, bool sync, IslandView iv, const int* bail) {
     return B2G_ERR_DEVICE;
   }
   const int total = a.host[4];
-  if (a.host[2] > 0 || total > a.cap) {
-    // the pairs and their predecessors by the launches (a walk overflowed its slots, or the set outgrew
-    // its arrays)
-    if ((st = reserve_contacts(w, dst, total))) return st;
-    hipLaunchKernelGGL(k_pairs_from_slots, dim3(blocks_for(nt, kBlock)), dim3(kBlock), 0, w->stream, nt, bp.leafrec.p,
-                       bp.count.p, bp.slots.p, dst.off.p, dst.pair.p);
-    if (a.host[2] > 0)
-      hipLaunchKernelGGL(k_traverse<true>, dim3(blocks_for(nt * kTravLanes, kTravBlock)), dim3(kTravBlock), 0, w->stream,
-                         nt, w->f.fat.p, tv, pf, bp.count.p, bp.slots.p, dst.off.p, dst.pair.p, a.flags, nullptr);
-    hipLaunchKernelGGL(k_merge, dim3(blocks_for(total, kBlock)), dim3(kBlock), 0, w->stream, total, dst.pair.p,
-                       a.old_np, old.off.p, old.pair.p, dst.old_index.p, dst.colour.p);
-    B2G_HIP(hipGetLastError());
-  }
+  if ((a.host[2] > 0 || total > a.out.cap) &&
+      (st = finish_pairs(w, w->f.fat.p, tv, pf, dst, &old, total, a.host[2] > 0, a.flags)))
+    return st;
   w->set_np[next] = np;
   w->cur = next;
   w->n_pairs_old = w->n_pairs;

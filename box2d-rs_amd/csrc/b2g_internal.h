@@ -98,6 +98,7 @@ struct ProxyArrays {
   DevArray<int> moved;      // the tree's moved flag (set when the fat AABB was re-fattened)
   DevArray<int> world;      // world id of the proxy's body (batched worlds never interact)
   DevArray<int> tree_list;  // proxies kept in the BVH
+  DevArray<unsigned char> in_tree;  // per proxy: it is one of them
   DevArray<int> loose_off;  // per world: range in `loose` of its big static proxies
   DevArray<int> loose;      // big static proxies (ground, walls) tested directly, not in the BVH
   DevArray<ShapeV> shapev;  // per proxy: its shape as the collide functions read it (by reference)
@@ -333,6 +334,7 @@ struct World {
   int n_tree = 0;                       // proxies in the BVH
   // host sources of asynchronous uploads must outlive the copy: kept here, not on the stack
   std::vector<int> h_tree, h_loose_off, h_loose;
+  std::vector<unsigned char> h_in_tree;
   int n_worlds = 1;
   std::vector<ShapeV> h_shapev;
   std::vector<int> h_awake, h_auto_sleep, h_bullet;
@@ -383,7 +385,7 @@ struct World {
   DevArray<int> counters;   // small device counters: 4 solver counters, then the colour histogram
   // pinned host memory (kPinnedInts ints): [0, 134) the solver's counters read back after the
   // colouring (4 counters, 128 colour counts, last round, large-island constraints),
-  // [kPinnedPairFlags, +4) the pair search's flags and total, [kPinnedColourOffsets, +385) the
+  // [kPinnedColourOffsets, +385) the
   // colour offsets uploaded for the solve, [kPinnedToi, +8) the counters of a separable TOI pass,
   // [kPinnedSmall, +134) and [kPinnedFind, +6) what the small-world kernels publish,
   // [kPinnedStage, +2) the last transfer through each half of the stage
@@ -446,7 +448,7 @@ struct World {
   JointArrays j;
 };
 
-constexpr int kPinnedInts = 1024, kPinnedPairFlags = 192, kPinnedColourOffsets = 256, kPinnedToi = 768,
+constexpr int kPinnedInts = 1024, kPinnedColourOffsets = 256, kPinnedToi = 768,
               kPinnedSmall = 800, kPinnedFind = 944, kPinnedStage = 960;
 
 // Capacity floor of the arrays sized by the contact set (the pairs, and the solver's arrays,
@@ -540,11 +542,10 @@ int kt_harvest(World* w);
 
 // phase drivers (each returns a B2G_* status)
 int upload_world(World* w);
-int phase_broadphase_general(World* w);
 int phase_broadphase(World* w);  // fat AABBs -> next contact set (pairs + old indices)
 int phase_collide(World* w);     // narrowphase on the current contact set
 int phase_solve(World* w, float dt, float dt_ratio, int vel_iters, int pos_iters);
-int phase_synchronize(World* w); // swept + fat AABBs of non-static proxies
+int phase_find(World* w);  // synchronize the proxies of the awake islands, then the new contact set
 struct IslandView;
 // Small worlds (b2g_world_step): a step's solve in one launch and its pair search in three
 constexpr int kSmallBodies = 2048, kSmallTree = 2048, kSmallProxies = 4096, kSmallPairs = 4096, kSmallTouch = 2048;
@@ -614,7 +615,10 @@ int toi_carry_state(World* w);              // TOI state of the previous contact
 void release_solve_graphs(World* w);
 // primitives
 int exclusive_scan(World* w, const int* in, int* out, int n, int* total_dev, int* total2 = nullptr);
-int radix_sort_pairs(World* w, unsigned* keys, unsigned* vals, int n, int bits);
+// tiles of the radix sort, 8-bit digits; histograms are digit-major: hist[d * tiles + tile]
+constexpr int kSortBlock = 256, kSortItems = 4, kSortTile = kSortBlock * kSortItems, kRadix = 256;
+int radix_reserve(World* w, int n);
+int radix_sort_pairs(World* w, unsigned* keys, unsigned* vals, int n, int bits, bool first_hist = false);
 // stateless collide of fixture pairs under given transforms (parity entry point)
 int collide_fixture_pairs(World* w, int n, const int32_t* pairs, const float* xfa, const float* xfb,
                           b2g_manifold* out);
@@ -641,9 +645,6 @@ struct IslandView {
   const int* isl_awake;  // per root; null: every island is awake
   __device__ bool asleep(int b) const { return isl_awake && !isl_awake[parent[b]]; }
 };
-// phase_synchronize for the bodies the view holds awake; any_moved (optional) is set to 1 when a
-// proxy is re-fattened
-int phase_synchronize_view(World* w, IslandView iv, int* any_moved);
 
 // Kernel arguments of the joint solve (b2g_joints.hip).
 struct JointArgs {

@@ -241,10 +241,6 @@ int exclusive_scan(World* w, const int* in, int* out, int n, int* total_dev, int
 }
 
 // ---- radix sort ---------------------------------------------------------------------------
-static constexpr int kSortBlock = 256;
-static constexpr int kSortItems = 4;
-static constexpr int kSortTile = kSortBlock * kSortItems;
-static constexpr int kRadix = 256;
 
 // histogram of one 8-bit digit per tile; hist is digit-major: hist[d * nblocks + block]
 __global__ void __launch_bounds__(kSortBlock) k_radix_hist(const unsigned* __restrict__ keys, int n, int shift,
@@ -343,19 +339,27 @@ __global__ void __launch_bounds__(kSortBlock) k_radix_scatter(const unsigned* __
 // Sorted (keys, vals) end in the given arrays; when those are the world's bp.keys / bp.vals and an
 // odd number of passes leaves the result in the alternate buffers, the buffers are swapped
 // instead of copied (callers read bp.keys.p / bp.vals.p again after the call).
-int radix_sort_pairs(World* w, unsigned* keys, unsigned* vals, int n, int bits) {
+// first_hist: bp.hist holds the low digit's histogram already (the kernel that made the keys counted them).
+int radix_reserve(World* w, int n) {
+  int st;
+  BroadphaseArrays& bp = w->bp;
+  if ((st = bp.keys_alt.reserve(n)) || (st = bp.vals_alt.reserve(n)) ||
+      (st = bp.hist.reserve(size_t(kRadix) * blocks_for(n, kSortTile))))
+    return st;
+  return B2G_OK;
+}
+int radix_sort_pairs(World* w, unsigned* keys, unsigned* vals, int n, int bits, bool first_hist) {
   if (n <= 1) return B2G_OK;
   BroadphaseArrays& bp = w->bp;
   int st;
-  if ((st = bp.keys_alt.reserve(n))) return st;
-  if ((st = bp.vals_alt.reserve(n))) return st;
+  if ((st = radix_reserve(w, n))) return st;
   int nblocks = blocks_for(n, kSortTile);
-  if ((st = bp.hist.reserve(size_t(kRadix) * nblocks))) return st;
   unsigned *k0 = keys, *v0 = vals, *k1 = bp.keys_alt.p, *v1 = bp.vals_alt.p;
   int passes = (bits + 7) / 8;
   for (int p = 0; p < passes; ++p) {
     int shift = 8 * p;
-    hipLaunchKernelGGL(k_radix_hist, dim3(nblocks), dim3(kSortBlock), 0, w->stream, k0, n, shift, bp.hist.p, nblocks);
+    if (p > 0 || !first_hist)
+      hipLaunchKernelGGL(k_radix_hist, dim3(nblocks), dim3(kSortBlock), 0, w->stream, k0, n, shift, bp.hist.p, nblocks);
     if (nblocks <= kRadixFuseMax) {
       hipLaunchKernelGGL(k_radix_scatter<true>, dim3(nblocks), dim3(kSortBlock), 0, w->stream, k0, v0, n, shift,
                          bp.hist.p, nblocks, k1, v1);
