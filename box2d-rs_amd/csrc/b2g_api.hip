@@ -838,6 +838,8 @@ int b2g_world_step(b2g_world* h, float dt, int32_t vi, int32_t pi) {
   if (w->continuous && dt > 0.0f && (st = phase_toi(w, dt, vi))) return st;
   (void)hipEventRecord(w->ev[3], w->stream);
   w->profile_pending = true;
+  // (a step need not wait for the stream; asked about it now and then, the runtime retires finished launches)
+  if ((++w->steps_taken & 31) == 0) (void)hipStreamQuery(w->stream);
   return B2G_OK;
 }
 

@@ -772,7 +772,8 @@ struct SmallFind {
 };
 
 struct SmallTree {
-  unsigned long long key[kSmallTree];  // Morton code << 32 | proxy
+  unsigned long long key[kSmallTree], key_alt[kSmallTree];  // Morton code << 32 | proxy
+  int count[kSmallBlock / 64][kRadix], first[kRadix], digits[kRadix / 64];
   float4 seg[2 * kSmallTree + 32];
   unsigned short lo[kSmallTree], hi[kSmallTree], split[kSmallTree];
 };
@@ -808,32 +809,85 @@ __global__ void __launch_bounds__(kSmallBlock) k_small_build(SmallFind a) {
   for (int w = 0; w < kSmallBlock / 64; ++w) {
     lx = fminf(lx, red[0][w]); ly = fminf(ly, red[1][w]); hx = fmaxf(hx, red[2][w]); hy = fmaxf(hy, red[3][w]);
   }
-  int m = 64;  // elements sorted: a power of two
-  while (m < a.nt) m <<= 1;
-  for (int i = t; i < m; i += kSmallBlock) {
-    unsigned long long key = ~0ull;
+  // Stable sort by code, three passes of 8 bits: wave w holds the keys [w * 128, w * 128 + 128), two a lane, ranks them
+  // by ballots, and the waves' counts per digit give the places. (A bitonic sort's 66 steps for 2048 keys took
+  // 20 us, in LDS as well as by lane exchanges: a workgroup's instructions bound it; this takes 8 us.)
+  constexpr int kWaves = kSmallBlock / 64, kPerWave = kSmallTree / kWaves;
+  static_assert(kPerWave == 128, "two keys per lane");
+  const int used = (a.nt + kPerWave - 1) / kPerWave;  // waves that hold keys
+  unsigned long long* from = s.key;
+  unsigned long long* to = s.key_alt;
+#pragma unroll
+  for (int r = 0; r < 2; ++r) {
+    const int i = wid * kPerWave + r * 64 + lane;
     if (i < a.nt) {
       const int p = a.list[i];
-      key = (static_cast<unsigned long long>(morton_code(a.s.ffat[p], lx, ly, hx, hy, a.mbits)) << 32) | unsigned(p);
+      from[i] = (static_cast<unsigned long long>(morton_code(a.s.ffat[p], lx, ly, hx, hy, a.mbits)) << 32) | unsigned(p);
     }
-    s.key[i] = key;
   }
-  __syncthreads();
-  for (int size = 2; size <= m; size <<= 1)
-    for (int step = size >> 1; step > 0; step >>= 1) {
-      for (int i = t; i < m / 2; i += kSmallBlock) {
-        const int lo = 2 * i - (i & (step - 1)), hi = lo + step;
-        const unsigned long long x = s.key[lo], y = s.key[hi];
-        if ((x > y) == ((lo & size) == 0)) {
-          s.key[lo] = y;
-          s.key[hi] = x;
-        }
+  for (int shift = 32; shift < 32 + 2 * a.mbits; shift += 8) {
+    for (int e = t; e < used * kRadix; e += kSmallBlock) (&s.count[0][0])[e] = 0;
+    __syncthreads();
+    unsigned long long key[2];
+    int digit[2], rank[2];
+#pragma unroll
+    for (int r = 0; r < 2; ++r) {
+      const int i = wid * kPerWave + r * 64 + lane;
+      const bool valid = i < a.nt;
+      if (wid * kPerWave + r * 64 >= a.nt) break;  // (uniform across the wave)
+      key[r] = valid ? from[i] : 0;
+      digit[r] = static_cast<int>(key[r] >> shift) & 0xff;
+      unsigned long long same = __ballot(valid);
+#pragma unroll
+      for (int bit = 0; bit < 8; ++bit) {
+        const bool on = (digit[r] >> bit) & 1;
+        const unsigned long long m = __ballot(on);
+        same &= on ? m : ~m;
       }
-      __syncthreads();
+      const unsigned long long lower = same & ((1ull << lane) - 1ull);
+      // the wave's earlier keys of this digit, then its own are added by the first lane that has it
+      const int before = s.count[wid][digit[r]];
+      __builtin_amdgcn_wave_barrier();
+      if (valid && lower == 0) s.count[wid][digit[r]] = before + __popcll(same);
+      __builtin_amdgcn_wave_barrier();
+      rank[r] = before + __popcll(lower);
     }
+    __syncthreads();
+    // per digit: the waves' counts become their offsets, the totals are scanned over the digits
+    int total = 0;
+    if (t < kRadix)
+      for (int w = 0; w < used; ++w) {
+        const int c = s.count[w][t];
+        s.count[w][t] = total;
+        total += c;
+      }
+    int inc = total;
+    for (int d = 1; d < 64; d <<= 1) {
+      const int y = __shfl_up(inc, d, 64);
+      if (lane >= d) inc += y;
+    }
+    if (t < kRadix && lane == 63) s.digits[wid] = inc;
+    __syncthreads();
+    if (t < kRadix) {
+      int first = inc - total;
+      for (int w = 0; w < wid; ++w) first += s.digits[w];
+      s.first[t] = first;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < 2; ++r) {
+      const int i = wid * kPerWave + r * 64 + lane;
+      if (i < a.nt) to[s.first[digit[r]] + s.count[wid][digit[r]] + rank[r]] = key[r];
+    }
+    unsigned long long* x = from;
+    from = to;
+    to = x;
+    __syncthreads();
+  }
+  const unsigned long long* sorted = from;
   // leaf boxes and records, then the segment tree level by level
   for (int i = t; i < a.nt; i += kSmallBlock) {
-    const int p = static_cast<int>(s.key[i] & 0xffffffffu);
+    const int p = static_cast<int>(sorted[i] & 0xffffffffu);
     s.seg[i] = a.s.ffat[p];
     a.leafrec[i] = leaf_record(p, a.li);
   }
@@ -848,7 +902,7 @@ __global__ void __launch_bounds__(kSmallBlock) k_small_build(SmallFind a) {
     }
     __syncthreads();
   }
-  const SmallKeys keys{s.key};
+  const SmallKeys keys{sorted};
   for (int i = t; i < a.nt - 1; i += kSmallBlock) {
     int lo, hi, gamma;
     lbvh_node(keys, a.nt, i, lo, hi, gamma);

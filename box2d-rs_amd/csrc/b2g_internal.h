@@ -388,7 +388,8 @@ struct World {
   // [kPinnedColourOffsets, +385) the
   // colour offsets uploaded for the solve, [kPinnedToi, +8) the counters of a separable TOI pass,
   // [kPinnedSmall, +134) and [kPinnedFind, +6) what the small-world kernels publish,
-  // [kPinnedStage, +2) the last transfer through each half of the stage
+  // [kPinnedStage, +2) the last transfer through each half of the stage,
+  // [kPinnedDropped, +2) the contacts dropped at a rebuild of the continuous pass
   int* h_counters = nullptr;
   int n_touch = 0, n_colors = 0, n_islands = 0;
   int color_rounds = 16;       // colouring rounds launched before the first readback
@@ -418,6 +419,7 @@ struct World {
   ContactArrays query_set;
   std::vector<int> static_bodies;  // (toi_note_bodies)
   int publish_epoch = 0;   // value of the last published word (pinned memory)
+  unsigned steps_taken = 0;
   int small_holdoff = 0;   // steps for which the small-world kernels are left alone after a world outgrew them
   int solve_groups = 0;  // groups per colour of the last solve's constraints (s.cw_off); 0: not grouped
   bool worlds_contiguous = false;         // every world's bodies are one index range (set at upload)
@@ -449,7 +451,7 @@ struct World {
 };
 
 constexpr int kPinnedInts = 1024, kPinnedColourOffsets = 256, kPinnedToi = 768,
-              kPinnedSmall = 800, kPinnedFind = 944, kPinnedStage = 960;
+              kPinnedSmall = 800, kPinnedFind = 944, kPinnedStage = 960, kPinnedDropped = 968;
 
 // Capacity floor of the arrays sized by the contact set (the pairs, and the solver's arrays,
 // which the pairs bound): reserving for a multiple of the proxy count from the first step keeps a

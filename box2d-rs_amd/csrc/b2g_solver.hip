@@ -1964,7 +1964,8 @@ static int launch_groups(World* w, int nc, bool worlds, GroupSolve a) {
 // (whose last colour is solved serially) is left untouched (*bail) and stepped by those launches.
 // A frame (step and states) of one box on the ground: 290 us -> 203 us; of the pyramid: 403 us -> 288 us;
 // 40 steps of 1531 stacked boxes: 20.8 ms -> 17.9 ms (one workgroup then is slower than the bins' many by 50 us
-// a step, the launches were 120 us).
+// a step, the launches were 120 us). Now 110 us, 190 us and 15.4 ms with the steps after it. The kernel takes
+// 26, 118 and 133 us: the group solve's phases 10, 85 and 72, the colouring rounds 2 each.
 constexpr int kSmallThreads = 512;
 static_assert(kSmallThreads >= kMaxColors, "a thread per colour");
 
@@ -2004,6 +2005,7 @@ struct SmallSetup {
   unsigned short bodyA[kSmallTouch], bodyB[kSmallTouch];
   int state[kSmallTouch];
   short prev[kSmallTouch];
+  unsigned short open[kSmallTouch];  // the constraints that round 0 left without a colour
   unsigned char type[kSmallBodies];
 };
 static_assert(kSmallBodies <= 65536 && kSmallTouch <= 65536, "16-bit body and constraint numbers");
@@ -2013,7 +2015,7 @@ __global__ void __launch_bounds__(kSmallThreads, 2) k_small_solve(SmallArgs a) {
   using Store = GroupStore<T, kSmallBodies, true>;
   __shared__ __align__(16) unsigned char raw[sizeof(Store) > sizeof(SmallSetup) ? sizeof(Store) : sizeof(SmallSetup)];
   __shared__ int wsum[T / 64], count[kMaxColors], launch[kMaxColors], base[kMaxColors + 1], cursor[kMaxColors];
-  __shared__ int n_touch, left, last_round, overflow, ncolors, nsolved;
+  __shared__ int n_touch, left, last_round, ncolors, nsolved;
   SmallSetup& s = *reinterpret_cast<SmallSetup*>(raw);
   const int t = threadIdx.x, lane = t & 63, wid = t >> 6;
   // exclusive scan over the threads' values; every thread gets its prefix, *total the sum
@@ -2034,7 +2036,7 @@ __global__ void __launch_bounds__(kSmallThreads, 2) k_small_solve(SmallArgs a) {
     *total = sum;
     return before + inc - x;
   };
-  if (t == 0) left = last_round = overflow = 0;
+  if (t == 0) left = last_round = 0;
   for (int c = t; c < kMaxColors; c += T) count[c] = cursor[c] = 0;
   // touching contacts in pair order: constraint j = its rank among them
   {
@@ -2158,24 +2160,38 @@ __global__ void __launch_bounds__(kSmallThreads, 2) k_small_solve(SmallArgs a) {
       if (kept) st = s.prev[j];
     }
     s.state[j] = st;
-    if (st == -1) left = 1;  // every writer stores 1
+    if (st == -1) s.open[atomicAdd(&left, 1)] = static_cast<unsigned short>(j);
   }
   __syncthreads();
   // Jones-Plassmann-Luby rounds (k_color_round): each colours at least the uncoloured constraint of
   // highest priority, so at most nt of them run
+  const int n_open = left;
   for (int round = 1; left; ++round) {
     __syncthreads();
     if (t == 0) left = 0;
     __syncthreads();
-    for (int j = t; j < nt; j += T) {
+    for (int e = t; e < n_open; e += T) {
+      const int j = s.open[e];
       if (s.state[j] != -1) continue;
       const unsigned long long pj = priority(j);
       unsigned long long used0 = 0, used1 = 0;
       bool lose = false;
-      neighbours(j, [&](int o) {
-        color_look(o, __hip_atomic_load(&s.state[o], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP), round, pj, lose,
-                   used0, used1);
-      });
+      // as in color_pick: a body's first entries, then their states, by independent loads
+      for (int side = 0; side < 2; ++side) {
+        const int b = side ? s.bodyB[j] : s.bodyA[j];
+        if (s.type[b] != 2) continue;
+        for (int e0 = s.off[b], e1 = s.off[b + 1]; e0 < e1; e0 += 4) {
+          int o[4], so[4];
+#pragma unroll
+          for (int u = 0; u < 4; ++u) o[u] = e0 + u < e1 ? s.adj[e0 + u] : j;
+#pragma unroll
+          for (int u = 0; u < 4; ++u)
+            so[u] = __hip_atomic_load(&s.state[o[u]], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+#pragma unroll
+          for (int u = 0; u < 4; ++u)
+            if (o[u] != j) color_look(o[u], so[u], round, pj, lose, used0, used1);
+        }
+      }
       int c = -1;
       if (!lose) c = ~used0 ? __ffsll(static_cast<long long>(~used0)) - 1
                             : ~used1 ? 64 + __ffsll(static_cast<long long>(~used1)) - 1 : kMaxColors - 1;
@@ -2196,17 +2212,18 @@ __global__ void __launch_bounds__(kSmallThreads, 2) k_small_solve(SmallArgs a) {
     bail_out();
     return;
   }
-  if (t == 0) {
-    int n = 0, nc = 0;
-    for (int c = 0; c < kMaxColors; ++c) {
-      launch[c] = nc;
-      if (count[c] == 0) continue;
-      base[nc++] = n;
-      n += count[c];
+  // offsets and launch indices of the colours in use
+  {
+    const int c = t < kMaxColors ? count[t] : 0;
+    int n, used;
+    const int before = scan(c, &n), index = scan(c > 0, &used);
+    if (t < kMaxColors) launch[t] = index;
+    if (c > 0) base[index] = before;
+    if (t == 0) {
+      base[used] = n;
+      ncolors = used;
+      nsolved = n;
     }
-    base[nc] = n;
-    ncolors = nc;
-    nsolved = n;
   }
   __syncthreads();
   const int nc = ncolors;

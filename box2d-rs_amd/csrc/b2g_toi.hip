@@ -995,6 +995,18 @@ __global__ void __launch_bounds__(kToiBlock) k_toi_begin(ToiArgs a, SepArgs p, i
   if (first) a.alpha0[b] = 0.0f;
 }
 
+// the pass's counters to the host, which sees them 10 us before a copy would have arrived
+__global__ void k_toi_publish(const SepCtl* ctl, SepCtl* host, int epoch) {
+  if (threadIdx.x > 0) return;
+  host->queued = ctl->queued;
+  host->waiting = ctl->waiting;
+  host->left = ctl->left;
+  host->events = ctl->events;
+  host->solved = ctl->solved;
+  __threadfence_system();
+  __hip_atomic_store(&host->pad[2], epoch, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 // One thread per contact of the set: contacts of a dynamic with a static body are linked to the
 // body, those without a cached time of impact get one, and the body of one below 1 is queued. The
 // two sweeps need no alignment in set order: the dynamic body's alpha0 is the largest (a static
@@ -1438,11 +1450,13 @@ __global__ void __launch_bounds__(kToiBlock) k_mark_successors(int n, const int*
   if (o >= 0 && o < n_old) succ[o] = 1;
 }
 
+// a touching contact without a successor
+__device__ inline int dropped_flag(int hdr, int succ) { return (hdr >> 8) > 0 && !succ ? 1 : 0; }
 __global__ void __launch_bounds__(kToiBlock) k_dropped_flags(int n_old, const int* __restrict__ hdr,
                                                              const int* __restrict__ succ, int* __restrict__ flag) {
   const int k = blockIdx.x * blockDim.x + threadIdx.x;
   if (k >= n_old) return;
-  flag[k] = (hdr[k] >> 8) > 0 && !succ[k] ? 1 : 0;
+  flag[k] = dropped_flag(hdr[k], succ[k]);
 }
 
 struct ContactView {
@@ -1494,6 +1508,47 @@ static int reserve_contacts(ContactArrays& c, int n, int keep) {
   return B2G_OK;
 }
 
+// The predecessor's touching contacts without a successor in the current set, and their places among
+// them, for sets that one workgroup holds: four launches, a copy and a wait on the stream (28 us) in one launch.
+constexpr int kDroppedBlock = 1024;
+__global__ void __launch_bounds__(kDroppedBlock) k_toi_dropped(int n_cur, const int* __restrict__ old_index, int n_old,
+                                                               const int* __restrict__ old_hdr, int* __restrict__ flag,
+                                                               int* __restrict__ pos, int* host, int epoch) {
+  __shared__ unsigned char succ[kSmallPairs];
+  __shared__ int wsum[kDroppedBlock / 64];
+  const int t = threadIdx.x, lane = t & 63, wid = t >> 6;
+  for (int k = t; k < n_old; k += kDroppedBlock) succ[k] = 0;
+  __syncthreads();
+  for (int k = t; k < n_cur; k += kDroppedBlock) {
+    const int o = old_index[k];
+    if (o >= 0 && o < n_old) succ[o] = 1;
+  }
+  __syncthreads();
+  const int chunk = (n_old + kDroppedBlock - 1) / kDroppedBlock, k0 = min(n_old, t * chunk), k1 = min(n_old, k0 + chunk);
+  int sum = 0;
+  for (int k = k0; k < k1; ++k) sum += dropped_flag(old_hdr[k], succ[k]);
+  int inc = sum;
+  for (int d = 1; d < 64; d <<= 1) {
+    const int y = __shfl_up(inc, d, 64);
+    if (lane >= d) inc += y;
+  }
+  if (lane == 63) wsum[wid] = inc;
+  __syncthreads();
+  int ex = inc - sum;
+  for (int v = 0; v < wid; ++v) ex += wsum[v];
+  for (int k = k0; k < k1; ++k) {
+    const int f = dropped_flag(old_hdr[k], succ[k]);
+    flag[k] = f;
+    pos[k] = ex;
+    ex += f;
+  }
+  if (t == kDroppedBlock - 1) {
+    host[1] = ex;
+    __threadfence_system();
+    __hip_atomic_store(host, epoch, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+  }
+}
+
 static int toi_rebuild(World* w) {
   int st;
   // the predecessor's dropped touching contacts (its extra entries included) before it is
@@ -1506,17 +1561,27 @@ static int toi_rebuild(World* w) {
     if ((st = w->toi_succ.reserve(n_old)) || (st = w->toi_drop_flag.reserve(n_old)) ||
         (st = w->toi_drop_pos.reserve(n_old)) || (st = w->toi_drop_total.reserve(1)))
       return st;
-    hipLaunchKernelGGL(k_clear, dim3(blocks_for(n_old, kToiBlock)), dim3(kToiBlock), 0, w->stream, n_old,
-                       w->toi_succ.p);
-    if (n_cur > 0)
-      hipLaunchKernelGGL(k_mark_successors, dim3(blocks_for(n_cur, kToiBlock)), dim3(kToiBlock), 0, w->stream, n_cur,
-                         w->c[w->cur].old_index.p, n_old, w->toi_succ.p);
-    hipLaunchKernelGGL(k_dropped_flags, dim3(blocks_for(n_old, kToiBlock)), dim3(kToiBlock), 0, w->stream, n_old,
-                       pred.hdr.p, w->toi_succ.p, w->toi_drop_flag.p);
-    B2G_HIP(hipGetLastError());
-    if ((st = exclusive_scan(w, w->toi_drop_flag.p, w->toi_drop_pos.p, n_old, w->toi_drop_total.p))) return st;
-    B2G_HIP(hipMemcpyAsync(&dropped, w->toi_drop_total.p, sizeof(int), hipMemcpyDeviceToHost, w->stream));
-    B2G_HIP(hipStreamSynchronize(w->stream));
+    if (std::max(n_old, n_cur) <= kSmallPairs) {
+      int* host = w->h_counters + kPinnedDropped;
+      const int epoch = ++w->publish_epoch;
+      hipLaunchKernelGGL(k_toi_dropped, dim3(1), dim3(kDroppedBlock), 0, w->stream, n_cur, w->c[w->cur].old_index.p, n_old,
+                         pred.hdr.p, w->toi_drop_flag.p, w->toi_drop_pos.p, host, epoch);
+      B2G_HIP(hipGetLastError());
+      if ((st = wait_published(w, host, epoch))) return st;
+      dropped = host[1];
+    } else {
+      hipLaunchKernelGGL(k_clear, dim3(blocks_for(n_old, kToiBlock)), dim3(kToiBlock), 0, w->stream, n_old,
+                         w->toi_succ.p);
+      if (n_cur > 0)
+        hipLaunchKernelGGL(k_mark_successors, dim3(blocks_for(n_cur, kToiBlock)), dim3(kToiBlock), 0, w->stream, n_cur,
+                           w->c[w->cur].old_index.p, n_old, w->toi_succ.p);
+      hipLaunchKernelGGL(k_dropped_flags, dim3(blocks_for(n_old, kToiBlock)), dim3(kToiBlock), 0, w->stream, n_old,
+                         pred.hdr.p, w->toi_succ.p, w->toi_drop_flag.p);
+      B2G_HIP(hipGetLastError());
+      if ((st = exclusive_scan(w, w->toi_drop_flag.p, w->toi_drop_pos.p, n_old, w->toi_drop_total.p))) return st;
+      B2G_HIP(hipMemcpyAsync(&dropped, w->toi_drop_total.p, sizeof(int), hipMemcpyDeviceToHost, w->stream));
+      B2G_HIP(hipStreamSynchronize(w->stream));
+    }
     if (dropped > 0) {
       if ((st = reserve_contacts(w->toi_dropped, dropped, 0))) return st;
       if ((st = move_dropped(w, n_old, w->toi_drop_flag.p, w->toi_drop_pos.p, pred, w->toi_dropped, 0))) return st;
@@ -1686,8 +1751,10 @@ static int toi_separable(World* w, float dt, int vi, bool* dirty, bool* left) {
       hipLaunchKernelGGL(k_toi_bodies, dim3(std::min(nb, kSepBlocks)), dim3(64), 0, w->stream, a, p);
     }
     B2G_HIP(hipGetLastError());
-    B2G_HIP(hipMemcpyAsync(host, p.ctl, sizeof(SepCtl), hipMemcpyDeviceToHost, w->stream));
-    B2G_HIP(hipStreamSynchronize(w->stream));
+    const int epoch = ++w->publish_epoch;
+    hipLaunchKernelGGL(k_toi_publish, dim3(1), dim3(64), 0, w->stream, p.ctl, host, epoch);
+    B2G_HIP(hipGetLastError());
+    if ((st = wait_published(w, &host->pad[2], epoch))) return st;
     if (host->events > events) *dirty = true;
     events = host->events;
     solved = host->solved;
