@@ -43,7 +43,7 @@ HBM_PEAK_GBS = 8000.0
 # bandwidth, which the fraction shows. In steps where every island is small the whole solve (set-up,
 # warm start, velocity and position iterations) runs as one launch of k_solve_groups; the bytes are
 # still those of its velocity iterations (224 B per constraint-iteration), so the fraction understates
-# it, while its HBM traffic is far lower: it reads each constraint and body once and keeps them on chip
+# it, while its HBM traffic is lower: it reads each constraint and body once and keeps them on chip
 # (registers and LDS) across the iterations.
 # k_collide (--roofline-kernel collide): algorithmic HBM bytes of one narrowphase launch (f32/i32 sizes, each read or written once): per
 # candidate pair 120 B (pair, fixture and body records, the two transforms, the previous

@@ -20,7 +20,7 @@
 //
 // Where the recorded solve was grouped (bins of islands, worlds of a batch: no two groups share a
 // dynamic body), one workgroup runs a group's iterations with a constraint per thread, the
-// constraint and its cotangents in registers and the group's bodies in LDS, as k_solve_bins_* do:
+// constraint and its cotangents in registers and the group's bodies in LDS, as k_solve_groups does:
 // one launch for all velocity iterations instead of one per colour and iteration. Steps that were not
 // grouped, or hold a group of more than 512 constraints, launch per colour.
 //
@@ -461,7 +461,7 @@ __global__ void __launch_bounds__(kBlock) k_af_intpos(AdjCtx a) {
 }
 
 // ---- groups: a workgroup per group, a constraint per thread ---------------------------------------
-// The group's bodies sit in an LDS hash table (as in k_solve_bins_velocity), its constraints in
+// The group's bodies sit in an LDS hash table (as in k_solve_groups), its constraints in
 // registers; a barrier separates the colours. Each phase is one constraint's chain of dependent
 // arithmetic, about a microsecond, whatever the number of constraints: bound by that latency times
 // colours times iterations, with the other groups' workgroups beside it.

@@ -1000,7 +1000,7 @@ bool small_find_fits(const World* w) {
          w->kt.kernel == B2G_KERNEL_NONE;
 }
 
-// phase_synchronize (sync) and phase_broadphase for a world that small_find_fits accepts; with *bail set
+// phase_find (sync) or phase_broadphase for a world that small_find_fits accepts; with *bail set
 // on the device the kernels do nothing and the new set is empty (the caller then takes the step back)
 int small_find(World* w, bool sync, IslandView iv, const int* bail) {
   BroadphaseArrays& bp = w->bp;

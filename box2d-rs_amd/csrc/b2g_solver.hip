@@ -2471,7 +2471,7 @@ int phase_solve(World* w, float dt, float dt_ratio, int vel_iters, int pos_iters
     return st;
   const IntegrateArgs ia{w->b.type.p, w->b.pos.p, w->b.vel.p, w->b.pos0.p, w->b.props.p, w->b.mass.p, w->b.force.p,
                          w->gravity.x, w->gravity.y, dt};
-  // batched worlds: each world's iterations in one workgroup (k_solve_worlds_*); otherwise small
+  // batched worlds: each world's solve in one workgroup (k_solve_groups); otherwise small
   // islands packed into bins (k_solve_bins_*); neither with joints
   const bool want_world = w->nj == 0 && w->worlds_contiguous && w->n_worlds > 1 &&
                           (w->world_solve == 1 || (w->world_solve == -1 && w->n_worlds >= kWorldSolveMin));

@@ -411,14 +411,14 @@ enum {
  *                           fewer than 64 bodies / 64-255 bodies / 256 or more (defaults 64, 256,
  *                           512; box2d-rs_amd/b2g/autotune.py sweeps them).
  *   B2G_TUNE_ISLAND_SOLVE   1: islands of at most B2G_TUNE_ISLAND_THREADS / 2 constraints are packed
- *                           into bins, and one workgroup per bin runs all velocity (and all position)
- *                           iterations of its islands, colour after colour with workgroup barriers,
- *                           its constraints in registers and its bodies in LDS (two launches per step
- *                           instead of one per colour and iteration); larger islands keep the
- *                           per-colour launches. 0: per-colour launches only. -1 (default): bins
- *                           in steps whose small islands hold at least half of the constraints, unless
- *                           the per-world solve is on. Islands share no dynamic body, so the results
- *                           are the same bit for bit.
+ *                           into bins, and one workgroup per bin runs the solve of its islands, colour
+ *                           after colour with workgroup barriers, its constraints in registers and its
+ *                           bodies in LDS (one launch per step where no island is larger, instead of one
+ *                           per colour and iteration); larger islands keep the per-colour launches. 0:
+ *                           per-colour launches only. -1 (default): bins in steps whose small islands
+ *                           hold at least half of the constraints, unless the per-world solve is on; a
+ *                           small single world is solved as one group. Islands share no dynamic body, so
+ *                           the results are the same bit for bit.
  *   B2G_TUNE_ISLAND_THREADS threads per bin of that solve: 64, 128, 256 (default) or 512.
  *   B2G_TUNE_TOI_GLOBAL_ISLAND 1: every TOI island in the global-memory store that islands too large
  *                           for the event workgroup's LDS use (a check of that path; same results);
